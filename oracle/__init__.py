@@ -31,9 +31,9 @@ _ref_loaded = False
 
 
 def build(ref: bool = False) -> None:
-    """Compile liboracle.so (and _ref/libcint_ref.so when ref and /root/reference exist)."""
+    """Compile liboracle.so (and _ref/libcint_ref.so when ref and the reference's libcint sources exist)."""
     subprocess.run(["make", "-s", "-C", str(HERE)], check=True)
-    if ref and Path("/root/reference").is_dir():
+    if ref and Path("/root/reference/src/gradscf/integrals/_native/vendor/libcint").is_dir():
         subprocess.run(["make", "-s", "-C", str(HERE), "ref"], check=True)
 
 
