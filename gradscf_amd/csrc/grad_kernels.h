@@ -21,19 +21,6 @@
 namespace gscf {
 
 
-__device__ __forceinline__ void map_item_g(const GradArgs& a, int64_t item, int64_t& g, int& s, int& S) {
-  int lo = 0, hi = a.ntasks;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (a.tasks[mid].item0 <= item) lo = mid; else hi = mid;
-  }
-  const SubTask t = a.tasks[lo];
-  const int64_t r = item - t.item0;
-  s = (int)(r / t.nq);
-  g = t.q0 + (r - (int64_t)s * t.nq);
-  S = t.S;
-}
-
 template <int LA, int LB, int LC, int LD>
 __global__ __launch_bounds__(256) void grad_kernel(GradArgs a) {
   constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
@@ -49,8 +36,7 @@ __global__ __launch_bounds__(256) void grad_kernel(GradArgs a) {
     const int kc = (int)(t - item * NKET);
     const int ic = kc / ND, id = kc - (kc / ND) * ND;
     int64_t g;
-    int s0, S;
-    map_item_g(a, item, g, s0, S);
+    const PrimSlice sl = map_item(a.tasks, a.ntasks, item, g);
     const int2 qk = a.quartets[g];
     const Pair bp = a.pairs[qk.x];
     const Pair kp = a.pairs[qk.y];
@@ -106,9 +92,9 @@ __global__ __launch_bounds__(256) void grad_kernel(GradArgs a) {
       }
     }
     double gA[3] = {0, 0, 0}, gB[3] = {0, 0, 0}, gC[3] = {0, 0, 0};
-    for (int ip = s0; ip < bp.np; ip += S) {
+    for (int ip = sl.b; ip < bp.np; ip += sl.Sb) {
       const PrimPair P = a.prims[bp.poff + ip];
-      for (int kq = 0; kq < kp.np; ++kq) {
+      for (int kq = sl.k; kq < kp.np; kq += sl.Sk) {
         const PrimPair Q = a.prims[kp.poff + kq];
         PrimQ<NR> q;
         prim_setup<NR>(P, Q, geo, q);

@@ -67,13 +67,15 @@ struct MolInfo {
 // Work of one quartet class is a list of canonical quartets (bra pair, ket
 // pair), grouped into sub-tasks of similar primitive counts.  Sub-task t owns
 // quartets [q0, q0+nq) and work items [item0, item0 + S*nq): item
-// item0 + s*nq + g processes quartet q0+g for bra primitive pairs s, s+S, ...
+// item0 + s*nq + g processes quartet q0+g for slice s of its primitive
+// quartets, S = Sb * Sk: bra primitive pairs s % Sb, s % Sb + Sb, ... with ket
+// primitive pairs s / Sb, s / Sb + Sk, ...
 struct SubTask {
   int64_t item0;
   int64_t q0;
   int64_t nq;
   int32_t S;
-  int32_t pad;
+  int32_t Sk;
 };
 
 struct JKArgs {
@@ -105,6 +107,8 @@ struct BraChunk {
   int32_t nbra;
   int32_t ket0;   // first ket pair of the chunk's ket window
   int32_t nket;   // window length when the ket-side J is accumulated in LDS (0: global atomics)
+  int32_t Sk;     // ket part of the primitive split S (powers of two)
+  int32_t pad;
   // partial-sum slab of the chunk (per density): its exchange rows
   // [nbra][ROWS][n_m], then its ket window [nket][NKET]
   int64_t poff;

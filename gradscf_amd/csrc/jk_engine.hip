@@ -1244,6 +1244,44 @@ static int bucket_of(int np) {
   return b;
 }
 
+// Lanes and workgroups a quartet class should at least offer the device, and
+// the fewest primitive quartets worth a lane of their own.  A class with less
+// work than its schedule's target_prim and chunk_items were tuned for runs a
+// few workgroups of long serial primitive chains: the work per lane then
+// shrinks until the class has kFillLanes lanes (one wavefront on half of the
+// chip's SIMDs; the class shares the chip with those of the other streams)
+// and kFillGroups workgroups (one per CU).  Two nonsymmetric densities of
+// (H2O)7 cc-pVDZ took 1803 us a build without the rule, 1228 us with
+// 32768 / 256, 1270 / 1340 us with 65536 lanes / 512 groups, and 1840 us
+// with 262144 / 2048 (more slab flushes and cross-lane sums than the shorter
+// chains save); (H2O)16 and C20H42 builds lie above both lines in their long
+// classes and gain in the short ones (3.29 -> 2.99 and 6.30 -> 6.22 ms).
+constexpr int64_t kFillLanes = 32768;
+constexpr int64_t kFillGroups = 256;
+constexpr int64_t kMinPrim = 2;
+
+// Primitive split S = Sb * Sk (powers of two, S <= 64: the bra-major kernel
+// sums the S slices of a quartet across adjacent lanes) of a sub-task whose
+// bras and kets have np in [npb0, npb1] and [npk0, npk1]: the largest S that
+// leaves `target` primitive quartets per lane, shared between bra and ket so
+// that the longest lane runs the fewest iterations (the bra first on ties).
+static void choose_split(int npb0, int npb1, int npk0, int npk1, int64_t target, SubTask& t) {
+  const int64_t want = ((int64_t)npb1 * npk1 + target - 1) / target;
+  int64_t rounds = (int64_t)npb1 * npk1;
+  t.S = t.Sk = 1;
+  for (int S = 2; S <= 64 && S <= want; S *= 2)
+    for (int Sk = 1; Sk <= S; Sk *= 2) {
+      const int Sb = S / Sk;
+      if (Sb > npb0 || Sk > npk0) continue;
+      const int64_t r = (int64_t)((npb1 + Sb - 1) / Sb) * ((npk1 + Sk - 1) / Sk);
+      if (r < rounds) {
+        rounds = r;
+        t.S = S;
+        t.Sk = Sk;
+      }
+    }
+}
+
 struct PairCand {
   Pair pr;
   int cls, pat, mol;
@@ -1375,11 +1413,10 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
           qc.pk = pk;
           qc.tuning_index = cb * (cb + 1) / 2 + ck;
           const gscf_class_tuning& tu = P.tuning[qc.tuning_index];
-          const int64_t kTargetPrim = tu.target_prim, kChunkItems = tu.chunk_items;
           const int kChunkBrasMax = tu.bras_max;
           qc.nq = 0;
           qc.nitems = 0;
-          struct Pending { std::vector<int64_t> qoff; int bra0, ket0, nbra; int64_t q0, nq; int rk, seg; };
+          struct Pending { std::vector<int64_t> qoff; int bra0, ket0, nbra; int64_t q0, nq; int rk, seg, rb; };
           std::vector<Pending> pend;
           for (int rbi = 0; rbi < (int)runs.size(); ++rbi) {
             const Run& rb = runs[rbi];
@@ -1414,15 +1451,8 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
               SubTask t;
               t.q0 = qc.nq;
               t.nq = nq;
-              const int64_t work = (int64_t)rb.npmax * rk.npmax;
-              // primitive split: a power of two <= 64 (the bra-major kernel
-              // sums the S slices of a quartet across adjacent lanes)
-              const int64_t sreq = std::max<int64_t>(1, std::min<int64_t>(rb.npmin, (work + kTargetPrim - 1) / kTargetPrim));
-              t.S = 1;
-              while (t.S < 64 && 2 * t.S <= sreq) t.S *= 2;
-              t.pad = 0;
-              t.item0 = qc.nitems;
-              qc.nitems += (int64_t)t.S * nq;
+              t.S = t.Sk = 1;
+              t.item0 = 0;
               {
                 // rough work model: primitive quartets weighted by the class's
                 // Cartesian block size, plus a per-quartet digestion term
@@ -1433,17 +1463,39 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
               }
               qc.nq += nq;
               qc.tasks.push_back(t);
-              pend.push_back({std::move(qoff), rb.beg, rk.beg, nbra, t.q0, nq, rki, std::numeric_limits<int>::max()});
+              pend.push_back({std::move(qoff), rb.beg, rk.beg, nbra, t.q0, nq, rki, std::numeric_limits<int>::max(), rbi});
             }
           }
           if (qc.nq == 0) continue;
+          // widths count every contraction column of a shell
+          const int wa = ncart_h(qc.la) * (1 + (pb & 1)), wb = ncart_h(qc.lb) * (1 + (pb >> 1));
+          const int wc = ncart_h(qc.lc) * (1 + (pk & 1)), wd = ncart_h(qc.ld) * (1 + (pk >> 1));
+          const int split = (wa * wb * wc * wd > 36) ? wc * wd : 1;
+          // primitive split and chunk size: the schedule's values, or less
+          // work per lane and per workgroup where the class would otherwise
+          // leave the device idle (kFillLanes, kFillGroups)
+          double lane_work = 0.0;
+          for (const Pending& pd : pend) {
+            const Run &rb = runs[pd.rb], &rk = runs[pd.rk];
+            lane_work += 0.25 * (double)pd.nq * split * (rb.npmin + rb.npmax) * (rk.npmin + rk.npmax);
+          }
+          const int64_t kTargetPrim = std::max<int64_t>(
+              1, std::min<int64_t>(tu.target_prim, (int64_t)std::max(lane_work / kFillLanes, (double)kMinPrim)));
+          int64_t items = 0;
+          for (size_t ti = 0; ti < pend.size(); ++ti) {
+            SubTask& t = qc.tasks[ti];
+            const Run &rb = runs[pend[ti].rb], &rk = runs[pend[ti].rk];
+            choose_split(rb.npmin, rb.npmax, rk.npmin, rk.npmax, kTargetPrim, t);
+            t.item0 = qc.nitems;
+            qc.nitems += (int64_t)t.S * t.nq;
+            items += (int64_t)t.S * t.nq * split;
+          }
+          const int64_t fill_items = (items / kFillGroups + tu.threads - 1) / tu.threads * tu.threads;
+          const int64_t kChunkItems =
+              std::min<int64_t>(tu.chunk_items, std::max<int64_t>(tu.threads, fill_items));
           if (with_chunks) {
-            // bra-major chunks: consecutive bras of one sub-task, bounded LDS slots and lane-items;
-            // widths count every contraction column of a shell
-            const int wa = ncart_h(qc.la) * (1 + (pb & 1)), wb = ncart_h(qc.lb) * (1 + (pb >> 1));
-            const int wc = ncart_h(qc.lc) * (1 + (pk & 1)), wd = ncart_h(qc.ld) * (1 + (pk >> 1));
+            // bra-major chunks: consecutive bras of one sub-task, bounded LDS slots and lane-items
             const int rows = wa + wb;
-            const int split = (wa * wb * wc * wd > 36) ? wc * wd : 1;
             // full-block classes stage their chunk's bra primitive pairs in
             // LDS (kStagedPrim doubles each, kStagedPrimCoef with bra columns)
             const bool stage = split == 1;
@@ -1495,6 +1547,7 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
                     c.q0 = t.q0 + pd.qoff[b] + k0;
                     c.nq = (int32_t)std::min<int64_t>(step, cnt - k0);
                     c.S = t.S;
+                    c.Sk = t.Sk;
                     c.bra0 = pd.bra0 + b;
                     c.nbra = 1;
                     c.ket0 = pd.ket0 + (int32_t)k0;
@@ -1507,6 +1560,7 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
                 BraChunk c;
                 c.q0 = t.q0 + pd.qoff[b];
                 c.S = t.S;
+                c.Sk = t.Sk;
                 c.bra0 = pd.bra0 + b;
                 int64_t items = 0;
                 int e = b;

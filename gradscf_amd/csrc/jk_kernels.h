@@ -22,18 +22,26 @@
 
 namespace gscf {
 
-// Work item -> (quartet index, primitive split index s, split count S).
-__device__ __forceinline__ void map_item(const JKArgs& a, int64_t item, int64_t& g, int& s, int& S) {
-  int lo = 0, hi = a.ntasks;  // tasks[lo].item0 <= item < tasks[hi].item0
+// First primitive pairs and strides of one slice of a quartet's primitive
+// quartets: bra pairs b, b + Sb, ... with ket pairs k, k + Sk, ...
+struct PrimSlice {
+  int b, Sb, k, Sk;
+};
+
+// Work item -> quartet index and its slice.
+__device__ __forceinline__ PrimSlice map_item(const SubTask* __restrict__ tasks, int ntasks, int64_t item,
+                                              int64_t& g) {
+  int lo = 0, hi = ntasks;  // tasks[lo].item0 <= item < tasks[hi].item0
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
-    if (a.tasks[mid].item0 <= item) lo = mid; else hi = mid;
+    if (tasks[mid].item0 <= item) lo = mid; else hi = mid;
   }
-  const SubTask t = a.tasks[lo];
+  const SubTask t = tasks[lo];
   const int64_t r = item - t.item0;
-  s = (int)(r / t.nq);
+  const int s = (int)(r / t.nq);
   g = t.q0 + (r - (int64_t)s * t.nq);
-  S = t.S;
+  const int Sb = t.S / t.Sk;
+  return {s & (Sb - 1), Sb, s / Sb, t.Sk};
 }
 
 template <int LA, int LB, int LC, int LD>
@@ -330,8 +338,7 @@ __global__ __launch_bounds__(256) void jk_full_kernel(JKArgs a) {
   const int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (item >= a.nitems) return;
   int64_t g;
-  int s0, S;
-  map_item(a, item, g, s0, S);
+  const PrimSlice sl = map_item(a.tasks, a.ntasks, item, g);
   const int2 qk = a.quartets[g];
   const Pair bp = a.pairs[qk.x];
   const Pair kp = a.pairs[qk.y];
@@ -348,9 +355,9 @@ __global__ __launch_bounds__(256) void jk_full_kernel(JKArgs a) {
       for (int ic = 0; ic < K::NC; ++ic)
 #pragma unroll
         for (int id = 0; id < K::ND; ++id) acc[ia][ib][ic][id] = 0.0;
-  for (int ip = s0; ip < bp.np; ip += S) {
+  for (int ip = sl.b; ip < bp.np; ip += sl.Sb) {
     const PrimPair P = a.prims[bp.poff + ip];
-    for (int kq = 0; kq < kp.np; ++kq) {
+    for (int kq = sl.k; kq < kp.np; kq += sl.Sk) {
       const PrimPair Q = a.prims[kp.poff + kq];
       PrimQ<K::NR> q;
       prim_setup<K::NR>(P, Q, geo, q);
@@ -476,8 +483,7 @@ __global__ __launch_bounds__(256) void jk_split_kernel(JKArgs a) {
   const int kc = (int)(t - item * K::SPLIT);
   const int ic = kc / K::ND, id = kc - (kc / K::ND) * K::ND;
   int64_t g;
-  int s0, S;
-  map_item(a, item, g, s0, S);
+  const PrimSlice sl = map_item(a.tasks, a.ntasks, item, g);
   const int2 qk = a.quartets[g];
   const Pair bp = a.pairs[qk.x];
   const Pair kp = a.pairs[qk.y];
@@ -496,9 +502,9 @@ __global__ __launch_bounds__(256) void jk_split_kernel(JKArgs a) {
   for (int ia = 0; ia < K::NA; ++ia)
 #pragma unroll
     for (int ib = 0; ib < K::NB; ++ib) acc[ia][ib] = 0.0;
-  for (int ip = s0; ip < bp.np; ip += S) {
+  for (int ip = sl.b; ip < bp.np; ip += sl.Sb) {
     const PrimPair P = a.prims[bp.poff + ip];
-    for (int kq = 0; kq < kp.np; ++kq) {
+    for (int kq = sl.k; kq < kp.np; kq += sl.Sk) {
       const PrimPair Q = a.prims[kp.poff + kq];
       PrimQ<K::NR> q;
       prim_setup<K::NR>(P, Q, geo, q);
@@ -608,7 +614,8 @@ struct Wide {
 };
 
 // One work item of the bra-major kernel in real type R: evaluate the quartet
-// (or its wide ket-component slice) over bra primitive pairs s0, s0+S, ... and
+// (or its wide ket-component slice) over slice s0 of S of its primitive
+// quartets (Sk slices of the ket primitive pairs, the bra slice fastest) and
 // digest it (exchange rows / bra J block into LDS, ket J block into the LDS
 // window or to global).  With general contraction each primitive quartet is
 // evaluated once, coefficient-free, and added to every column combination
@@ -619,7 +626,7 @@ struct Wide {
 template <int LA, int LB, int LC, int LD, int CA, int CB, int CC, int CD, bool MOMENTS, typename R, int MODE = 0,
           bool DET = false>
 __device__ __forceinline__ void bra_item(const BraArgs& a, const MolInfo& mi, const Pair& bp, const Pair& kp,
-                                         const int2 qk, int slot, int s0, int S, int kc, double* __restrict__ krow,
+                                         const int2 qk, int slot, int s0, int S, int Sk, int kc, double* __restrict__ krow,
                                          double* __restrict__ jrow, double* __restrict__ jket, int kwin0,
                                          const double* __restrict__ tab, double* __restrict__ cq,
                                          double dscale = 1.0, const double* __restrict__ bpl = nullptr,
@@ -629,6 +636,7 @@ __device__ __forceinline__ void bra_item(const BraArgs& a, const MolInfo& mi, co
   constexpr int WA = W::WA, WB = W::WB, WC = W::WC, WD = W::WD;
   constexpr int ROWS = WA + WB;
   const int ns = a.n;  // LDS row length
+  const int Sb = S / Sk, sb = s0 & (Sb - 1), sk = s0 / Sb;
   const ShellXYZ sA = a.shells[bp.sa], sB = a.shells[bp.sb], sC = a.shells[kp.sa], sD = a.shells[kp.sb];
   // digestion addresses: molecule bases are chunk-uniform (scalar), element
   // offsets 32-bit (n <= 16384 Cartesian AOs per molecule, checked at plan
@@ -664,13 +672,13 @@ __device__ __forceinline__ void bra_item(const BraArgs& a, const MolInfo& mi, co
     const bool staged = bpl != nullptr;
     // staged bra primitives: ket primitives outermost (one memory read of
     // each per lane), the chunk's bra primitives from LDS inside
-    for (int kq = 0; staged && kq < kp.np; ++kq) {
+    for (int kq = sk; staged && kq < kp.np; kq += Sk) {
       const PrimPair Q = a.prims[kp.poff + kq];
       // ket primitive relative to the bra's first centre and its own
       const double QA[3] = {Q.px - geo.A[0], Q.py - geo.A[1], Q.pz - geo.A[2]};
       const double QC[3] = {Q.px - geo.C[0], Q.py - geo.C[1], Q.pz - geo.C[2]};
       if constexpr (!W::GEN) {
-        for (int ip = s0; ip < bp.np; ip += S)
+        for (int ip = sb; ip < bp.np; ip += Sb)
           staged_quartet<LA, LB, LC, LD, MOMENTS, R>(bpl + ip * kStagedPrim, Q, QA, QC, AB, CD_, tab, acc);
       } else {
         // general contraction: coefficient-free blocks summed over the bra
@@ -680,7 +688,7 @@ __device__ __forceinline__ void bra_item(const BraArgs& a, const MolInfo& mi, co
         R tmp[WA][WB][K::NC][K::ND];
 #pragma unroll
         for (int e = 0; e < WA * WB * K::NC * K::ND; ++e) (&tmp[0][0][0][0])[e] = R(0);
-        for (int ip = s0; ip < bp.np; ip += S) {
+        for (int ip = sb; ip < bp.np; ip += Sb) {
           const double* __restrict__ r = bpl + ip * REC;
           R blk[K::NA][K::NB][K::NC][K::ND];
 #pragma unroll
@@ -722,13 +730,13 @@ __device__ __forceinline__ void bra_item(const BraArgs& a, const MolInfo& mi, co
       }
     }
     if (!staged)
-    for (int ip = s0; ip < bp.np; ip += S) {
+    for (int ip = sb; ip < bp.np; ip += Sb) {
       const PrimPair P = a.prims[bp.poff + ip];
       // a side with one column already carries its coefficients in e
       PrimCoef cP = {{1.0, 0.0}, {1.0, 0.0}};
       if constexpr (CA * CB > 1) cP = a.coef[bp.poff + ip];
       const PrimPair* __restrict__ kpr = a.prims + kp.poff;
-      for (int kq = 0; kq < kp.np; ++kq) {
+      for (int kq = sk; kq < kp.np; kq += Sk) {
         const PrimPair Q = kpr[kq];
         PrimQ<K::NR> q;
         prim_setup<K::NR, MOMENTS>(P, Q, geo, q, tab);
@@ -907,12 +915,12 @@ __device__ __forceinline__ void bra_item(const BraArgs& a, const MolInfo& mi, co
     for (int ia = 0; ia < WA; ++ia)
 #pragma unroll
       for (int ib = 0; ib < WB; ++ib) acc[ia][ib] = R(0);
-    for (int ip = s0; ip < bp.np; ip += S) {
+    for (int ip = sb; ip < bp.np; ip += Sb) {
       const PrimPair P = a.prims[bp.poff + ip];
       PrimCoef cP = {{1.0, 0.0}, {1.0, 0.0}};
       if constexpr (CA * CB > 1) cP = a.coef[bp.poff + ip];
       const PrimPair* __restrict__ kpr = a.prims + kp.poff;
-      for (int kq = 0; kq < kp.np; ++kq) {
+      for (int kq = sk; kq < kp.np; kq += Sk) {
         const PrimPair Q = kpr[kq];
         PrimQ<K::NR> q;
         prim_setup<K::NR, MOMENTS>(P, Q, geo, q, tab);
@@ -1149,15 +1157,17 @@ __global__ __launch_bounds__(512) void jk_bra_kernel(BraArgs a) {
   // walk the kets in the same order make their ket-side J atomics collide on
   // the same addresses at the same time (the memory-side atomic unit then
   // serialises them).
-  const int S = MODE == 2 ? 1 : ch.S;
-  const int64_t total = (int64_t)ch.nq * S * W::SPLIT;
-  const int64_t rot = ((int64_t)blockIdx.x * 40503) % ch.nq;
+  // (a chunk holds at most 2^20 lane-items, or one quartet's 64 * 36: 32 bits)
+  const int S = MODE == 2 ? 1 : ch.S, Sk = MODE == 2 ? 1 : ch.Sk;
+  const int lgS = __ffs(S) - 1;
+  const int total = ch.nq * S * W::SPLIT;
+  const int rot = (int)((unsigned)(blockIdx.x * 40503u) % (unsigned)ch.nq);
   constexpr int kBlock = W::kSplit ? W::NBRA : W::NBRA * W::NKET;
-  for (int64_t it = threadIdx.x; it < total; it += blockDim.x) {
-    const int s0 = (int)(it & (S - 1));
-    const int64_t rest = it / S;
-    const int kc = (int)(rest % W::SPLIT);
-    int64_t qr = rest / W::SPLIT + rot;
+  for (int it = threadIdx.x; it < total; it += blockDim.x) {
+    const int s0 = it & (S - 1);
+    const int rest = it >> lgS;
+    const int kc = rest % W::SPLIT;
+    int qr = rest / W::SPLIT + rot;
     if (qr >= ch.nq) qr -= ch.nq;
     const int64_t g = ch.q0 + qr;
     const int2 qk = a.quartets[g];
@@ -1184,13 +1194,13 @@ __global__ __launch_bounds__(512) void jk_bra_kernel(BraArgs a) {
     if constexpr (MIX) {
       if (lowp) {
         bra_item<LA, LB, LC, LD, CA, CB, CC, CD, kMoments, float>(
-            a, mi, bp, kp, qk, slot, s0, S, kc, krow, jrow, jket, ch.ket0, tab, cq, 1.0,
+            a, mi, bp, kp, qk, slot, s0, S, Sk, kc, krow, jrow, jket, ch.ket0, tab, cq, 1.0,
             (kStage && a.bra_stage) ? bstage + kRec * bslot[slot] : nullptr, dabs);
         continue;
       }
     }
     const double* bpl = (kStage && a.bra_stage) ? bstage + kRec * bslot[slot] : nullptr;
-    bra_item<LA, LB, LC, LD, CA, CB, CC, CD, kMoments, double, MODE, DET>(a, mi, bp, kp, qk, slot, s0, S, kc, krow,
+    bra_item<LA, LB, LC, LD, CA, CB, CC, CD, kMoments, double, MODE, DET>(a, mi, bp, kp, qk, slot, s0, S, Sk, kc, krow,
                                                                            jrow, jket, ch.ket0, tab, cq, dscale, bpl,
                                                                            dabs);
   }

@@ -38,19 +38,7 @@ __global__ __launch_bounds__(256) void param_kernel(ParamArgs a) {
     const int kc = (int)(t - item * NKET);
     const int ic = kc / ND, id = kc - (kc / ND) * ND;
     int64_t g;
-    int s0, S;
-    {
-      int lo = 0, hi = a.ntasks;
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (a.tasks[mid].item0 <= item) lo = mid; else hi = mid;
-      }
-      const SubTask tk = a.tasks[lo];
-      const int64_t r = item - tk.item0;
-      s0 = (int)(r / tk.nq);
-      g = tk.q0 + (r - (int64_t)s0 * tk.nq);
-      S = tk.S;
-    }
+    const PrimSlice sl = map_item(a.tasks, a.ntasks, item, g);
     const int2 qk = a.quartets[g];
     const Pair bp = a.pairs[qk.x];
     const Pair kp = a.pairs[qk.y];
@@ -102,11 +90,11 @@ __global__ __launch_bounds__(256) void param_kernel(ParamArgs a) {
     }
     const int pA = a.seg_prim0[bp.sa], pB = a.seg_prim0[bp.sb];
     const int pC = a.seg_prim0[kp.sa], pD = a.seg_prim0[kp.sb];
-    for (int ip = s0; ip < bp.np; ip += S) {
+    for (int ip = sl.b; ip < bp.np; ip += sl.Sb) {
       PrimPair P = a.prims[bp.poff + ip];
       const PrimAux xP = a.aux[bp.poff + ip];
       P.e = xP.ek;  // coefficient-free bra factor
-      for (int kq = 0; kq < kp.np; ++kq) {
+      for (int kq = sl.k; kq < kp.np; kq += sl.Sk) {
         PrimPair Q = a.prims[kp.poff + kq];
         const PrimAux xQ = a.aux[kp.poff + kq];
         Q.e = xQ.ek;
