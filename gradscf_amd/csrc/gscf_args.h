@@ -61,6 +61,11 @@ struct MolInfo {
   int64_t dbase;
   int32_t n;
   int32_t nseg;
+  int32_t nuc0;   // nuclei of the molecule: [nuc0, nuc0 + nnuc) of the plan's list
+  int32_t nnuc;
+  int64_t sbase;  // the molecule's matrix in the requested AO basis, ns x ns
+  int32_t ns;
+  int32_t pad;
 };
 
 

@@ -3,100 +3,204 @@
 // reference performs on the CPU before its SCF loop (src/gradscf/integrals/
 // _native/csrc/ffi.cc:11-86 via libcint cint1e.c and autocode/intor1.c).
 //
-// One lane per segmented shell pair (all classes with l <= 2).  Overlap and
+// One wavefront per segmented shell pair (all classes with l <= 2).  Overlap and
 // kinetic from 1D Obara-Saika tables; nuclear attraction by Rys quadrature with
 // a point charge, (a|1/r_C|b) = 2 pi/p K_AB sum_r w_r Ix Iy Iz, with
 // C00 = (P - A) - (P - C) u and B10 = (1 - u)/(2p).
+#include <algorithm>
+
 #include "gscf_device.h"
 
 namespace gscf {
+
+// Lanes of a pair's wavefront over (nucleus, primitive pair): W lanes (a power
+// of two) take W consecutive nuclei, the 64 / W groups of W lanes alternate
+// over the primitive pairs.  What bounds these kernels is the length of a
+// lane's chain of Rys evaluations (each one dependent gathers of the root
+// table and an FP64 recurrence): with one lane per pair a pair of contracted
+// s shells ran 64 primitive pairs x 48 nuclei = 3072 evaluations in a row for
+// (H2O)16 cc-pVDZ while most of the chip idled; a wavefront runs them in 64
+// rounds (of which 48 lanes are busy).  (H2O)16 cc-pVDZ, the six classes: S, T,
+// V 2.1 -> 0.12 ms (ss 949 -> 29 us), the gradient 11.5 -> 0.18 ms (ss 5380 ->
+// 57 us).
+struct NucLanes {
+  int W, c, grp, ngrp;
+};
+
+__device__ __forceinline__ NucLanes nuc_lanes(int lane, int nnuc) {
+  int W = 1;
+  while (W < nnuc && W < 64) W <<= 1;
+  return {W, lane & (W - 1), lane / W, 64 / W};
+}
+
+template <typename R>
+__device__ __forceinline__ R wave_sum(R v) {
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m);
+  return v;
+}
+
+// Real solid harmonics of l <= 2 as sums of Cartesian components, in
+// libcint's order and normalisation (identity for s and p).
+template <int L, bool SPH>
+__host__ __device__ constexpr int nfun() { return SPH ? 2 * L + 1 : ncart(L); }
+
+template <int L, bool SPH>
+__host__ __device__ constexpr double c2s_coef(int m, int i) {
+  if (!SPH || L < 2) return m == i ? 1.0 : 0.0;
+  constexpr double a = 1.0925484305920792;    // sqrt(15 / (4 pi))
+  constexpr double b = 0.31539156525252005;   // sqrt(5 / (16 pi))
+  constexpr double c = 0.5462742152960396;    // sqrt(15 / (16 pi))
+  switch (m) {  // components xx, xy, xz, yy, yz, zz
+    case 0: return i == 1 ? a : 0.0;
+    case 1: return i == 4 ? a : 0.0;
+    case 2: return (i == 0 || i == 3) ? -b : (i == 5 ? 2.0 * b : 0.0);
+    case 3: return i == 2 ? a : 0.0;
+    default: return i == 0 ? c : (i == 3 ? -c : 0.0);
+  }
+}
 
 struct Int1eArgs {
   const Pair* pairs;
   const PrimPair* prims;
   const ShellXYZ* shells;
+  const int* shell_ao;    // first AO of every segmented shell in the requested basis
   const double* nuclei;   // [nnuc][6]: x, y, z, Z, molecule, atm row
-  int nnuc;
   int npairs;
-  const MolInfo* mols;    // Cartesian matrix of each molecule
-  double* s;
+  const MolInfo* mols;
+  double* s;              // matrices in the requested AO basis
   double* t;
   double* v;
 };
 
-template <int LA, int LB>
+// Writes one matrix's block: every lane holds the block's sums, so lane
+// (p, q) transforms and stores element (p, q) and its transpose.
+template <int LA, int LB, bool SPH>
+__device__ __forceinline__ void store_block(const double (&acc)[ncart(LA)][ncart(LB)], double* __restrict__ out, int n,
+                                            int oa, int ob, bool diag, int lane) {
+  constexpr int WB = nfun<LB, SPH>();
+#pragma unroll
+  for (int p = 0; p < nfun<LA, SPH>(); ++p)
+#pragma unroll
+    for (int q = 0; q < WB; ++q) {
+      double x = 0.0;
+#pragma unroll
+      for (int i = 0; i < ncart(LA); ++i)
+#pragma unroll
+        for (int j = 0; j < ncart(LB); ++j) {
+          constexpr double one = 1.0;
+          const double f = c2s_coef<LA, SPH>(p, i) * c2s_coef<LB, SPH>(q, j);
+          if (f == one) x += acc[i][j];
+          else if (f != 0.0) x += f * acc[i][j];
+        }
+      if (lane == p * WB + q) {
+        out[(size_t)(oa + p) * n + ob + q] = x;
+        if (!diag) out[(size_t)(ob + q) * n + oa + p] = x;
+      }
+    }
+}
+
+// The transform to the requested basis acts inside a shell pair's block, so
+// the kernel stores final matrix elements: no Cartesian staging matrices, no
+// transform pass.
+template <int LA, int LB, bool SPH>
 __global__ __launch_bounds__(256) void int1e_kernel(Int1eArgs a) {
   constexpr int NA = ncart(LA), NB = ncart(LB);
   constexpr int NR = (LA + LB) / 2 + 1;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int i = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (i >= a.npairs) return;
   const Pair pr = a.pairs[i];
   const ShellXYZ A = a.shells[pr.sa], B = a.shells[pr.sb];
+  const MolInfo mi = a.mols[A.mol];
   const double Ar[3] = {A.x, A.y, A.z}, Br[3] = {B.x, B.y, B.z};
-  double accS[NA][NB], accT[NA][NB], accV[NA][NB];
-#pragma unroll
-  for (int ia = 0; ia < NA; ++ia)
-#pragma unroll
-    for (int ib = 0; ib < NB; ++ib) accS[ia][ib] = accT[ia][ib] = accV[ia][ib] = 0.0;
   const double pi = 3.14159265358979323846;
   const double s2p = sqrt(2.0 * pi * pi * sqrt(pi));
-  for (int ip = 0; ip < pr.np; ++ip) {
-    const PrimPair P = a.prims[pr.poff + ip];
-    const double p = P.p, ip2 = 0.5 / P.p;
-    const double Pr[3] = {P.px, P.py, P.pz};
-    const double ckab = P.e * p / s2p;  // c_a c_b K_AB
-    const double aj = P.ab;
-    // 1D overlap tables S[x][a][b], a <= LA, b <= LB + 2 (unit base; (pi/p)^{3/2} applied below)
-    double S1[3][LA + 1][LB + 3];
+  const int oa = a.shell_ao[pr.sa], ob = a.shell_ao[pr.sb];
+  const bool diag = pr.sa == pr.sb;
+  {
+    double accS[NA][NB], accT[NA][NB];
 #pragma unroll
-    for (int x = 0; x < 3; ++x) {
-      const double pa = Pr[x] - Ar[x], pb = Pr[x] - Br[x];
+    for (int ia = 0; ia < NA; ++ia)
 #pragma unroll
-      for (int ia = 0; ia <= LA; ++ia)
+      for (int ib = 0; ib < NB; ++ib) accS[ia][ib] = accT[ia][ib] = 0.0;
+    for (int ip = lane; ip < pr.np; ip += 64) {
+      const PrimPair P = a.prims[pr.poff + ip];
+      const double p = P.p, ip2 = 0.5 / P.p;
+      const double Pr[3] = {P.px, P.py, P.pz};
+      const double ckab = P.e * p / s2p;  // c_a c_b K_AB
+      const double aj = P.ab;
+      // 1D overlap tables S[x][a][b], a <= LA, b <= LB + 2 (unit base; (pi/p)^{3/2} applied below)
+      double S1[3][LA + 1][LB + 3];
 #pragma unroll
-        for (int ib = 0; ib <= LB + 2; ++ib) {
-          double val;
-          if (ia == 0 && ib == 0) {
-            val = 1.0;
-          } else if (ia > 0) {
-            val = pa * S1[x][ia - 1][ib];
-            if (ia > 1) val += (ia - 1) * ip2 * S1[x][ia - 2][ib];
-            if (ib > 0) val += ib * ip2 * S1[x][ia - 1][ib - 1];
-          } else {
-            val = pb * S1[x][0][ib - 1];
-            if (ib > 1) val += (ib - 1) * ip2 * S1[x][0][ib - 2];
+      for (int x = 0; x < 3; ++x) {
+        const double pa = Pr[x] - Ar[x], pb = Pr[x] - Br[x];
+#pragma unroll
+        for (int ia = 0; ia <= LA; ++ia)
+#pragma unroll
+          for (int ib = 0; ib <= LB + 2; ++ib) {
+            double val;
+            if (ia == 0 && ib == 0) {
+              val = 1.0;
+            } else if (ia > 0) {
+              val = pa * S1[x][ia - 1][ib];
+              if (ia > 1) val += (ia - 1) * ip2 * S1[x][ia - 2][ib];
+              if (ib > 0) val += ib * ip2 * S1[x][ia - 1][ib - 1];
+            } else {
+              val = pb * S1[x][0][ib - 1];
+              if (ib > 1) val += (ib - 1) * ip2 * S1[x][0][ib - 2];
+            }
+            S1[x][ia][ib] = val;
           }
-          S1[x][ia][ib] = val;
+      }
+      const double sfac = ckab * (pi / p) * sqrt(pi / p);
+#pragma unroll
+      for (int ia = 0; ia < NA; ++ia)
+#pragma unroll
+        for (int ib = 0; ib < NB; ++ib) {
+          int ea[3] = {cart_comp(LA, ia, 0), cart_comp(LA, ia, 1), cart_comp(LA, ia, 2)};
+          int eb[3] = {cart_comp(LB, ib, 0), cart_comp(LB, ib, 1), cart_comp(LB, ib, 2)};
+          const double sx = S1[0][ea[0]][eb[0]], sy = S1[1][ea[1]][eb[1]], sz = S1[2][ea[2]][eb[2]];
+          double tk = 0.0;
+#pragma unroll
+          for (int x = 0; x < 3; ++x) {
+            const int bx = eb[x];
+            double tx = -2.0 * aj * aj * S1[x][ea[x]][bx + 2] + aj * (2 * bx + 1) * S1[x][ea[x]][bx];
+            if (bx > 1) tx -= 0.5 * bx * (bx - 1) * S1[x][ea[x]][bx - 2];
+            tk += tx * (x == 0 ? sy * sz : (x == 1 ? sx * sz : sx * sy));
+          }
+          accS[ia][ib] += sfac * sx * sy * sz;
+          accT[ia][ib] += sfac * tk;
         }
     }
-    const double sfac = ckab * (pi / p) * sqrt(pi / p);
 #pragma unroll
     for (int ia = 0; ia < NA; ++ia)
 #pragma unroll
       for (int ib = 0; ib < NB; ++ib) {
-        int ea[3] = {cart_comp(LA, ia, 0), cart_comp(LA, ia, 1), cart_comp(LA, ia, 2)};
-        int eb[3] = {cart_comp(LB, ib, 0), cart_comp(LB, ib, 1), cart_comp(LB, ib, 2)};
-        const double sx = S1[0][ea[0]][eb[0]], sy = S1[1][ea[1]][eb[1]], sz = S1[2][ea[2]][eb[2]];
-        double tk = 0.0;
-#pragma unroll
-        for (int x = 0; x < 3; ++x) {
-          const int bx = eb[x];
-          double tx = -2.0 * aj * aj * S1[x][ea[x]][bx + 2] + aj * (2 * bx + 1) * S1[x][ea[x]][bx];
-          if (bx > 1) tx -= 0.5 * bx * (bx - 1) * S1[x][ea[x]][bx - 2];
-          tk += tx * (x == 0 ? sy * sz : (x == 1 ? sx * sz : sx * sy));
-        }
-        accS[ia][ib] += sfac * sx * sy * sz;
-        accT[ia][ib] += sfac * tk;
+        accS[ia][ib] = wave_sum(accS[ia][ib]);
+        accT[ia][ib] = wave_sum(accT[ia][ib]);
       }
-    // nuclear attraction
-    for (int c = 0; c < a.nnuc; ++c) {
-      const double* C = a.nuclei + 6 * c;
-      if ((int)C[4] != A.mol) continue;
-      const double pc[3] = {Pr[0] - C[0], Pr[1] - C[1], Pr[2] - C[2]};
+    store_block<LA, LB, SPH>(accS, a.s + mi.sbase, mi.ns, oa, ob, diag, lane);
+    store_block<LA, LB, SPH>(accT, a.t + mi.sbase, mi.ns, oa, ob, diag, lane);
+  }
+  double accV[NA][NB];
+#pragma unroll
+  for (int ia = 0; ia < NA; ++ia)
+#pragma unroll
+    for (int ib = 0; ib < NB; ++ib) accV[ia][ib] = 0.0;
+  const NucLanes nl = nuc_lanes(lane, mi.nnuc);
+  for (int c = nl.c; c < mi.nnuc; c += nl.W) {
+    const double* C = a.nuclei + 6 * (mi.nuc0 + c);
+    const double Cx[3] = {C[0], C[1], C[2]}, Z = C[3];
+    for (int ip = nl.grp; ip < pr.np; ip += nl.ngrp) {
+      const PrimPair P = a.prims[pr.poff + ip];
+      const double p = P.p, ip2 = 0.5 / P.p;
+      const double Pr[3] = {P.px, P.py, P.pz};
+      const double pc[3] = {Pr[0] - Cx[0], Pr[1] - Cx[1], Pr[2] - Cx[2]};
       const double T = p * (pc[0] * pc[0] + pc[1] * pc[1] + pc[2] * pc[2]);
       double u[NR], w[NR];
       rys_roots<NR>(T, u, w);
-      const double vf = -C[3] * 2.0 * pi / p * ckab;
+      const double vf = -Z * 2.0 * pi / s2p * P.e;  // 2 pi / p c_a c_b K_AB
 #pragma unroll
       for (int r = 0; r < NR; ++r) {
         const double b10 = ip2 * (1.0 - u[r]);
@@ -120,18 +224,11 @@ __global__ __launch_bounds__(256) void int1e_kernel(Int1eArgs a) {
       }
     }
   }
-  const MolInfo mi = a.mols[A.mol];
-  const int nc = mi.n;
 #pragma unroll
   for (int ia = 0; ia < NA; ++ia)
 #pragma unroll
-    for (int ib = 0; ib < NB; ++ib) {
-      const size_t x = mi.base + (size_t)(A.ao + ia) * nc + B.ao + ib;
-      const size_t y = mi.base + (size_t)(B.ao + ib) * nc + A.ao + ia;
-      a.s[x] = accS[ia][ib]; a.s[y] = accS[ia][ib];
-      a.t[x] = accT[ia][ib]; a.t[y] = accT[ia][ib];
-      a.v[x] = accV[ia][ib]; a.v[y] = accV[ia][ib];
-    }
+    for (int ib = 0; ib < NB; ++ib) accV[ia][ib] = wave_sum(accV[ia][ib]);
+  store_block<LA, LB, SPH>(accV, a.v + mi.sbase, mi.ns, oa, ob, diag, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -145,16 +242,21 @@ __global__ __launch_bounds__(256) void int1e_kernel(Int1eArgs a) {
 // invariant (d/dB = -d/dA); for V the B derivative uses the raised b and the
 // derivative with respect to the nucleus C follows from
 // d/dA + d/dB + d/dC = 0 for each nucleus's term (the Hellmann-Feynman force).
-// One lane per segmented shell pair (S >= T); pair factor 2 for S != T with
-// symmetrised D and W.  Per-atom sums in LDS, one flush per workgroup.
+// One wavefront per segmented shell pair (S >= T), its lanes over nuclei and
+// primitive pairs (NucLanes); pair factor 2 for S != T with symmetrised D and
+// W.  A lane keeps its nucleus's force in registers over the primitive pairs.
+// Workgroups are persistent (kGrad1eGroups of four wavefronts, each striding
+// over the pairs): per-atom sums stay in LDS and reach global memory once per
+// workgroup, since every workgroup of a molecule adds into the same rows.
 // ---------------------------------------------------------------------------
+constexpr int kGrad1eGroups = 512;
+
 struct Grad1eArgs {
   const Pair* pairs;
   const PrimPair* prims;
   const ShellXYZ* shells;
   const int* seg_atom;    // atm row of each segmented shell's centre
   const double* nuclei;   // [nnuc][6]: x, y, z, Z, molecule, atm row
-  int nnuc;
   int npairs;
   const MolInfo* mols;
   const double* dens;     // packed Cartesian D
@@ -170,8 +272,8 @@ __global__ __launch_bounds__(256) void grad1e_kernel(Grad1eArgs a) {
   extern __shared__ double gl[];
   for (int i = threadIdx.x; i < 3 * a.natm; i += blockDim.x) gl[i] = 0.0;
   __syncthreads();
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < a.npairs) {
+  const int lane = threadIdx.x & 63, wpg = blockDim.x >> 6;
+  for (int i = blockIdx.x * wpg + (threadIdx.x >> 6); i < a.npairs; i += gridDim.x * wpg) {
     const Pair pr = a.pairs[i];
     const ShellXYZ A = a.shells[pr.sa], B = a.shells[pr.sb];
     const double Ar[3] = {A.x, A.y, A.z}, Br[3] = {B.x, B.y, B.z};
@@ -192,7 +294,7 @@ __global__ __launch_bounds__(256) void grad1e_kernel(Grad1eArgs a) {
     const double pi = 3.14159265358979323846;
     const double s2p = sqrt(2.0 * pi * pi * sqrt(pi));
     double gA[3] = {0, 0, 0}, gB[3] = {0, 0, 0};
-    for (int ip = 0; ip < pr.np; ++ip) {
+    for (int ip = lane; ip < pr.np; ip += 64) {
       const PrimPair P = a.prims[pr.poff + ip];
       const double p = P.p, ip2 = 0.5 / P.p;
       const double Pr[3] = {P.px, P.py, P.pz};
@@ -252,16 +354,23 @@ __global__ __launch_bounds__(256) void grad1e_kernel(Grad1eArgs a) {
             gB[x] -= v;
           }
         }
-      // nuclear attraction: A and B derivatives per nucleus, C by invariance
-      for (int c = 0; c < a.nnuc; ++c) {
-        const double* C = a.nuclei + 6 * c;
-        if ((int)C[4] != A.mol) continue;
-        const double pc[3] = {Pr[0] - C[0], Pr[1] - C[1], Pr[2] - C[2]};
+    }
+    // nuclear attraction: A and B derivatives, the nucleus's by invariance
+    const NucLanes nl = nuc_lanes(lane, mi.nnuc);
+    for (int c = nl.c; c < mi.nnuc; c += nl.W) {
+      const double* C = a.nuclei + 6 * (mi.nuc0 + c);
+      const double Cx[3] = {C[0], C[1], C[2]}, Z = C[3];
+      double cA[3] = {0, 0, 0}, cB[3] = {0, 0, 0};
+      for (int ip = nl.grp; ip < pr.np; ip += nl.ngrp) {
+        const PrimPair P = a.prims[pr.poff + ip];
+        const double p = P.p, ip2 = 0.5 / P.p;
+        const double Pr[3] = {P.px, P.py, P.pz};
+        const double ai = P.aa, aj = P.ab;
+        const double pc[3] = {Pr[0] - Cx[0], Pr[1] - Cx[1], Pr[2] - Cx[2]};
         const double T = p * (pc[0] * pc[0] + pc[1] * pc[1] + pc[2] * pc[2]);
         double u[NR], w[NR];
         rys_roots<NR>(T, u, w);
-        const double vf = -C[3] * 2.0 * pi / p * ckab;
-        double cA[3] = {0, 0, 0}, cB[3] = {0, 0, 0};
+        const double vf = -Z * 2.0 * pi / s2p * P.e;
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
           const double b10 = ip2 * (1.0 - u[r]);
@@ -298,20 +407,23 @@ __global__ __launch_bounds__(256) void grad1e_kernel(Grad1eArgs a) {
               }
             }
         }
-        const int atc = (int)C[5];
+      }
+      const int atc = (int)C[5];
 #pragma unroll
-        for (int x = 0; x < 3; ++x) {
-          gA[x] += cA[x];
-          gB[x] += cB[x];
-          atomicAdd(gl + 3 * atc + x, -(cA[x] + cB[x]));
-        }
+      for (int x = 0; x < 3; ++x) {
+        gA[x] += cA[x];
+        gB[x] += cB[x];
+        atomicAdd(gl + 3 * atc + x, -(cA[x] + cB[x]));
       }
     }
     const int atA = a.seg_atom[pr.sa], atB = a.seg_atom[pr.sb];
 #pragma unroll
     for (int x = 0; x < 3; ++x) {
-      atomicAdd(gl + 3 * atA + x, gA[x]);
-      atomicAdd(gl + 3 * atB + x, gB[x]);
+      const double sA = wave_sum(gA[x]), sB = wave_sum(gB[x]);
+      if (lane == 0) {
+        atomicAdd(gl + 3 * atA + x, sA);
+        atomicAdd(gl + 3 * atB + x, sB);
+      }
     }
   }
   __syncthreads();
@@ -322,12 +434,12 @@ __global__ __launch_bounds__(256) void grad1e_kernel(Grad1eArgs a) {
 }
 
 void launch_grad1e_class(int la, int lb, const Pair* pairs, int npairs, const PrimPair* prims,
-                         const ShellXYZ* shells, const int* seg_atom, const double* nuclei, int nnuc,
+                         const ShellXYZ* shells, const int* seg_atom, const double* nuclei,
                          const MolInfo* mols, const double* dens, const double* wdens, int natm, double* grad,
                          hipStream_t st) {
   if (npairs <= 0) return;
-  Grad1eArgs a{pairs, prims, shells, seg_atom, nuclei, nnuc, npairs, mols, dens, wdens, natm, grad};
-  const dim3 grid((npairs + 255) / 256), block(256);
+  Grad1eArgs a{pairs, prims, shells, seg_atom, nuclei, npairs, mols, dens, wdens, natm, grad};
+  const dim3 grid(std::min(kGrad1eGroups, (npairs + 3) / 4)), block(256);
   const size_t lds = sizeof(double) * 3 * natm;
 #define G1E(A, B)                                                          \
   if (la == A && lb == B) {                                                \
@@ -531,16 +643,19 @@ void launch_param1e_class(int la, int lb, const Pair* pairs, int npairs, const P
 #undef P1E
 }
 
-void launch_int1e_class(int la, int lb, const Pair* pairs, int npairs, const PrimPair* prims,
-                        const ShellXYZ* shells, const double* nuclei, int nnuc, const MolInfo* mols, double* s,
-                        double* t, double* v, hipStream_t st) {
+void launch_int1e_class(int la, int lb, bool sph, const Pair* pairs, int npairs, const PrimPair* prims,
+                        const ShellXYZ* shells, const int* shell_ao, const double* nuclei, const MolInfo* mols,
+                        double* s, double* t, double* v, hipStream_t st) {
   if (npairs <= 0) return;
-  Int1eArgs a{pairs, prims, shells, nuclei, nnuc, npairs, mols, s, t, v};
-  const dim3 grid((npairs + 255) / 256), block(256);
-#define L1E(A, B)                                                          \
-  if (la == A && lb == B) {                                                \
-    hipLaunchKernelGGL((int1e_kernel<A, B>), grid, block, 0, st, a);       \
-    return;                                                                \
+  Int1eArgs a{pairs, prims, shells, shell_ao, nuclei, npairs, mols, s, t, v};
+  const dim3 grid((npairs + 3) / 4), block(256);
+#define L1E(A, B)                                                                      \
+  if (la == A && lb == B) {                                                            \
+    if (sph && A == 2)                                                                 \
+      hipLaunchKernelGGL((int1e_kernel<A, B, A == 2>), grid, block, 0, st, a);         \
+    else                                                                               \
+      hipLaunchKernelGGL((int1e_kernel<A, B, false>), grid, block, 0, st, a);          \
+    return;                                                                            \
   }
   L1E(0, 0) L1E(1, 0) L1E(1, 1) L1E(2, 0) L1E(2, 1) L1E(2, 2)
 #undef L1E

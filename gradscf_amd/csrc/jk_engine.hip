@@ -360,6 +360,7 @@ struct PlanData {
   double* d_det_mol = nullptr;
   double* d_det_scale = nullptr;
   int* d_seg_atom = nullptr; // atm row of each segmented shell
+  int* d_seg_ao = nullptr;   // first AO of each segmented shell in its molecule, requested basis
   // basis-parameter derivatives
   PrimAux* d_aux = nullptr;
   int* d_seg_prim0 = nullptr;
@@ -400,15 +401,15 @@ bool launch_df_blocks_c2(int la, int lb, const BlockArgs& a, hipStream_t s);
 bool launch_df_blocks_c3(int la, int lb, const BlockArgs& a, hipStream_t s);
 bool launch_df_blocks_c4(int la, int lb, const BlockArgs& a, hipStream_t s);
 
-void launch_int1e_class(int la, int lb, const Pair* pairs, int npairs, const PrimPair* prims,
-                        const ShellXYZ* shells, const double* nuclei, int nnuc, const MolInfo* mols, double* s,
-                        double* t, double* v, hipStream_t st);
+void launch_int1e_class(int la, int lb, bool sph, const Pair* pairs, int npairs, const PrimPair* prims,
+                        const ShellXYZ* shells, const int* shell_ao, const double* nuclei, const MolInfo* mols,
+                        double* s, double* t, double* v, hipStream_t st);
 void launch_param1e_class(int la, int lb, const Pair* pairs, int npairs, const PrimPair* prims, const PrimAux* aux,
                           const ShellXYZ* shells, const int* seg_prim0, const double* nuclei, int nnuc,
                           const MolInfo* mols, const double* dens, const double* wdens, int nprim, double* gcoef,
                           double* gexp, hipStream_t st);
 void launch_grad1e_class(int la, int lb, const Pair* pairs, int npairs, const PrimPair* prims,
-                         const ShellXYZ* shells, const int* seg_atom, const double* nuclei, int nnuc,
+                         const ShellXYZ* shells, const int* seg_atom, const double* nuclei,
                          const MolInfo* mols, const double* dens, const double* wdens, int natm, double* grad,
                          hipStream_t st);
 
@@ -685,31 +686,6 @@ __global__ void finalize_kernel(const double* __restrict__ jp, const double* __r
       double v = A[(size_t)P * nc + Q] + B[(size_t)Q * nc + P];
       if (X) v += X[8 * ((size_t)P * nc + Q)] + X[8 * ((size_t)Q * nc + P)];
       s += c1 * c2 * v;
-    }
-  }
-  out[i] = s;
-}
-
-// out[p][q] = sum T[p,P] T[q,Q] M[P][Q] (Cartesian -> requested AO basis), per molecule
-__global__ void sandwich_kernel(const double* __restrict__ Mc, int64_t nn_tot, const MolAO* __restrict__ M, int nmol,
-                                const int* __restrict__ idx, const double* __restrict__ coef,
-                                double* __restrict__ out) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (size_t)nn_tot) return;
-  const MolAO m = M[find_mol(M, nmol, (int64_t)i, 0)];
-  const int rem = (int)((int64_t)i - m.sbase);
-  const int p = rem / m.n, q = rem - (rem / m.n) * m.n;
-  const double* A = Mc + m.cbase;
-  const int gp = m.ao0 + p, gq = m.ao0 + q;
-  double s = 0.0;
-  for (int e1 = 0; e1 < 3; ++e1) {
-    const double c1 = coef[gp * 3 + e1];
-    if (c1 == 0.0) continue;
-    const int P = idx[gp * 3 + e1];
-    for (int e2 = 0; e2 < 3; ++e2) {
-      const double c2 = coef[gq * 3 + e2];
-      if (c2 == 0.0) continue;
-      s += c1 * c2 * A[(size_t)P * m.nc + idx[gq * 3 + e2]];
     }
   }
   out[i] = s;
@@ -2110,6 +2086,10 @@ static void build_plan(PlanData& P, double cutoff, hipStream_t s) {
     std::vector<int> at;
     for (const Seg& g : P.seg) at.push_back(P.bas[g.parent * BAS_SLOTS + ATOM_OF]);
     P.d_seg_atom = dev_upload(at, s);
+    std::vector<int> ao;
+    for (const Seg& g : P.seg)
+      ao.push_back(P.ao[g.parent] - P.mols[g.mol].ao0 + g.ctr * (P.cart ? ncart_h(g.l) : 2 * g.l + 1));
+    P.d_seg_ao = dev_upload(ao, s);
   }
   // J/K pair set: parent shells with their general-contraction columns where
   // the basis has them (and the exchange slabs fit), segmented shells otherwise
@@ -2125,6 +2105,16 @@ static void build_plan(PlanData& P, double cutoff, hipStream_t s) {
       mi[m].dbase = P.mols[m].dbase;
       mi[m].n = P.mols[m].nc;
       mi[m].nseg = P.mols[m].nseg;
+    }
+    for (int m = 0, a0 = 0; m < P.nmol; ++m) {
+      int k = 0;
+      for (int a = P.mol_atm[m]; a < P.mol_atm[m + 1]; ++a) k += P.atm[a * ATM_SLOTS + CHARGE_OF] != 0;
+      mi[m].nuc0 = a0;
+      mi[m].nnuc = k;
+      a0 += k;
+      mi[m].sbase = P.mols[m].sbase;
+      mi[m].ns = P.mols[m].n;
+      mi[m].pad = 0;
     }
     P.d_molinfo = dev_upload(mi, s);
     P.d_molao = dev_upload(P.mols, s);
@@ -2171,7 +2161,7 @@ static int64_t plan_bytes(const PlanData& P, int64_t npairs, int64_t nq, int64_t
   b += part_doubles * (int64_t)sizeof(double) * nbd;
   b += std::min<int64_t>(part_doubles, nq * 48) * (int64_t)sizeof(int64_t) +
        (int64_t)(P.n_cart + npairs + 2) * (int64_t)(2 * sizeof(int64_t) + sizeof(int));
-  b += (int64_t)P.seg.size() * (sizeof(ShellXYZ) + 3 * sizeof(int));         // shells, seg_ao, seg_atom
+  b += (int64_t)P.seg.size() * (sizeof(ShellXYZ) + 4 * sizeof(int));         // shells, blocks, seg_atom, seg_ao
   b += (int64_t)std::max<size_t>(P.prims.size(), 1) * (sizeof(PrimPair) + sizeof(PrimAux));
   b += (int64_t)(P.seg.size() + 1) * sizeof(int);
   for (const Seg& g : P.seg) b += (int64_t)g.np * (sizeof(int2) + 3 * sizeof(double));  // slots, fsp, sums
@@ -2251,7 +2241,7 @@ static void free_plan(PlanData& P) {
   f(P.d_c2s_idx); f(P.d_c2s_coef); f(P.d_s2c_idx); f(P.d_s2c_coef);
   f(P.d_dc); f(P.d_jp); f(P.d_jpad); f(P.d_kp); f(P.d_flag); f(P.d_incore); f(P.d_part);
   f(P.d_pairs1e); f(P.d_nuclei);
-  f(P.d_dmax); f(P.d_seg_atom);
+  f(P.d_dmax); f(P.d_seg_atom); f(P.d_seg_ao);
   f(P.d_det_qblk); f(P.d_det_mol); f(P.d_det_scale);
   f(P.d_molinfo); f(P.d_molao);
   f(P.d_aux); f(P.d_seg_prim0); f(P.d_prim_slots); f(P.d_prim_fsp); f(P.d_gparam);
@@ -2711,23 +2701,14 @@ static void incore_set(PlanData& P, int enable, hipStream_t s) {
 
 static void int1e(PlanData& P, double* s_out, double* t_out, double* v_out, hipStream_t st) {
   if (!s_out || !t_out || !v_out) throw InvalidArgument("int1e requires three device output buffers");
-  const size_t ncc = (size_t)P.ncc_tot;
-  double* tmp = nullptr;
-  HIP_OK(hipMalloc(&tmp, sizeof(double) * 3 * ncc));
-  hipLaunchKernelGGL(fill_kernel, dim3(nblocks(3 * ncc)), dim3(256), 0, st, tmp, 3 * ncc, 0.0);
   static const int pl[kNumPairClasses][2] = {{0, 0}, {1, 0}, {1, 1}, {2, 0}, {2, 1}, {2, 2}};
   for (int c = 0; c < kNumPairClasses; ++c) {
     const int b = P.p1e_begin[c], e = P.p1e_begin[c + 1];
-    launch_int1e_class(pl[c][0], pl[c][1], P.d_pairs1e + b, e - b, P.d_prims, P.d_shells, P.d_nuclei, P.nnuc,
-                       P.d_molinfo, tmp, tmp + ncc, tmp + 2 * ncc, st);
+    launch_int1e_class(pl[c][0], pl[c][1], !P.cart, P.d_pairs1e + b, e - b, P.d_prims, P.d_shells, P.d_seg_ao,
+                       P.d_nuclei, P.d_molinfo, s_out, t_out, v_out, st);
   }
-  double* outs[3] = {s_out, t_out, v_out};
-  for (int k = 0; k < 3; ++k)
-    hipLaunchKernelGGL(sandwich_kernel, dim3(nblocks((size_t)P.nn_tot)), dim3(256), 0, st, tmp + k * ncc,
-                       P.nn_tot, P.d_molao, P.nmol, P.d_s2c_idx, P.d_s2c_coef, outs[k]);
   HIP_OK(hipGetLastError());
   HIP_OK(hipStreamSynchronize(st));
-  HIP_OK(hipFree(tmp));
 }
 
 // One-electron gradient sum D d(T+V)/dR - W dS/dR into grad[natm][3] (+=).
@@ -2744,7 +2725,7 @@ static void int1e_gradient(PlanData& P, const double* dens, const double* wdens,
   for (int c = 0; c < kNumPairClasses; ++c) {
     const int b = P.p1e_begin[c], e = P.p1e_begin[c + 1];
     launch_grad1e_class(pl[c][0], pl[c][1], P.d_pairs1e + b, e - b, P.d_prims, P.d_shells, P.d_seg_atom, P.d_nuclei,
-                        P.nnuc, P.d_molinfo, P.d_dc, P.d_dc + ncc, P.natm, grad, s);
+                        P.d_molinfo, P.d_dc, P.d_dc + ncc, P.natm, grad, s);
   }
   HIP_OK(hipGetLastError());
 }
