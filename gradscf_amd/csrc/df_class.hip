@@ -1,26 +1,151 @@
-// Block kernels of the density-fitting integrals, one auxiliary angular
-// momentum per translation unit (built with -DGSCF_DF_LC=0..4): orbital pairs
-// (LA, LB) with LA <= 2, LB <= LA, and auxiliary "pairs" (LA, s0) with LA <= 4
-// (an auxiliary shell times the unit function), against one auxiliary shell
-// (LC, s0).
+// Two- and three-centre density-fitting integrals, one auxiliary angular
+// momentum LC of the ket per translation unit (built with -DGSCF_DF_LC=0..4).
+//
+// A one-centre factor P(r) is the pair of P with a unit function (one
+// exponent-0 s primitive), so both kinds are quartets (A B|C u): orbital pairs
+// (l <= 2) for three centres, (A, u) with A an auxiliary shell (l <= 4) for
+// two.  The tasks of a launch are all (bra pair, ket shell) combinations of
+// every bra class, enumerated from the block index; a block evaluates the
+// Cartesian blocks of its tasks into LDS and stores the requested-basis
+// elements from there, so nothing but the result goes through HBM.
+//
+// What bounds it: the chain of Rys evaluations per lane.  Bra pairs are sorted
+// by primitive count and a range whose pairs have many primitives spreads
+// them over S adjacent lanes; all bra classes share one launch so that the
+// few long dd blocks run beside the many short ss ones.  Both matrices of
+// (H2O)4 cc-pVDZ / JKFIT: 58 launches with staged blocks, 0.85 ms of kernels
+// between 20 ms of host task lists, before; 8 launches, 0.47 ms, now.
 #include "jk_kernels.h"
+
+namespace gscf {
+
+template <int LA, int LB, int LC>
+__device__ __forceinline__ void df_blocks(const DfArgs& a, const DfRange& r, double* __restrict__ buf) {
+  using K = Class<LA, LB, LC, 0>;
+  constexpr int SPL = df_split(LA, LB, LC);
+  constexpr int NBRA = K::NBRA, NC = K::NC;
+  const int lanes = SPL * r.S;
+  const int local = threadIdx.x / lanes;
+  const int s0 = threadIdx.x & (r.S - 1);
+  const int kc = (threadIdx.x / r.S) % SPL;
+  const int64_t t0 = (int64_t)(blockIdx.x - r.block0) * r.T;
+  const int64_t ntask = (int64_t)r.npair * a.nket;
+  if (local < r.T && t0 + local < ntask) {
+    const int64_t t = t0 + local;
+    const Pair bp = a.pairs[r.pair0 + t / a.nket];
+    const Pair kp = a.pairs[a.ket0 + t % a.nket];
+    const ShellXYZ sA = a.shells[bp.sa], sB = a.shells[bp.sb], sC = a.shells[kp.sa];
+    QuartetGeom geo;
+    double AB[3], CD[3];
+    load_geom(sA, sB, sC, sC, geo, AB, CD);
+    double* __restrict__ dst = buf + local * (NBRA * NC);
+    if constexpr (SPL == 1) {
+      double acc[K::NA][K::NB][NC][1];
+#pragma unroll
+      for (int e = 0; e < NBRA * NC; ++e) (&acc[0][0][0][0])[e] = 0.0;
+      for (int ip = s0; ip < bp.np; ip += r.S) {
+        const PrimPair P = a.prims[bp.poff + ip];
+        for (int kq = 0; kq < kp.np; ++kq) {
+          PrimQ<K::NR> q;
+          prim_setup<K::NR>(P, a.prims[kp.poff + kq], geo, q);
+          accumulate_full<LA, LB, LC, 0>(q, AB, CD, acc);
+        }
+      }
+      group_sum<NBRA * NC>(&acc[0][0][0][0], r.S);
+      if (s0 == 0)
+#pragma unroll
+        for (int e = 0; e < NBRA * NC; ++e) dst[e] = (&acc[0][0][0][0])[e];
+    } else {
+      // one lane per ket component; the second ket function has l = 0, so
+      // the weights pick G(n, m) at the component's exponents
+      int ec[3];
+      cart_xyz<LC>(kc, ec);
+      double wk[3][LC + 1];
+#pragma unroll
+      for (int x = 0; x < 3; ++x) ket_weights<LC>(ec[x], 0, 0.0, wk[x]);
+      double acc[K::NA][K::NB];
+#pragma unroll
+      for (int e = 0; e < NBRA; ++e) (&acc[0][0])[e] = 0.0;
+      for (int ip = s0; ip < bp.np; ip += r.S) {
+        const PrimPair P = a.prims[bp.poff + ip];
+        for (int kq = 0; kq < kp.np; ++kq) {
+          PrimQ<K::NR> q;
+          prim_setup<K::NR>(P, a.prims[kp.poff + kq], geo, q);
+          accumulate_split<LA, LB, LC, 0>(q, AB, wk, acc);
+        }
+      }
+      group_sum<NBRA>(&acc[0][0], r.S);
+      if (s0 == 0)
+#pragma unroll
+        for (int e = 0; e < NBRA; ++e) dst[e * NC + kc] = (&acc[0][0])[e];
+    }
+  }
+  __syncthreads();
+  // requested-basis elements of every task: the solid-harmonic (or identity)
+  // terms of each slot
+  const SphTerm* __restrict__ ta = a.terms + LA * kDfMaxFun;
+  const SphTerm* __restrict__ tb = a.terms + LB * kDfMaxFun;
+  const SphTerm* __restrict__ tc = a.terms + LC * kDfMaxFun;
+  const int fa = a.nfun[LA], fb = a.nfun[LB], fc = a.nfun[LC];
+  const int nout = fa * fb * fc;
+  for (int e = threadIdx.x; e < r.T * nout; e += blockDim.x) {
+    const int64_t t = t0 + e / nout;
+    if (t >= ntask) break;
+    int rem = e % nout;
+    const int p = rem % fa;
+    rem /= fa;
+    const int q = rem % fb, u = rem / fb;
+    const int bi = r.pair0 + (int)(t / a.nket), ki = a.ket0 + (int)(t % a.nket);
+    const Pair bp = a.pairs[bi], kp = a.pairs[ki];
+    const int64_t oa = a.shells[bp.sa].ao + p, oc = a.shells[kp.sa].ao + u;
+    const int64_t ob = a.layout == 3 ? a.shells[bp.sb].ao + q : 0;
+    if (a.layout == 3) {
+      if (bp.sa == bp.sb && p < q) continue;
+    } else if (LA == LC && (bp.sa < kp.sa || (bp.sa == kp.sa && p < u))) {
+      continue;  // the other order stores both elements, alike to the last bit
+    }
+    const double* __restrict__ blk = buf + (e / nout) * (NBRA * NC);
+    double v = 0.0;
+    for (int i = 0; i < ta[p].n; ++i)
+      for (int j = 0; j < tb[q].n; ++j) {
+        const double f = ta[p].c[i] * tb[q].c[j];
+        const double* __restrict__ row = blk + (ta[p].idx[i] * K::NB + tb[q].idx[j]) * NC;
+        for (int k = 0; k < tc[u].n; ++k) v += f * tc[u].c[k] * row[tc[u].idx[k]];
+      }
+    if (a.layout == 3) {
+      const int64_t hi = oa > ob ? oa : ob, lo = oa > ob ? ob : oa;
+      a.out[oc * a.np + hi * (hi + 1) / 2 + lo] = v;
+    } else {
+      a.out[oa * a.m + oc] = v;
+      a.out[oc * a.m + oa] = v;
+    }
+  }
+}
+
+template <int LC>
+__global__ __launch_bounds__(256) void df_kernel(DfArgs a) {
+  extern __shared__ double buf[];
+  int k = 0;
+  while (k + 1 < a.nrange && a.ranges[k + 1].block0 <= (int)blockIdx.x) ++k;
+  const DfRange r = a.ranges[k];
+  switch (r.la * 8 + r.lb) {
+    case 0: df_blocks<0, 0, LC>(a, r, buf); break;
+    case 8: df_blocks<1, 0, LC>(a, r, buf); break;
+    case 9: df_blocks<1, 1, LC>(a, r, buf); break;
+    case 16: df_blocks<2, 0, LC>(a, r, buf); break;
+    case 17: df_blocks<2, 1, LC>(a, r, buf); break;
+    case 18: df_blocks<2, 2, LC>(a, r, buf); break;
+    case 24: df_blocks<3, 0, LC>(a, r, buf); break;
+    default: df_blocks<4, 0, LC>(a, r, buf); break;
+  }
+}
 
 #define GSCF_DF_CAT(a, b) a##b
 #define GSCF_DF_NAME(p, c) GSCF_DF_CAT(p, c)
 
-namespace gscf {
-
-template <int LA, int LB>
-static bool df_try(int la, int lb, const BlockArgs& a, hipStream_t s) {
-  if (la != LA || lb != LB) return false;
-  launch_blocks_t<LA, LB, GSCF_DF_LC, 0>(a, s);
-  return true;
-}
-
-bool GSCF_DF_NAME(launch_df_blocks_c, GSCF_DF_LC)(int la, int lb, const BlockArgs& a, hipStream_t s) {
-  return df_try<0, 0>(la, lb, a, s) || df_try<1, 0>(la, lb, a, s) || df_try<1, 1>(la, lb, a, s) ||
-         df_try<2, 0>(la, lb, a, s) || df_try<2, 1>(la, lb, a, s) || df_try<2, 2>(la, lb, a, s) ||
-         df_try<3, 0>(la, lb, a, s) || df_try<4, 0>(la, lb, a, s);
+void GSCF_DF_NAME(launch_df_c, GSCF_DF_LC)(const DfArgs& a, int blocks, size_t lds, hipStream_t s) {
+  request_lds(df_kernel<GSCF_DF_LC>, lds);
+  hipLaunchKernelGGL((df_kernel<GSCF_DF_LC>), dim3((unsigned)blocks), dim3(256), lds, s, a);
 }
 
 }  // namespace gscf

@@ -220,6 +220,52 @@ struct BlockArgs {
   double* out;
 };
 
+// ----------------------------------------------------------------------------
+// Density-fitting integrals (A B|C u), u the unit function
+// ----------------------------------------------------------------------------
+constexpr int kDfMaxL = 4;      // auxiliary shells up to g
+constexpr int kDfMaxFun = 15;   // functions of one shell
+constexpr int kDfMaxTerms = 6;  // Cartesian terms of one real solid harmonic up to g
+
+// One requested-basis function as a sum of its shell's Cartesian components.
+struct SphTerm {
+  int n;
+  int idx[kDfMaxTerms];
+  double c[kDfMaxTerms];
+};
+
+// Bra pairs [pair0, pair0 + npair) of one class (la, lb) with similar
+// primitive counts: T (bra pair, ket shell) tasks per block, each on
+// S (x ket components) lanes, blocks from block0 on.
+struct DfRange {
+  int la, lb;
+  int pair0, npair;
+  int S, T;
+  int block0;
+  int pad;
+};
+
+// Lanes over ket components: blocks of more than 36 Cartesian components do
+// not fit one lane's registers.
+__host__ __device__ constexpr int df_ncart(int l) { return (l + 1) * (l + 2) / 2; }
+__host__ __device__ constexpr int df_split(int la, int lb, int lc) {
+  return df_ncart(la) * df_ncart(lb) * df_ncart(lc) > 36 ? df_ncart(lc) : 1;
+}
+
+struct DfArgs {
+  const Pair* pairs;
+  const PrimPair* prims;
+  const ShellXYZ* shells;   // ao: first AO in the requested basis (auxiliary: in the auxiliary set)
+  const DfRange* ranges;    // bra ranges of this launch
+  int nrange;
+  int ket0, nket;           // ket pairs (C, u) of this launch's angular momentum
+  int layout;               // 3: out[c][pair(a, b)], 2: out[a][c]
+  int64_t np, m;            // row lengths of the two layouts
+  const SphTerm* terms;     // [l][kDfMaxFun]
+  int nfun[kDfMaxL + 1];
+  double* out;
+};
+
 // Pair classes for l <= 2: index la*(la+1)/2 + lb with la >= lb.
 constexpr int kNumPairClasses = 6;
 __host__ __device__ constexpr int pair_class(int la, int lb) { return la * (la + 1) / 2 + lb; }

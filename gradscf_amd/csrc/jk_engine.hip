@@ -394,12 +394,12 @@ struct PlanData {
 GSCF_CLASSES(X)
 #undef X
 
-// density-fitting block kernels, one translation unit per auxiliary l (df_class.hip)
-bool launch_df_blocks_c0(int la, int lb, const BlockArgs& a, hipStream_t s);
-bool launch_df_blocks_c1(int la, int lb, const BlockArgs& a, hipStream_t s);
-bool launch_df_blocks_c2(int la, int lb, const BlockArgs& a, hipStream_t s);
-bool launch_df_blocks_c3(int la, int lb, const BlockArgs& a, hipStream_t s);
-bool launch_df_blocks_c4(int la, int lb, const BlockArgs& a, hipStream_t s);
+// density-fitting kernels, one translation unit per auxiliary l (df_class.hip)
+void launch_df_c0(const DfArgs& a, int blocks, size_t lds, hipStream_t s);
+void launch_df_c1(const DfArgs& a, int blocks, size_t lds, hipStream_t s);
+void launch_df_c2(const DfArgs& a, int blocks, size_t lds, hipStream_t s);
+void launch_df_c3(const DfArgs& a, int blocks, size_t lds, hipStream_t s);
+void launch_df_c4(const DfArgs& a, int blocks, size_t lds, hipStream_t s);
 
 void launch_int1e_class(int la, int lb, bool sph, const Pair* pairs, int npairs, const PrimPair* prims,
                         const ShellXYZ* shells, const int* shell_ao, const double* nuclei, const MolInfo* mols,
@@ -3104,95 +3104,37 @@ static void packed_eri(PlanData& P, int layout, double* out, int64_t size, hipSt
 // a >= b at pair_index(a, b)), csrc/density_fitting.cc:5-34.  The tables hold
 // orbital shells [0, split) and auxiliary shells [split, nbas).  A one-centre
 // factor P(r) is evaluated as the pair of P with a unit function (one
-// exponent-0 s primitive, coefficient 1, at P's centre), so the two- and
-// three-centre integrals run through the four-centre block kernels with the
-// libcint conventions of the two- and three-centre drivers.
+// exponent-0 s primitive, coefficient 1, at P's centre), with the libcint
+// conventions of the two- and three-centre drivers (df_class.hip).
 // ----------------------------------------------------------------------------
-constexpr int kMaxAuxL = 4;
-constexpr int kDfMaxTerms = 6;  // Cartesian terms of one real solid harmonic up to g
-
-struct DfPack {
-  int64_t off;   // first requested-basis element of the block
-  int64_t coff;  // first element of the staged Cartesian block
-  int ao[3];     // first AO (requested basis) and width of the three slots
-  int d[3];
-  int cao[3];    // first Cartesian AO and width
-  int cd[3];
+// Host tables uploaded as one buffer: parts are appended 16-byte aligned and
+// addressed by their offset once the buffer is on the device.
+struct Upload {
+  std::vector<char> host;
+  char* dev = nullptr;
+  template <class T>
+  size_t add(const std::vector<T>& v) {
+    const size_t at = (host.size() + 15) & ~(size_t)15;
+    host.resize(at + std::max<size_t>(1, v.size()) * sizeof(T));
+    if (!v.empty()) std::memcpy(host.data() + at, v.data(), v.size() * sizeof(T));
+    return at;
+  }
+  void send(hipStream_t s) {
+    HIP_OK(hipMalloc(&dev, host.size()));
+    HIP_OK(hipMemcpyAsync(dev, host.data(), host.size(), hipMemcpyHostToDevice, s));
+  }
+  template <class T>
+  const T* at(size_t off) const { return reinterpret_cast<const T*>(dev + off); }
+  ~Upload() {
+    if (dev) (void)hipFree(dev);
+  }
 };
-
-static void launch_df_blocks(int la, int lb, int lc, const BlockArgs& a, hipStream_t s) {
-  bool ok = false;
-  switch (lc) {
-    case 0: ok = launch_df_blocks_c0(la, lb, a, s); break;
-    case 1: ok = launch_df_blocks_c1(la, lb, a, s); break;
-    case 2: ok = launch_df_blocks_c2(la, lb, a, s); break;
-    case 3: ok = launch_df_blocks_c3(la, lb, a, s); break;
-    case 4: ok = launch_df_blocks_c4(la, lb, a, s); break;
-    default: break;
-  }
-  if (!ok) throw Internal("no density-fitting kernel for this angular-momentum class");
-}
-
-// One thread per requested-basis element of a staged block: the solid-harmonic
-// (or identity) transform of every slot, then the scatter into the layout.
-// layout 3: out[(c - n) np + a (a + 1) / 2 + b] for a >= b (slots: a, b, c);
-// layout 2: out[(a - n) m + (c - n)] and its transpose for a >= c (slots a, -, c).
-__global__ void df_pack_kernel(const double* __restrict__ stage, const DfPack* __restrict__ tasks, int64_t ntask,
-                               int64_t total, int layout, int64_t n, int64_t m, int64_t np,
-                               const int* __restrict__ s2c_idx, const double* __restrict__ s2c_coef,
-                               double* __restrict__ out) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= total) return;
-  int64_t lo = 0, hi = ntask;
-  while (hi - lo > 1) {
-    const int64_t mid = (lo + hi) >> 1;
-    if (tasks[mid].off <= e) lo = mid; else hi = mid;
-  }
-  const DfPack t = tasks[lo];
-  int64_t r = e - t.off;  // first slot fastest
-  const int p = (int)(r % t.d[0]);
-  r /= t.d[0];
-  const int q = (int)(r % t.d[1]);
-  const int u = (int)(r / t.d[1]);
-  const int64_t a = t.ao[0] + p, b = t.ao[1] + q, c = t.ao[2] + u;
-  if (layout == 3 && a < b) return;
-  if (layout == 2 && a < c) return;
-  const double* __restrict__ blk = stage + t.coff;
-  const int64_t g[3] = {a, layout == 3 ? b : -1, c};
-  double v = 0.0;
-  for (int k2 = 0; k2 < kDfMaxTerms; ++k2) {
-    const double c2 = s2c_coef[g[2] * kDfMaxTerms + k2];
-    if (c2 == 0.0) continue;
-    const int64_t i2 = s2c_idx[g[2] * kDfMaxTerms + k2] - t.cao[2];
-    for (int k1 = 0; k1 < (g[1] < 0 ? 1 : kDfMaxTerms); ++k1) {
-      double c1 = 1.0;
-      int64_t i1 = 0;
-      if (g[1] >= 0) {
-        c1 = s2c_coef[g[1] * kDfMaxTerms + k1];
-        if (c1 == 0.0) continue;
-        i1 = s2c_idx[g[1] * kDfMaxTerms + k1] - t.cao[1];
-      }
-      const double f = c1 * c2;
-      const int64_t base = (int64_t)t.cd[0] * (i1 + (int64_t)t.cd[1] * i2);
-      for (int k0 = 0; k0 < kDfMaxTerms; ++k0) {
-        const double c0 = s2c_coef[g[0] * kDfMaxTerms + k0];
-        if (c0 != 0.0) v += c0 * f * blk[base + s2c_idx[g[0] * kDfMaxTerms + k0] - t.cao[0]];
-      }
-    }
-  }
-  if (layout == 3) {
-    out[(c - n) * np + a * (a + 1) / 2 + b] = v;
-  } else {
-    out[(a - n) * m + (c - n)] = v;
-    out[(c - n) * m + (a - n)] = v;
-  }
-}
 
 static void density_fitting(const int32_t* atm, int natm, const int32_t* bas, int nbas, const double* env, int nenv,
                             int cart, int layout, int split, double* out, int64_t size, hipStream_t s) {
   if (layout != 2 && layout != 3) throw Internal("Unknown compact integral layout");
   PlanData P;
-  validate_tables(P, atm, natm, bas, nbas, env, nenv, cart, 1, nullptr, nullptr, kMaxAuxL);
+  validate_tables(P, atm, natm, bas, nbas, env, nenv, cart, 1, nullptr, nullptr, kDfMaxL);
   if (split < 1 || split >= nbas) throw Internal("Invalid orbital/auxiliary shell split");
   for (int sh = 0; sh < split; ++sh)
     if (P.bas[(size_t)sh * BAS_SLOTS + ANG_OF] > kMaxL)
@@ -3200,118 +3142,76 @@ static void density_fitting(const int32_t* atm, int natm, const int32_t* bas, in
   const int64_t n = P.ao[split], m = P.n - n, np = n * (n + 1) / 2;
   if (!out || size != (layout == 2 ? m * m : m * np)) throw Internal("Auxiliary integral shape mismatch");
   build_segments(P);
-  // unit functions: one exponent-0 s segment at the centre of every auxiliary segment
-  const int nseg0 = (int)P.seg.size();
-  std::vector<int> unit_of(nseg0, -1);
-  for (int i = 0; i < nseg0; ++i) {
-    if (P.seg[i].parent < split) continue;
-    Seg g;
-    g.parent = -1;
-    g.ctr = 0;
-    g.l = 0;
-    g.np = 1;
-    for (int x = 0; x < 3; ++x) g.r[x] = P.seg[i].r[x];
-    g.ao_cart = 0;
-    g.mol = 0;
-    g.lseg = 0;
-    g.a = {0.0};
-    g.c = {1.0};
-    unit_of[i] = (int)P.seg.size();
-    P.seg.push_back(std::move(g));
-  }
-  std::vector<int> seg_first(nbas, 0);
-  for (int i = nseg0 - 1; i >= 0; --i) seg_first[P.seg[i].parent] = i;
-  // pairs: the orbital segment pairs and every auxiliary segment with its unit
-  // function; make_pair wants the higher angular momentum first
-  std::vector<Pair> pairs;
-  std::map<std::pair<int, int>, int> pair_of;
-  auto get_pair = [&](int a, int b) {
-    if (P.seg[b].l > P.seg[a].l) std::swap(a, b);
-    auto it = pair_of.find({a, b});
-    if (it != pair_of.end()) return it->second;
-    Pair pr;
-    make_pair(P, a, b, pr);
-    pairs.push_back(pr);
-    pair_of[{a, b}] = (int)pairs.size() - 1;
-    return (int)pairs.size() - 1;
-  };
-  struct Item {
-    std::array<int, 3> cls;
-    BlockTask t;
-    int blk;  // index of the requested block (DfPack)
-  };
-  std::vector<Item> items;
-  std::vector<DfPack> packs;
-  auto ncomp = [&](int sh) { return P.ao_cart[sh + 1] - P.ao_cart[sh]; };
-  auto add_block = [&](int i, int j, int k) {
-    // requested block (i, j | k) (layout 3) or (i | k) (layout 2, j < 0)
-    DfPack pk;
-    const int sh[3] = {i, j, k};
-    for (int x = 0; x < 3; ++x) {
-      if (sh[x] < 0) {
-        pk.ao[x] = -1; pk.d[x] = 1; pk.cao[x] = 0; pk.cd[x] = 1;
-        continue;
-      }
-      pk.ao[x] = P.ao[sh[x]];
-      pk.d[x] = P.ao[sh[x] + 1] - P.ao[sh[x]];
-      pk.cao[x] = P.ao_cart[sh[x]];
-      pk.cd[x] = ncomp(sh[x]);
-    }
-    packs.push_back(pk);
-    const int bi = (int)packs.size() - 1;
-    const int st[3] = {1, pk.cd[0], pk.cd[0] * pk.cd[1]};
-    const int nci = P.bas[(size_t)i * BAS_SLOTS + NCTR_OF], ncj = j < 0 ? 1 : P.bas[(size_t)j * BAS_SLOTS + NCTR_OF];
-    const int nck = P.bas[(size_t)k * BAS_SLOTS + NCTR_OF];
-    for (int ci = 0; ci < nci; ++ci)
-      for (int cj = 0; cj < ncj; ++cj)
-        for (int ck = 0; ck < nck; ++ck) {
-          const int si = seg_first[i] + ci, sk = seg_first[k] + ck;
-          const int sj = j < 0 ? unit_of[si] : seg_first[j] + cj;
-          Item it;
-          it.blk = bi;
-          const int bra = get_pair(si, sj);
-          const int ket = get_pair(sk, unit_of[sk]);
-          it.t.bra = bra;
-          it.t.ket = ket;
-          it.t.base = 0;  // set per staging pass
-          const bool swapped = pairs[bra].sa != si;
-          const int off_i = ci * ncart_h(P.seg[si].l), off_j = j < 0 ? 0 : cj * ncart_h(P.seg[sj].l);
-          it.t.stride[0] = swapped ? (j < 0 ? 0 : st[1]) : st[0];
-          it.t.coff[0] = swapped ? off_j : off_i;
-          it.t.stride[1] = swapped ? st[0] : (j < 0 ? 0 : st[1]);
-          it.t.coff[1] = swapped ? off_i : off_j;
-          it.t.stride[2] = st[2];
-          it.t.coff[2] = ck * ncart_h(P.seg[sk].l);
-          it.t.stride[3] = 0;
-          it.t.coff[3] = 0;
-          it.cls = {P.seg[pairs[bra].sa].l, P.seg[pairs[bra].sb].l, P.seg[sk].l};
-          items.push_back(it);
-        }
-  };
-  if (layout == 3) {
-    for (int i = 0; i < split; ++i)
-      for (int j = 0; j <= i; ++j)
-        for (int k = split; k < nbas; ++k) add_block(i, j, k);
-  } else {
-    for (int i = split; i < nbas; ++i)
-      for (int k = split; k <= i; ++k) add_block(i, -1, k);
-  }
-  // device tables
-  std::vector<ShellXYZ> sh(P.seg.size());
-  for (size_t i = 0; i < P.seg.size(); ++i) {
-    sh[i].x = P.seg[i].r[0];
-    sh[i].y = P.seg[i].r[1];
-    sh[i].z = P.seg[i].r[2];
-    sh[i].ao = P.seg[i].ao_cart;
-    sh[i].l = P.seg[i].l;
+  const int nseg = (int)P.seg.size();
+  int first_aux = 0;
+  while (first_aux < nseg && P.seg[first_aux].parent < split) ++first_aux;
+  std::vector<ShellXYZ> sh(nseg);
+  for (int i = 0; i < nseg; ++i) {
+    const Seg& g = P.seg[i];
+    sh[i].x = g.r[0];
+    sh[i].y = g.r[1];
+    sh[i].z = g.r[2];
+    sh[i].ao = P.ao[g.parent] - (i < first_aux ? 0 : (int)n) + g.ctr * (cart ? ncart_h(g.l) : 2 * g.l + 1);
+    sh[i].l = g.l;
     sh[i].mol = 0;
     sh[i].lseg = 0;
   }
-  // solid-harmonic (or identity) map of every requested AO: up to six Cartesian terms
-  std::vector<int> sidx((size_t)P.n * kDfMaxTerms, 0);
-  std::vector<double> scoef((size_t)P.n * kDfMaxTerms, 0.0);
-  for (int shl = 0; shl < nbas; ++shl) {
-    const int l = P.bas[(size_t)shl * BAS_SLOTS + ANG_OF], nc = P.bas[(size_t)shl * BAS_SLOTS + NCTR_OF];
+  // (auxiliary shell, unit function) pairs by angular momentum, most primitives first
+  const double s2p = std::sqrt(2.0 * std::pow(3.14159265358979323846, 2.5));
+  std::vector<Pair> pairs;
+  int aux0[kDfMaxL + 2];
+  for (int l = 0; l <= kDfMaxL; ++l) {
+    aux0[l] = (int)pairs.size();
+    for (int i = first_aux; i < nseg; ++i) {
+      const Seg& g = P.seg[i];
+      if (g.l != l) continue;
+      Pair pr{i, i, (int)P.prims.size(), g.np};
+      for (int k = 0; k < g.np; ++k) {
+        PrimPair pp;
+        pp.p = pp.aa = g.a[k];
+        pp.px = pp.p * g.r[0] / pp.p;  // the centre as make_pair rounds it
+        pp.py = pp.p * g.r[1] / pp.p;
+        pp.pz = pp.p * g.r[2] / pp.p;
+        pp.e = g.c[k] * s2p / pp.p;
+        pp.ab = 0.0;
+        pp.ip = 1.0 / pp.p;
+        P.prims.push_back(pp);
+      }
+      pairs.push_back(pr);
+    }
+    std::stable_sort(pairs.begin() + aux0[l], pairs.end(), [](const Pair& x, const Pair& y) { return x.np > y.np; });
+  }
+  aux0[kDfMaxL + 1] = (int)pairs.size();
+  // bra classes: orbital pairs by class and primitive count, or the auxiliary pairs
+  struct Bra { int la, lb, beg, end; };
+  std::vector<Bra> bras;
+  if (layout == 3) {
+    std::vector<std::vector<Pair>> by_class(kNumPairClasses);
+    for (int S = 0; S < first_aux; ++S)
+      for (int T = 0; T <= S; ++T) {
+        int a = S, b = T;
+        if (P.seg[b].l > P.seg[a].l) std::swap(a, b);
+        Pair pr;
+        make_pair(P, a, b, pr);
+        by_class[pair_class(P.seg[a].l, P.seg[b].l)].push_back(pr);
+      }
+    static const int pl[kNumPairClasses][2] = {{0, 0}, {1, 0}, {1, 1}, {2, 0}, {2, 1}, {2, 2}};
+    for (int c = kNumPairClasses - 1; c >= 0; --c) {
+      auto& v = by_class[c];
+      if (v.empty()) continue;
+      std::stable_sort(v.begin(), v.end(), [](const Pair& x, const Pair& y) { return x.np > y.np; });
+      bras.push_back({pl[c][0], pl[c][1], (int)pairs.size(), (int)(pairs.size() + v.size())});
+      pairs.insert(pairs.end(), v.begin(), v.end());
+    }
+  } else {
+    for (int l = kDfMaxL; l >= 0; --l)
+      if (aux0[l] < aux0[l + 1]) bras.push_back({l, 0, aux0[l], aux0[l + 1]});
+  }
+  // functions of every angular momentum as terms of its Cartesian components
+  DfArgs a;
+  std::memset(&a, 0, sizeof(a));
+  std::vector<SphTerm> terms((kDfMaxL + 1) * kDfMaxFun, SphTerm{});
+  for (int l = 0; l <= kDfMaxL; ++l) {
     std::vector<std::vector<double>> rows;
     if (cart) {
       rows.assign(ncart_h(l), std::vector<double>(ncart_h(l), 0.0));
@@ -3319,86 +3219,79 @@ static void density_fitting(const int32_t* atm, int natm, const int32_t* bas, in
     } else {
       c2s_rows(l, rows);
     }
-    const int w = (int)rows.size();
-    for (int c = 0; c < nc; ++c)
-      for (int r = 0; r < w; ++r) {
-        const size_t ao = (size_t)P.ao[shl] + (size_t)c * w + r;
-        int t = 0;
-        for (int k = 0; k < ncart_h(l); ++k) {
-          if (rows[r][k] == 0.0) continue;
-          if (t == kDfMaxTerms) throw Internal("solid harmonic with more Cartesian terms than the map holds");
-          sidx[ao * kDfMaxTerms + t] = P.ao_cart[shl] + c * ncart_h(l) + k;
-          scoef[ao * kDfMaxTerms + t] = rows[r][k];
-          ++t;
-        }
+    a.nfun[l] = (int)rows.size();
+    for (size_t r = 0; r < rows.size(); ++r) {
+      SphTerm& t = terms[l * kDfMaxFun + r];
+      for (int k = 0; k < ncart_h(l); ++k) {
+        if (rows[r][k] == 0.0) continue;
+        if (t.n == kDfMaxTerms) throw Internal("solid harmonic with more Cartesian terms than the map holds");
+        t.idx[t.n] = k;
+        t.c[t.n++] = rows[r][k];
       }
+    }
   }
-  ShellXYZ* d_shells = dev_upload(sh, s);
-  PrimPair* d_prims = dev_upload(P.prims, s);
-  Pair* d_pairs = dev_upload(pairs, s);
-  int* d_sidx = dev_upload(sidx, s);
-  double* d_scoef = dev_upload(scoef, s);
-  hipLaunchKernelGGL(fill_kernel, dim3(nblocks((size_t)size)), dim3(256), 0, s, out, (size_t)size, 0.0);
-  // staging passes of at most kStage doubles, blocks in class order inside a pass
-  constexpr int64_t kStage = int64_t(1) << 24;
-  double* stage = nullptr;
-  HIP_OK(hipMalloc(&stage, sizeof(double) * kStage));
-  std::vector<int64_t> blk_coff(packs.size(), -1);
-  size_t ib = 0;  // items are grouped by block, in block order
-  while (ib < items.size()) {
-    // blocks [b0, b1) of this pass
-    const int b0 = items[ib].blk;
-    int64_t ctot = 0;
-    size_t ie = ib;
-    while (ie < items.size()) {
-      const DfPack& pk = packs[items[ie].blk];
-      const int64_t csz = (int64_t)pk.cd[0] * pk.cd[1] * pk.cd[2];
-      if (ctot > 0 && ctot + csz > kStage) break;
-      if (csz > kStage) throw Internal("auxiliary integral block larger than the staging buffer");
-      const int bk = items[ie].blk;
-      blk_coff[bk] = ctot;
-      ctot += csz;
-      while (ie < items.size() && items[ie].blk == bk) ++ie;
+  // ranges of every launch: the pairs of a class whose primitive counts share
+  // a power-of-two bucket, S lanes each so that a lane runs at most
+  // kDfPrim primitive quartets, T tasks per 256-lane block within 64 KB of LDS
+  constexpr int kDfPrim = 16;
+  std::vector<DfRange> ranges;
+  struct Launch { int lc, r0, nrange, blocks; size_t lds; };
+  std::vector<Launch> launches;
+  for (int lc = kDfMaxL; lc >= 0; --lc) {
+    const int nket = aux0[lc + 1] - aux0[lc];
+    if (nket == 0) continue;
+    Launch L{lc, (int)ranges.size(), 0, 0, 0};
+    int64_t blocks = 0;
+    for (const Bra& b : bras) {
+      if (layout == 2 && b.la < lc) continue;  // stored by the launch of the other order
+      const size_t blk = (size_t)ncart_h(b.la) * ncart_h(b.lb) * ncart_h(lc);
+      for (int i = b.beg; i < b.end;) {
+        int e = i;
+        while (e < b.end && (pairs[e].np ? bucket_of(pairs[e].np) : -1) == (pairs[i].np ? bucket_of(pairs[i].np) : -1)) ++e;
+        DfRange r{b.la, b.lb, i, e - i, 1, 1, (int)blocks, 0};
+        const int64_t work = (int64_t)pairs[i].np * pairs[aux0[lc]].np;
+        while (r.S < 16 && (int64_t)r.S * kDfPrim < work && 2 * r.S <= pairs[e - 1].np) r.S *= 2;
+        r.T = (int)std::max<size_t>(1, std::min<size_t>(256 / (r.S * df_split(b.la, b.lb, lc)), kLdsBudget / (8 * blk)));
+        L.lds = std::max(L.lds, 8 * blk * r.T);
+        blocks += ((int64_t)r.npair * nket + r.T - 1) / r.T;
+        if (blocks > std::numeric_limits<int>::max()) throw Internal("too many auxiliary integral blocks");
+        ranges.push_back(r);
+        ++L.nrange;
+        i = e;
+      }
     }
-    const int b1 = items[ie - 1].blk + 1;
-    std::vector<Item> pass(items.begin() + ib, items.begin() + ie);
-    for (Item& it : pass) it.t.base = blk_coff[it.blk];
-    std::stable_sort(pass.begin(), pass.end(), [](const Item& x, const Item& y) { return x.cls < y.cls; });
-    std::vector<BlockTask> tasks;
-    for (const Item& it : pass) tasks.push_back(it.t);
-    BlockTask* d_tasks = dev_upload(tasks, s);
-    size_t i = 0;
-    while (i < pass.size()) {
-      size_t j = i;
-      while (j < pass.size() && pass[j].cls == pass[i].cls) ++j;
-      BlockArgs a;
-      a.pairs = d_pairs;
-      a.prims = d_prims;
-      a.shells = d_shells;
-      a.tasks = d_tasks + i;
-      a.ntasks = (int64_t)(j - i);
-      a.out = stage;
-      launch_df_blocks(pass[i].cls[0], pass[i].cls[1], pass[i].cls[2], a, s);
-      i = j;
-    }
-    std::vector<DfPack> pp(packs.begin() + b0, packs.begin() + b1);
-    int64_t tot = 0;
-    for (int b = b0; b < b1; ++b) {
-      pp[b - b0].coff = blk_coff[b];
-      pp[b - b0].off = tot;
-      tot += (int64_t)pp[b - b0].d[0] * pp[b - b0].d[1] * pp[b - b0].d[2];
-    }
-    DfPack* d_pp = dev_upload(pp, s);
-    hipLaunchKernelGGL(df_pack_kernel, dim3(nblocks((size_t)tot)), dim3(256), 0, s, stage, d_pp, (int64_t)pp.size(),
-                       tot, layout, n, m, np, d_sidx, d_scoef, out);
-    HIP_OK(hipGetLastError());
-    HIP_OK(hipStreamSynchronize(s));
-    HIP_OK(hipFree(d_tasks));
-    HIP_OK(hipFree(d_pp));
-    ib = ie;
+    L.blocks = (int)blocks;
+    launches.push_back(L);
   }
-  HIP_OK(hipFree(stage));
-  for (void* p : {(void*)d_shells, (void*)d_prims, (void*)d_pairs, (void*)d_sidx, (void*)d_scoef}) (void)hipFree(p);
+  if (P.prims.empty()) P.prims.push_back(PrimPair{});
+  Upload up;
+  const size_t o_sh = up.add(sh), o_prims = up.add(P.prims), o_pairs = up.add(pairs), o_terms = up.add(terms),
+               o_ranges = up.add(ranges);
+  up.send(s);
+  a.pairs = up.at<Pair>(o_pairs);
+  a.prims = up.at<PrimPair>(o_prims);
+  a.shells = up.at<ShellXYZ>(o_sh);
+  a.terms = up.at<SphTerm>(o_terms);
+  a.layout = layout;
+  a.np = np;
+  a.m = m;
+  a.out = out;
+  for (const Launch& L : launches) {
+    if (L.blocks == 0) continue;
+    a.ranges = up.at<DfRange>(o_ranges) + L.r0;
+    a.nrange = L.nrange;
+    a.ket0 = aux0[L.lc];
+    a.nket = aux0[L.lc + 1] - aux0[L.lc];
+    switch (L.lc) {
+      case 0: launch_df_c0(a, L.blocks, L.lds, s); break;
+      case 1: launch_df_c1(a, L.blocks, L.lds, s); break;
+      case 2: launch_df_c2(a, L.blocks, L.lds, s); break;
+      case 3: launch_df_c3(a, L.blocks, L.lds, s); break;
+      default: launch_df_c4(a, L.blocks, L.lds, s); break;
+    }
+  }
+  HIP_OK(hipGetLastError());
+  HIP_OK(hipStreamSynchronize(s));
 }
 
 static void packed_jk(const double* eri, int64_t eri_size, int ndim, const double* density, int nb, int n,
