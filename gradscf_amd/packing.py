@@ -64,8 +64,14 @@ def pack_environment(topology, parameters: BasisParameters, coefficients, *, ori
 
 def pack(topology: BasisTopology, parameters: BasisParameters, *, origin=None):
     """(atm int32[natm,6], bas int32[nbas,8], env float64[nenv]) with normalised coefficients."""
-    coefficients = tuple(normalized_shell_coefficients(l, a, c) for l, a, c in
-                         zip(topology.angular_momenta, parameters.exponents, parameters.coefficients))
+    # atoms of one element carry the same shells: each distinct shell is normalised once
+    known, coefficients = {}, []
+    for l, a, c in zip(topology.angular_momenta, parameters.exponents, parameters.coefficients):
+        a, c = np.asarray(a, dtype=np.float64), np.asarray(c, dtype=np.float64)
+        key = (int(l), c.shape, a.tobytes(), c.tobytes())
+        if key not in known:
+            known[key] = normalized_shell_coefficients(l, a, c)
+        coefficients.append(known[key])
     return pack_environment(topology, parameters, coefficients, origin=origin)
 
 
