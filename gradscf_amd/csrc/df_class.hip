@@ -14,7 +14,7 @@
 // them over S adjacent lanes; all bra classes share one launch so that the
 // few long dd blocks run beside the many short ss ones.  Both matrices of
 // (H2O)4 cc-pVDZ / JKFIT: 58 launches with staged blocks, 0.85 ms of kernels
-// between 20 ms of host task lists, before; 8 launches, 0.47 ms, now.
+// between 20 ms of host task lists, before; 8 launches, 0.29 ms, now.
 #include "jk_kernels.h"
 
 namespace gscf {
@@ -22,63 +22,16 @@ namespace gscf {
 template <int LA, int LB, int LC>
 __device__ __forceinline__ void df_blocks(const DfArgs& a, const DfRange& r, double* __restrict__ buf) {
   using K = Class<LA, LB, LC, 0>;
-  constexpr int SPL = df_split(LA, LB, LC);
   constexpr int NBRA = K::NBRA, NC = K::NC;
-  const int lanes = SPL * r.S;
+  const int lanes = K::SPLIT * r.S;
   const int local = threadIdx.x / lanes;
-  const int s0 = threadIdx.x & (r.S - 1);
-  const int kc = (threadIdx.x / r.S) % SPL;
   const int64_t t0 = (int64_t)(blockIdx.x - r.block0) * r.T;
   const int64_t ntask = (int64_t)r.npair * a.nket;
   if (local < r.T && t0 + local < ntask) {
     const int64_t t = t0 + local;
-    const Pair bp = a.pairs[r.pair0 + t / a.nket];
-    const Pair kp = a.pairs[a.ket0 + t % a.nket];
-    const ShellXYZ sA = a.shells[bp.sa], sB = a.shells[bp.sb], sC = a.shells[kp.sa];
-    QuartetGeom geo;
-    double AB[3], CD[3];
-    load_geom(sA, sB, sC, sC, geo, AB, CD);
-    double* __restrict__ dst = buf + local * (NBRA * NC);
-    if constexpr (SPL == 1) {
-      double acc[K::NA][K::NB][NC][1];
-#pragma unroll
-      for (int e = 0; e < NBRA * NC; ++e) (&acc[0][0][0][0])[e] = 0.0;
-      for (int ip = s0; ip < bp.np; ip += r.S) {
-        const PrimPair P = a.prims[bp.poff + ip];
-        for (int kq = 0; kq < kp.np; ++kq) {
-          PrimQ<K::NR> q;
-          prim_setup<K::NR>(P, a.prims[kp.poff + kq], geo, q);
-          accumulate_full<LA, LB, LC, 0>(q, AB, CD, acc);
-        }
-      }
-      group_sum<NBRA * NC>(&acc[0][0][0][0], r.S);
-      if (s0 == 0)
-#pragma unroll
-        for (int e = 0; e < NBRA * NC; ++e) dst[e] = (&acc[0][0][0][0])[e];
-    } else {
-      // one lane per ket component; the second ket function has l = 0, so
-      // the weights pick G(n, m) at the component's exponents
-      int ec[3];
-      cart_xyz<LC>(kc, ec);
-      double wk[3][LC + 1];
-#pragma unroll
-      for (int x = 0; x < 3; ++x) ket_weights<LC>(ec[x], 0, 0.0, wk[x]);
-      double acc[K::NA][K::NB];
-#pragma unroll
-      for (int e = 0; e < NBRA; ++e) (&acc[0][0])[e] = 0.0;
-      for (int ip = s0; ip < bp.np; ip += r.S) {
-        const PrimPair P = a.prims[bp.poff + ip];
-        for (int kq = 0; kq < kp.np; ++kq) {
-          PrimQ<K::NR> q;
-          prim_setup<K::NR>(P, a.prims[kp.poff + kq], geo, q);
-          accumulate_split<LA, LB, LC, 0>(q, AB, wk, acc);
-        }
-      }
-      group_sum<NBRA>(&acc[0][0], r.S);
-      if (s0 == 0)
-#pragma unroll
-        for (int e = 0; e < NBRA; ++e) dst[e * NC + kc] = (&acc[0][0])[e];
-    }
+    // (the second shell of a (C, u) pair is C itself: same centre, no l)
+    block_to_lds<LA, LB, LC, 0>(a.prims, a.shells, a.pairs[r.pair0 + t / a.nket], a.pairs[a.ket0 + t % a.nket], r.S, 1,
+                                threadIdx.x & (r.S - 1), (threadIdx.x / r.S) % K::SPLIT, buf + local * (NBRA * NC));
   }
   __syncthreads();
   // requested-basis elements of every task: the solid-harmonic (or identity)

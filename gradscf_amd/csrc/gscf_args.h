@@ -266,6 +266,32 @@ struct DfArgs {
   double* out;
 };
 
+// ----------------------------------------------------------------------------
+// Packed ERIs
+// ----------------------------------------------------------------------------
+// Tasks (bra pair, ket pair) of two pair ranges with similar primitive counts
+// (tri: one range with itself, ket <= bra): T per block on S = Sb * Sk lanes
+// (x ket components) each, blocks from block0 on.
+struct EriRange {
+  int bra0, nbra, ket0, nket;
+  int S, Sk, T, tri;
+  int block0;
+  int pad;
+};
+
+struct EriArgs {
+  const Pair* pairs;
+  const PrimPair* prims;
+  const ShellXYZ* shells;   // ao: first AO in the requested basis
+  const EriRange* ranges;   // ranges of this launch
+  int nrange;
+  int layout;               // 0: symmetric pair matrix, 1: s8 triangle
+  int64_t np;
+  const SphTerm* terms;     // [l][kDfMaxFun]
+  int nfun[kDfMaxL + 1];
+  double* out;
+};
+
 // Pair classes for l <= 2: index la*(la+1)/2 + lb with la >= lb.
 constexpr int kNumPairClasses = 6;
 __host__ __device__ constexpr int pair_class(int la, int lb) { return la * (la + 1) / 2 + lb; }

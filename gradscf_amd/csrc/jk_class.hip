@@ -24,4 +24,8 @@ void GSCF_NAME(launch_param_c, GSCF_LA, GSCF_LB, GSCF_LC, GSCF_LD)(const ParamAr
 void GSCF_NAME(launch_blocks_c, GSCF_LA, GSCF_LB, GSCF_LC, GSCF_LD)(const BlockArgs& a, hipStream_t s) {
   launch_blocks_t<GSCF_LA, GSCF_LB, GSCF_LC, GSCF_LD>(a, s);
 }
+void GSCF_NAME(launch_eri_c, GSCF_LA, GSCF_LB, GSCF_LC, GSCF_LD)(const EriArgs& a, int blocks, size_t lds,
+                                                               hipStream_t s) {
+  launch_eri_t<GSCF_LA, GSCF_LB, GSCF_LC, GSCF_LD>(a, blocks, lds, s);
+}
 }  // namespace gscf

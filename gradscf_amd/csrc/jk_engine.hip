@@ -390,6 +390,7 @@ struct PlanData {
   X(2, 2, 2, 0) X(2, 2, 2, 1) X(2, 2, 2, 2)
 #define X(A, B, C, D)                                                       \
   void launch_jk_c##A##B##C##D(const JKArgs& a, hipStream_t s);            \
+  void launch_eri_c##A##B##C##D(const EriArgs& a, int blocks, size_t lds, hipStream_t s); \
   void launch_blocks_c##A##B##C##D(const BlockArgs& a, hipStream_t s);
 GSCF_CLASSES(X)
 #undef X
@@ -2920,193 +2921,171 @@ static void eri_blocks(PlanData& P, const int32_t* shls, int64_t nq, const int64
 // Packed ERIs and packed J/K (the reference's compact-integral and packed J/K
 // targets, csrc/packed_eri.cc:5-14, csrc/compact.cc:5-17, csrc/packed_jk.cc:6-79)
 // ----------------------------------------------------------------------------
-struct PackTask {
-  int64_t off;   // first requested-basis element of the block (element enumeration)
-  int64_t coff;  // first element of the staged Cartesian block
-  int ao[4];     // first AO of each shell (requested basis) and its width
-  int d[4];
-  int cao[4];    // first Cartesian AO of each shell and its width
-  int cd[4];
-};
+// J/K from packed ERIs.  The stored lower triangle is read once: a workgroup
+// takes R rows (a b_r | of one a, its four wavefronts share the ket index c
+// and the lanes run over d <= c, so loads are contiguous.  Per element v:
+//   J_ab += v (D_cd + D_dc)          lane sums, one add per row and lane group
+//   J_cd += v (D_ab + D_ba)          summed over the R rows, one add per element
+//   K_a., K_b. (8 terms)             the terms of column c by a wavefront sum,
+//                                    those of column d in the lane's registers,
+//                                    both into LDS rows flushed once
+// J goes to its lower triangle only (mirrored afterwards).  Bound by device
+// atomics: one thread per element issued 12 per stored element on few
+// addresses ((H2O)2 6-31G*, n = 38: 375 us); now one per R elements and
+// 4 (R + 1) n per workgroup (60 us).
+constexpr int kPackedRows = 8;
+constexpr int kPackedWide = 455;  // n up to which 2 (R + 1) rows of K fit 64 KB of LDS
 
-__device__ __forceinline__ int64_t tri_row(int64_t idx) {
-  // largest r with r (r + 1) / 2 <= idx
-  int64_t r = (int64_t)((sqrt(8.0 * (double)idx + 1.0) - 1.0) * 0.5);
-  while (r * (r + 1) / 2 > idx) --r;
-  while ((r + 1) * (r + 2) / 2 <= idx) ++r;
-  return r;
-}
+// An integral that is zero (or a lane without one) adds nothing, whatever the
+// density holds there.
+__device__ __forceinline__ double times(double v, double x) { return v == 0.0 ? 0.0 : v * x; }
 
-// One thread per block element in the requested basis: unique AO quartets
-// (a >= b, c >= d, ab >= cd) go to the packed layout (0: pair matrix, both
-// triangles; 1: s8 triangle), transformed from the staged Cartesian block by
-// the plan's spherical-to-Cartesian map (up to 3 terms per AO; identity for
-// Cartesian plans).
-__global__ void pack_eri_kernel(const double* __restrict__ blocks, const PackTask* __restrict__ tasks,
-                                int64_t ntask, int64_t total, int layout, int64_t np,
-                                const int* __restrict__ s2c_idx, const double* __restrict__ s2c_coef,
-                                double* __restrict__ out) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= total) return;
-  int64_t lo = 0, hi = ntask;
-  while (hi - lo > 1) {
-    const int64_t mid = (lo + hi) >> 1;
-    if (tasks[mid].off <= e) lo = mid; else hi = mid;
-  }
-  const PackTask t = tasks[lo];
-  int64_t r = e - t.off;  // libcint layout: first index fastest
-  const int p = (int)(r % t.d[0]);
-  r /= t.d[0];
-  const int q = (int)(r % t.d[1]);
-  r /= t.d[1];
-  const int u = (int)(r % t.d[2]);
-  const int w = (int)(r / t.d[2]);
-  const int64_t a = t.ao[0] + p, b = t.ao[1] + q, c = t.ao[2] + u, d = t.ao[3] + w;
-  if (a < b || c < d) return;
-  const int64_t ab = a * (a + 1) / 2 + b, cd = c * (c + 1) / 2 + d;
-  if (ab < cd) return;
-  const int64_t g[4] = {a, b, c, d};
-  int ci[4][3];
-  double cc[4][3];
-  for (int x = 0; x < 4; ++x)
-    for (int m = 0; m < 3; ++m) {
-      ci[x][m] = s2c_idx[g[x] * 3 + m] - t.cao[x];
-      cc[x][m] = s2c_coef[g[x] * 3 + m];
-    }
-  const double* __restrict__ blk = blocks + t.coff;
-  double v = 0.0;
-  for (int m3 = 0; m3 < 3; ++m3) {
-    if (cc[3][m3] == 0.0) continue;
-    for (int m2 = 0; m2 < 3; ++m2) {
-      if (cc[2][m2] == 0.0) continue;
-      for (int m1 = 0; m1 < 3; ++m1) {
-        if (cc[1][m1] == 0.0) continue;
-        const int64_t base = ci[1][m1] + (int64_t)t.cd[1] * (ci[2][m2] + (int64_t)t.cd[2] * ci[3][m3]);
-        const double f = cc[1][m1] * cc[2][m2] * cc[3][m3];
-        for (int m0 = 0; m0 < 3; ++m0)
-          if (cc[0][m0] != 0.0) v += cc[0][m0] * f * blk[ci[0][m0] + (int64_t)t.cd[0] * base];
-      }
-    }
-  }
-  if (layout == 0) {
-    out[ab * np + cd] = v;
-    out[cd * np + ab] = v;
-  } else {
-    out[ab * (ab + 1) / 2 + cd] = v;
-  }
-}
-
-// One thread per stored element (ab >= cd) of the s8 triangle or of the lower
-// triangle of the pair matrix: the 8-fold digestion of the reference's packed
-// J/K into out[op][b][n][n] with device-scope atomics.
-__global__ void packed_jk_kernel(const double* __restrict__ eri, int s8, int64_t np, const double* __restrict__ D,
-                                 int nb, int n, int with_j, int with_k, double* __restrict__ out) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= np * (np + 1) / 2) return;
-  const int64_t ab = tri_row(idx), cd = idx - ab * (ab + 1) / 2;
-  const double v = s8 ? eri[idx] : eri[ab * np + cd];
-  if (v == 0.0) return;
-  const int a = (int)tri_row(ab), b = (int)(ab - (int64_t)a * (a + 1) / 2);
-  const int c = (int)tri_row(cd), d = (int)(cd - (int64_t)c * (c + 1) / 2);
+template <int R>
+__global__ __launch_bounds__(256) void packed_jk_kernel(const double* __restrict__ eri, int s8, int64_t np,
+                                                        const double* __restrict__ Dall, int n, int with_j, int with_k,
+                                                        int64_t kbase, double* __restrict__ out) {
+  extern __shared__ double kl[];  // [row: a, b_0..b_{R-1}][set][n]
+  const int a = n - 1 - (int)blockIdx.y;
+  const int b0 = (int)blockIdx.x * R;
+  if (b0 > a) return;
   const size_t nn = (size_t)n * n;
-  for (int bt = 0; bt < nb; ++bt) {
-    const double* dm = D + (size_t)bt * nn;
-    if (with_j) {
-      double* j = out + (size_t)bt * nn;
-      const double jab = v * (dm[(size_t)c * n + d] + (c != d ? dm[(size_t)d * n + c] : 0.0));
-      atomicAdd(j + (size_t)a * n + b, jab);
-      if (a != b) atomicAdd(j + (size_t)b * n + a, jab);
-      if (ab != cd) {
-        const double jcd = v * (dm[(size_t)a * n + b] + (a != b ? dm[(size_t)b * n + a] : 0.0));
-        atomicAdd(j + (size_t)c * n + d, jcd);
-        if (c != d) atomicAdd(j + (size_t)d * n + c, jcd);
+  const double* __restrict__ D = Dall + (size_t)blockIdx.z * nn;
+  double* __restrict__ J = out + (size_t)blockIdx.z * nn;
+  double* __restrict__ Kd = out + kbase + (size_t)blockIdx.z * nn;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  if (with_k)
+    for (int i = threadIdx.x; i < 2 * (R + 1) * n; i += blockDim.x) kl[i] = 0.0;
+  __syncthreads();
+  const double* __restrict__ row[R];
+  double dab[R], jab[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int b = min(b0 + r, a);
+    const int64_t ab = (int64_t)a * (a + 1) / 2 + b;
+    row[r] = eri + (s8 ? ab * (ab + 1) / 2 : ab * np);
+    dab[r] = D[(size_t)a * n + b] + (a != b ? D[(size_t)b * n + a] : 0.0);
+    jab[r] = 0.0;
+  }
+  for (int d0 = 0; d0 <= a; d0 += 64) {
+    const int d = d0 + lane;
+    const bool din = d <= a;
+    // densities of the R + 1 bra functions against d: rows (set 0) and columns (set 1)
+    double ad[2] = {0.0, 0.0}, bd[R][2];
+    // sums of the terms that land in column d
+    double sa[2] = {0.0, 0.0}, sb[R][2];
+#pragma unroll
+    for (int r = 0; r < R; ++r) bd[r][0] = bd[r][1] = sb[r][0] = sb[r][1] = 0.0;
+    if (din && with_k) {
+      ad[0] = D[(size_t)a * n + d];
+      ad[1] = D[(size_t)d * n + a];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int b = min(b0 + r, a);
+        bd[r][0] = D[(size_t)b * n + d];
+        bd[r][1] = D[(size_t)d * n + b];
       }
     }
-    if (with_k) {
-      double* k = out + (size_t)(with_j * nb + bt) * nn;
-      atomicAdd(k + (size_t)a * n + c, v * dm[(size_t)b * n + d]);
-      if (c != d) atomicAdd(k + (size_t)a * n + d, v * dm[(size_t)b * n + c]);
-      if (a != b) atomicAdd(k + (size_t)b * n + c, v * dm[(size_t)a * n + d]);
-      if (a != b && c != d) atomicAdd(k + (size_t)b * n + d, v * dm[(size_t)a * n + c]);
-      if (ab != cd) {
-        atomicAdd(k + (size_t)c * n + a, v * dm[(size_t)d * n + b]);
-        if (a != b) atomicAdd(k + (size_t)c * n + b, v * dm[(size_t)d * n + a]);
-        if (c != d) atomicAdd(k + (size_t)d * n + a, v * dm[(size_t)c * n + b]);
-        if (a != b && c != d) atomicAdd(k + (size_t)d * n + b, v * dm[(size_t)c * n + a]);
+    for (int c = d0 + wave; c <= a; c += nw) {
+      const int64_t cd = (int64_t)c * (c + 1) / 2 + d;
+      double v[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int b = b0 + r;
+        v[r] = (d <= c && b <= a && (c < a || d <= b)) ? row[r][cd] : 0.0;
       }
+      if (with_j && d <= c) {
+        const double dcd = D[(size_t)c * n + d] + (c != d ? D[(size_t)d * n + c] : 0.0);
+        double jcd = 0.0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          jab[r] += times(v[r], dcd);
+          jcd += times((c == a && d == b0 + r) ? 0.0 : v[r], dab[r]);  // not twice on ab == cd
+        }
+        if (jcd != 0.0) atomicAdd(J + (size_t)c * n + d, jcd);
+      }
+      if (with_k) {
+        const double ac[2] = {D[(size_t)a * n + c], D[(size_t)c * n + a]};
+        double ca[2] = {0.0, 0.0}, cb[R][2];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const int b = b0 + r;
+          const double v1 = v[r], v2 = (c == a && d == b) ? 0.0 : v1;  // second set: (cd|ab)
+          const double w1 = b != a ? v1 : 0.0, w2 = b != a ? v2 : 0.0;  // b's own rows
+          const int bb = min(b, a);
+          const double bc0 = D[(size_t)bb * n + c], bc1 = D[(size_t)c * n + bb];
+          ca[0] += times(v1, bd[r][0]);
+          ca[1] += times(v2, bd[r][1]);
+          cb[r][0] = times(w1, ad[0]);
+          cb[r][1] = times(w2, ad[1]);
+          if (d != c) {
+            sa[0] += times(v1, bc0);
+            sa[1] += times(v2, bc1);
+            sb[r][0] += times(w1, ac[0]);
+            sb[r][1] += times(w2, ac[1]);
+          }
+        }
+#pragma unroll
+        for (int m = 1; m < 64; m <<= 1) {
+          ca[0] += __shfl_xor(ca[0], m);
+          ca[1] += __shfl_xor(ca[1], m);
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            cb[r][0] += __shfl_xor(cb[r][0], m);
+            cb[r][1] += __shfl_xor(cb[r][1], m);
+          }
+        }
+        if (lane == 0) {
+          atomicAdd(kl + c, ca[0]);
+          atomicAdd(kl + n + c, ca[1]);
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            atomicAdd(kl + (2 * r + 2) * n + c, cb[r][0]);
+            atomicAdd(kl + (2 * r + 3) * n + c, cb[r][1]);
+          }
+        }
+      }
+    }
+    if (din && with_k) {
+      atomicAdd(kl + d, sa[0]);
+      atomicAdd(kl + n + d, sa[1]);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        atomicAdd(kl + (2 * r + 2) * n + d, sb[r][0]);
+        atomicAdd(kl + (2 * r + 3) * n + d, sb[r][1]);
+      }
+    }
+  }
+  if (with_j) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      double s = jab[r];
+#pragma unroll
+      for (int m = 1; m < 64; m <<= 1) s += __shfl_xor(s, m);
+      if (lane == 0 && b0 + r <= a && s != 0.0) atomicAdd(J + (size_t)a * n + b0 + r, s);
+    }
+  }
+  if (with_k) {
+    __syncthreads();
+    for (int i = threadIdx.x; i < (R + 1) * n; i += blockDim.x) {
+      const int k = i / n, x = i - k * n;
+      const int f = k == 0 ? a : b0 + k - 1;
+      if (f > a || x > a) continue;
+      const double v1 = kl[(2 * k) * n + x], v2 = kl[(2 * k + 1) * n + x];
+      if (v1 != 0.0) atomicAdd(Kd + (size_t)f * n + x, v1);
+      if (v2 != 0.0) atomicAdd(Kd + (size_t)x * n + f, v2);
     }
   }
 }
 
-// Every unique AO quartet of the plan's molecule (no screening), staged shell
-// quartet by shell quartet in the reference's visiting order (i, j <= i,
-// k <= i, l <= k; csrc/coulomb_shells.h:98-125) through the block kernels.
-static void packed_eri(PlanData& P, int layout, double* out, int64_t size, hipStream_t s) {
-  if (layout != 0 && layout != 1) throw Internal("Unknown compact integral layout");
-  if (P.nmol != 1) throw Internal("Packed ERIs need a single-molecule plan");
-  const int64_t n = P.n, np = n * (n + 1) / 2;
-  if (!out || size != (layout == 0 ? np * np : np * (np + 1) / 2)) throw Internal("Packed ERI shape mismatch");
-  hipLaunchKernelGGL(fill_kernel, dim3(nblocks((size_t)size)), dim3(256), 0, s, out, (size_t)size, 0.0);
-  constexpr int64_t kStage = int64_t(1) << 24;  // doubles of staged blocks per pass
-  double* stage = nullptr;
-  HIP_OK(hipMalloc(&stage, sizeof(double) * kStage));
-  std::vector<int32_t> shls;
-  std::vector<int64_t> offs;
-  std::vector<PackTask> tasks;
-  int64_t tot = 0, ctot = 0;  // requested-basis elements, staged Cartesian doubles
-  auto flush = [&]() {
-    if (tasks.empty()) return;
-    eri_blocks(P, shls.data(), (int64_t)tasks.size(), offs.data(), stage, s);
-    PackTask* d_tasks = dev_upload(tasks, s);
-    hipLaunchKernelGGL(pack_eri_kernel, dim3(nblocks((size_t)tot)), dim3(256), 0, s, stage, d_tasks,
-                       (int64_t)tasks.size(), tot, layout, np, P.d_s2c_idx, P.d_s2c_coef, out);
-    HIP_OK(hipGetLastError());
-    HIP_OK(hipStreamSynchronize(s));
-    HIP_OK(hipFree(d_tasks));
-    shls.clear();
-    offs.clear();
-    tasks.clear();
-    tot = 0;
-    ctot = 0;
-  };
-  const int nbas = P.nbas;
-  for (int i = 0; i < nbas; ++i)
-    for (int j = 0; j <= i; ++j)
-      for (int k = 0; k <= i; ++k)
-        for (int l = 0; l <= k; ++l) {
-          const int sh[4] = {i, j, k, l};
-          PackTask t;
-          int64_t sz = 1, csz = 1;
-          for (int x = 0; x < 4; ++x) {
-            t.ao[x] = P.ao[sh[x]];
-            t.d[x] = P.ao[sh[x] + 1] - P.ao[sh[x]];
-            t.cao[x] = P.ao_cart[sh[x]];
-            t.cd[x] = P.ao_cart[sh[x] + 1] - P.ao_cart[sh[x]];
-            sz *= t.d[x];
-            csz *= t.cd[x];
-          }
-          if (ctot + csz > kStage) flush();
-          t.off = tot;
-          t.coff = ctot;
-          for (int x = 0; x < 4; ++x) shls.push_back(sh[x]);
-          offs.push_back(ctot);
-          tasks.push_back(t);
-          tot += sz;
-          ctot += csz;
-        }
-  flush();
-  HIP_OK(hipFree(stage));
+// upper triangle of every n x n matrix from its lower one
+__global__ void mirror_kernel(double* __restrict__ m, int nb, int n) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const size_t nn = (size_t)n * n;
+  if (i >= nn * nb) return;
+  const int r = (int)(i % nn / n), c = (int)(i % n);
+  if (c > r) m[i] = m[i - (size_t)r * n - c + (size_t)c * n + r];
 }
 
-// ----------------------------------------------------------------------------
-// Density-fitting integrals: the reference's compact layouts 2 (two-centre
-// metric (P|Q), m x m) and 3 (three-centre (ab|P), m x n(n+1)/2 over AO pairs
-// a >= b at pair_index(a, b)), csrc/density_fitting.cc:5-34.  The tables hold
-// orbital shells [0, split) and auxiliary shells [split, nbas).  A one-centre
-// factor P(r) is evaluated as the pair of P with a unit function (one
-// exponent-0 s primitive, coefficient 1, at P's centre), with the libcint
-// conventions of the two- and three-centre drivers (df_class.hip).
-// ----------------------------------------------------------------------------
 // Host tables uploaded as one buffer: parts are appended 16-byte aligned and
 // addressed by their offset once the buffer is on the device.
 struct Upload {
@@ -3130,6 +3109,170 @@ struct Upload {
   }
 };
 
+// Requested-basis functions of every l as terms of its Cartesian components;
+// nfun[l]: their number.
+static std::vector<SphTerm> function_terms(int cart, int (&nfun)[kDfMaxL + 1]) {
+  std::vector<SphTerm> terms((kDfMaxL + 1) * kDfMaxFun, SphTerm{});
+  for (int l = 0; l <= kDfMaxL; ++l) {
+    std::vector<std::vector<double>> rows;
+    if (cart) {
+      rows.assign(ncart_h(l), std::vector<double>(ncart_h(l), 0.0));
+      for (int k = 0; k < ncart_h(l); ++k) rows[k][k] = 1.0;
+    } else {
+      c2s_rows(l, rows);
+    }
+    nfun[l] = (int)rows.size();
+    for (size_t r = 0; r < rows.size(); ++r) {
+      SphTerm& t = terms[l * kDfMaxFun + r];
+      for (int k = 0; k < ncart_h(l); ++k) {
+        if (rows[r][k] == 0.0) continue;
+        if (t.n == kDfMaxTerms) throw Internal("solid harmonic with more Cartesian terms than the map holds");
+        t.idx[t.n] = k;
+        t.c[t.n++] = rows[r][k];
+      }
+    }
+  }
+  return terms;
+}
+
+// Segmented shells with their first AO in the requested basis, counted from
+// `base` for the segments from `first` on.
+static std::vector<ShellXYZ> requested_shells(const PlanData& P, int first, int base) {
+  std::vector<ShellXYZ> sh(P.seg.size());
+  for (size_t i = 0; i < P.seg.size(); ++i) {
+    const Seg& g = P.seg[i];
+    sh[i].x = g.r[0];
+    sh[i].y = g.r[1];
+    sh[i].z = g.r[2];
+    sh[i].ao = P.ao[g.parent] - ((int)i < first ? 0 : base) + g.ctr * (P.cart ? ncart_h(g.l) : 2 * g.l + 1);
+    sh[i].l = g.l;
+    sh[i].mol = 0;
+    sh[i].lseg = 0;
+  }
+  return sh;
+}
+
+// Orbital segment pairs of segments [0, nseg) by class, most primitives first.
+static std::vector<std::vector<Pair>> pairs_by_class(PlanData& P, int nseg) {
+  std::vector<std::vector<Pair>> by(kNumPairClasses);
+  for (int S = 0; S < nseg; ++S)
+    for (int T = 0; T <= S; ++T) {
+      int a = S, b = T;
+      if (P.seg[b].l > P.seg[a].l) std::swap(a, b);
+      Pair pr;
+      make_pair(P, a, b, pr);
+      by[pair_class(P.seg[a].l, P.seg[b].l)].push_back(pr);
+    }
+  for (auto& v : by)
+    std::stable_sort(v.begin(), v.end(), [](const Pair& x, const Pair& y) { return x.np > y.np; });
+  return by;
+}
+
+static int pair_bucket(const Pair& p) { return p.np ? bucket_of(p.np) : -1; }
+
+// Every unique AO quartet of one molecule, unscreened, by class launches.
+static void packed_eri(const int32_t* atm, int natm, const int32_t* bas, int nbas, const double* env, int nenv,
+                       int cart, int layout, double* out, int64_t size, hipStream_t s) {
+  PlanData P;
+  validate_tables(P, atm, natm, bas, nbas, env, nenv, cart);
+  if (layout != 0 && layout != 1) throw Internal("Unknown compact integral layout");
+  const int64_t n = P.n, np = n * (n + 1) / 2;
+  if (!out || size != (layout == 0 ? np * np : np * (np + 1) / 2)) throw Internal("Packed ERI shape mismatch");
+  build_segments(P);
+  auto by = pairs_by_class(P, (int)P.seg.size());
+  // runs of pairs whose primitive counts share a power-of-two bucket
+  struct Run { int beg, end; };
+  std::vector<Pair> pairs;
+  std::vector<std::vector<Run>> runs(kNumPairClasses);
+  for (int c = 0; c < kNumPairClasses; ++c)
+    for (size_t i = 0; i < by[c].size();) {
+      size_t e = i;
+      while (e < by[c].size() && pair_bucket(by[c][e]) == pair_bucket(by[c][i])) ++e;
+      runs[c].push_back({(int)pairs.size(), (int)(pairs.size() + e - i)});
+      pairs.insert(pairs.end(), by[c].begin() + i, by[c].begin() + e);
+      i = e;
+    }
+  // primitive quartets per lane where the split reaches it, and workgroups a
+  // launch spreads its tasks over before they share one: small molecules are
+  // bound by the chain in a lane and the store loop of a workgroup, not by
+  // idle lanes ((H2O)2 6-31G*: 868 us a call with full 256-lane workgroups and
+  // 8 primitive quartets, 480 us with these, 510 us with 1024 workgroups)
+  constexpr int64_t kEriPrim = 2, kEriGroups = 256;
+  std::vector<EriRange> ranges;
+  struct Launch { int cb, ck, r0, nrange, blocks; size_t lds; };
+  std::vector<Launch> launches;
+  static const int pl[kNumPairClasses][2] = {{0, 0}, {1, 0}, {1, 1}, {2, 0}, {2, 1}, {2, 2}};
+  for (int cb = kNumPairClasses - 1; cb >= 0; --cb)
+    for (int ck = cb; ck >= 0; --ck) {
+      const int nbra = ncart_h(pl[cb][0]) * ncart_h(pl[cb][1]), nket = ncart_h(pl[ck][0]) * ncart_h(pl[ck][1]);
+      const int split = nbra * nket > 36 ? nket : 1;
+      Launch L{cb, ck, (int)ranges.size(), 0, 0, 0};
+      int64_t blocks = 0;
+      const int64_t class_tasks = cb == ck ? (int64_t)by[cb].size() * (by[cb].size() + 1) / 2
+                                           : (int64_t)by[cb].size() * by[ck].size();
+      const int64_t share = std::max<int64_t>(1, class_tasks / kEriGroups);
+      for (size_t i = 0; i < runs[cb].size(); ++i)
+        for (size_t j = 0; j < runs[ck].size(); ++j) {
+          if (cb == ck && j < i) continue;  // one order of two runs
+          const Run &b = runs[cb][i], &k = runs[ck][j];
+          EriRange r{b.beg, b.end - b.beg, k.beg, k.end - k.beg, 1, 1, 1, cb == ck && i == j, (int)blocks, 0};
+          SubTask t;
+          // runs are sorted: the first pair has the most primitives, the last the fewest
+          choose_split(pairs[b.end - 1].np, pairs[b.beg].np, pairs[k.end - 1].np, pairs[k.beg].np, kEriPrim, t);
+          while (t.S * split > 256) {
+            if (t.Sk > 1) t.Sk /= 2;
+            t.S /= 2;
+          }
+          r.S = t.S;
+          r.Sk = t.Sk;
+          const size_t blk = sizeof(double) * nbra * nket;
+          r.T = (int)std::max<size_t>(1, std::min<size_t>({(size_t)256 / (r.S * split), kLdsBudget / blk, (size_t)share}));
+          L.lds = std::max(L.lds, blk * r.T);
+          const int64_t tasks = r.tri ? (int64_t)r.nbra * (r.nbra + 1) / 2 : (int64_t)r.nbra * r.nket;
+          blocks += (tasks + r.T - 1) / r.T;
+          if (blocks > std::numeric_limits<int>::max()) throw Internal("too many packed ERI blocks");
+          ranges.push_back(r);
+          ++L.nrange;
+        }
+      L.blocks = (int)blocks;
+      if (blocks) launches.push_back(L);
+    }
+  if (P.prims.empty()) P.prims.push_back(PrimPair{});
+  EriArgs a;
+  std::memset(&a, 0, sizeof(a));
+  Upload up;
+  const size_t o_sh = up.add(requested_shells(P, 0, 0)), o_prims = up.add(P.prims), o_pairs = up.add(pairs),
+               o_terms = up.add(function_terms(cart, a.nfun)), o_ranges = up.add(ranges);
+  up.send(s);
+  a.pairs = up.at<Pair>(o_pairs);
+  a.prims = up.at<PrimPair>(o_prims);
+  a.shells = up.at<ShellXYZ>(o_sh);
+  a.terms = up.at<SphTerm>(o_terms);
+  a.layout = layout;
+  a.np = np;
+  a.out = out;
+  for (const Launch& L : launches) {
+    a.ranges = up.at<EriRange>(o_ranges) + L.r0;
+    a.nrange = L.nrange;
+    const int la = pl[L.cb][0], lb = pl[L.cb][1], lc = pl[L.ck][0], ld = pl[L.ck][1];
+#define X(A, B, C, D)                                                \
+  if (la == A && lb == B && lc == C && ld == D) launch_eri_c##A##B##C##D(a, L.blocks, L.lds, s);
+    GSCF_CLASSES(X)
+#undef X
+  }
+  HIP_OK(hipGetLastError());
+  HIP_OK(hipStreamSynchronize(s));
+}
+
+// ----------------------------------------------------------------------------
+// Density-fitting integrals: the reference's compact layouts 2 (two-centre
+// metric (P|Q), m x m) and 3 (three-centre (ab|P), m x n(n+1)/2 over AO pairs
+// a >= b at pair_index(a, b)), csrc/density_fitting.cc:5-34.  The tables hold
+// orbital shells [0, split) and auxiliary shells [split, nbas).  A one-centre
+// factor P(r) is evaluated as the pair of P with a unit function (one
+// exponent-0 s primitive, coefficient 1, at P's centre), with the libcint
+// conventions of the two- and three-centre drivers (df_class.hip).
+// ----------------------------------------------------------------------------
 static void density_fitting(const int32_t* atm, int natm, const int32_t* bas, int nbas, const double* env, int nenv,
                             int cart, int layout, int split, double* out, int64_t size, hipStream_t s) {
   if (layout != 2 && layout != 3) throw Internal("Unknown compact integral layout");
@@ -3145,17 +3288,6 @@ static void density_fitting(const int32_t* atm, int natm, const int32_t* bas, in
   const int nseg = (int)P.seg.size();
   int first_aux = 0;
   while (first_aux < nseg && P.seg[first_aux].parent < split) ++first_aux;
-  std::vector<ShellXYZ> sh(nseg);
-  for (int i = 0; i < nseg; ++i) {
-    const Seg& g = P.seg[i];
-    sh[i].x = g.r[0];
-    sh[i].y = g.r[1];
-    sh[i].z = g.r[2];
-    sh[i].ao = P.ao[g.parent] - (i < first_aux ? 0 : (int)n) + g.ctr * (cart ? ncart_h(g.l) : 2 * g.l + 1);
-    sh[i].l = g.l;
-    sh[i].mol = 0;
-    sh[i].lseg = 0;
-  }
   // (auxiliary shell, unit function) pairs by angular momentum, most primitives first
   const double s2p = std::sqrt(2.0 * std::pow(3.14159265358979323846, 2.5));
   std::vector<Pair> pairs;
@@ -3186,20 +3318,11 @@ static void density_fitting(const int32_t* atm, int natm, const int32_t* bas, in
   struct Bra { int la, lb, beg, end; };
   std::vector<Bra> bras;
   if (layout == 3) {
-    std::vector<std::vector<Pair>> by_class(kNumPairClasses);
-    for (int S = 0; S < first_aux; ++S)
-      for (int T = 0; T <= S; ++T) {
-        int a = S, b = T;
-        if (P.seg[b].l > P.seg[a].l) std::swap(a, b);
-        Pair pr;
-        make_pair(P, a, b, pr);
-        by_class[pair_class(P.seg[a].l, P.seg[b].l)].push_back(pr);
-      }
+    auto by_class = pairs_by_class(P, first_aux);
     static const int pl[kNumPairClasses][2] = {{0, 0}, {1, 0}, {1, 1}, {2, 0}, {2, 1}, {2, 2}};
     for (int c = kNumPairClasses - 1; c >= 0; --c) {
       auto& v = by_class[c];
       if (v.empty()) continue;
-      std::stable_sort(v.begin(), v.end(), [](const Pair& x, const Pair& y) { return x.np > y.np; });
       bras.push_back({pl[c][0], pl[c][1], (int)pairs.size(), (int)(pairs.size() + v.size())});
       pairs.insert(pairs.end(), v.begin(), v.end());
     }
@@ -3210,36 +3333,24 @@ static void density_fitting(const int32_t* atm, int natm, const int32_t* bas, in
   // functions of every angular momentum as terms of its Cartesian components
   DfArgs a;
   std::memset(&a, 0, sizeof(a));
-  std::vector<SphTerm> terms((kDfMaxL + 1) * kDfMaxFun, SphTerm{});
-  for (int l = 0; l <= kDfMaxL; ++l) {
-    std::vector<std::vector<double>> rows;
-    if (cart) {
-      rows.assign(ncart_h(l), std::vector<double>(ncart_h(l), 0.0));
-      for (int k = 0; k < ncart_h(l); ++k) rows[k][k] = 1.0;
-    } else {
-      c2s_rows(l, rows);
-    }
-    a.nfun[l] = (int)rows.size();
-    for (size_t r = 0; r < rows.size(); ++r) {
-      SphTerm& t = terms[l * kDfMaxFun + r];
-      for (int k = 0; k < ncart_h(l); ++k) {
-        if (rows[r][k] == 0.0) continue;
-        if (t.n == kDfMaxTerms) throw Internal("solid harmonic with more Cartesian terms than the map holds");
-        t.idx[t.n] = k;
-        t.c[t.n++] = rows[r][k];
-      }
-    }
-  }
   // ranges of every launch: the pairs of a class whose primitive counts share
   // a power-of-two bucket, S lanes each so that a lane runs at most
-  // kDfPrim primitive quartets, T tasks per 256-lane block within 64 KB of LDS
-  constexpr int kDfPrim = 16;
+  // kDfPrim primitive quartets, T tasks per 256-lane block within 64 KB of LDS,
+  // fewer where the launch would not reach kDfGroups blocks ((H2O)4 cc-pVDZ /
+  // JKFIT: 1.39 ms a call pair with full blocks, 1.19 ms with 2048, 1.36 ms
+  // with 4096; 16 instead of 4 primitive quartets 1.24 ms)
+  constexpr int kDfPrim = 4;
+  constexpr int64_t kDfGroups = 2048;
   std::vector<DfRange> ranges;
   struct Launch { int lc, r0, nrange, blocks; size_t lds; };
   std::vector<Launch> launches;
   for (int lc = kDfMaxL; lc >= 0; --lc) {
     const int nket = aux0[lc + 1] - aux0[lc];
     if (nket == 0) continue;
+    int64_t tasks = 0;
+    for (const Bra& b : bras)
+      if (layout == 3 || b.la >= lc) tasks += (int64_t)(b.end - b.beg) * nket;
+    const size_t share = (size_t)std::max<int64_t>(1, tasks / kDfGroups);
     Launch L{lc, (int)ranges.size(), 0, 0, 0};
     int64_t blocks = 0;
     for (const Bra& b : bras) {
@@ -3247,11 +3358,11 @@ static void density_fitting(const int32_t* atm, int natm, const int32_t* bas, in
       const size_t blk = (size_t)ncart_h(b.la) * ncart_h(b.lb) * ncart_h(lc);
       for (int i = b.beg; i < b.end;) {
         int e = i;
-        while (e < b.end && (pairs[e].np ? bucket_of(pairs[e].np) : -1) == (pairs[i].np ? bucket_of(pairs[i].np) : -1)) ++e;
+        while (e < b.end && pair_bucket(pairs[e]) == pair_bucket(pairs[i])) ++e;
         DfRange r{b.la, b.lb, i, e - i, 1, 1, (int)blocks, 0};
         const int64_t work = (int64_t)pairs[i].np * pairs[aux0[lc]].np;
         while (r.S < 16 && (int64_t)r.S * kDfPrim < work && 2 * r.S <= pairs[e - 1].np) r.S *= 2;
-        r.T = (int)std::max<size_t>(1, std::min<size_t>(256 / (r.S * df_split(b.la, b.lb, lc)), kLdsBudget / (8 * blk)));
+        r.T = (int)std::max<size_t>(1, std::min<size_t>({(size_t)256 / (r.S * df_split(b.la, b.lb, lc)), kLdsBudget / (8 * blk), share}));
         L.lds = std::max(L.lds, 8 * blk * r.T);
         blocks += ((int64_t)r.npair * nket + r.T - 1) / r.T;
         if (blocks > std::numeric_limits<int>::max()) throw Internal("too many auxiliary integral blocks");
@@ -3265,8 +3376,8 @@ static void density_fitting(const int32_t* atm, int natm, const int32_t* bas, in
   }
   if (P.prims.empty()) P.prims.push_back(PrimPair{});
   Upload up;
-  const size_t o_sh = up.add(sh), o_prims = up.add(P.prims), o_pairs = up.add(pairs), o_terms = up.add(terms),
-               o_ranges = up.add(ranges);
+  const size_t o_sh = up.add(requested_shells(P, first_aux, (int)n)), o_prims = up.add(P.prims),
+               o_pairs = up.add(pairs), o_terms = up.add(function_terms(cart, a.nfun)), o_ranges = up.add(ranges);
   up.send(s);
   a.pairs = up.at<Pair>(o_pairs);
   a.prims = up.at<PrimPair>(o_prims);
@@ -3304,8 +3415,19 @@ static void packed_jk(const double* eri, int64_t eri_size, int ndim, const doubl
   if (!eri || !density || !out) throw Internal("Packed J/K requires device buffers");
   const size_t total = (size_t)(with_j + with_k) * nb * n * n;
   hipLaunchKernelGGL(fill_kernel, dim3(nblocks(total)), dim3(256), 0, s, out, total, 0.0);
-  hipLaunchKernelGGL(packed_jk_kernel, dim3(nblocks((size_t)(np * (np + 1) / 2))), dim3(256), 0, s, eri,
-                     ndim == 1 ? 1 : 0, np, density, nb, n, with_j, with_k, out);
+  const int64_t kbase = (int64_t)with_j * nb * n * n;
+  auto launch = [&](auto kernel, int R) {
+    const dim3 grid((unsigned)((n + R - 1) / R), (unsigned)n, (unsigned)nb);
+    const size_t lds = with_k ? sizeof(double) * 2 * (R + 1) * (size_t)n : 0;
+    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, s, eri, ndim == 1 ? 1 : 0, np, density, n, with_j, with_k,
+                       kbase, out);
+  };
+  if (n <= kPackedWide)
+    launch(packed_jk_kernel<kPackedRows>, kPackedRows);
+  else
+    launch(packed_jk_kernel<1>, 1);
+  if (with_j)
+    hipLaunchKernelGGL(mirror_kernel, dim3(nblocks((size_t)nb * n * n)), dim3(256), 0, s, out, nb, n);
   HIP_OK(hipGetLastError());
 }
 
@@ -3571,17 +3693,10 @@ int gscf_plan_get_schwarz(const gscf_plan* plan, double* q) {
 int gscf_packed_eri(const int32_t* atm, int32_t natm, const int32_t* bas, int32_t nbas, const double* env,
                     int32_t nenv, int32_t cart, int32_t layout, double* out, int64_t size, void* stream) {
   // every failure is Internal, as in the reference's compact target (compact.cc:16)
-  gscf_plan* plan = nullptr;
-  const int rc = gscf_plan_create(atm, natm, bas, nbas, env, nenv, cart, 0.0, stream, &plan);
-  if (rc != GSCF_OK) return GSCF_INTERNAL;
-  const int rc2 = guarded([&] { packed_eri(plan->d, layout, out, size, (hipStream_t)stream); });
-  if (rc2 != GSCF_OK) {
-    const std::string msg = g_error;
-    (void)gscf_plan_destroy(plan);
-    g_error = msg;
-    return GSCF_INTERNAL;
-  }
-  return gscf_plan_destroy(plan);
+  return guarded([&] { packed_eri(atm, natm, bas, nbas, env, nenv, cart, layout, out, size, (hipStream_t)stream); }) ==
+                 GSCF_OK
+             ? GSCF_OK
+             : GSCF_INTERNAL;
 }
 
 int gscf_density_fitting(const int32_t* atm, int32_t natm, const int32_t* bas, int32_t nbas, const double* env,

@@ -1345,6 +1345,157 @@ __global__ __launch_bounds__(256) void blocks_kernel(BlockArgs a) {
 }
 
 // ----------------------------------------------------------------------------
+// Integral blocks to LDS: slice sl of the primitive quartets of (bp|kp), all
+// components on one lane (blocks of at most 36) or one lane per ket component
+// kc; the S slices sit on adjacent lanes and the s0 = 0 lane stores the sum at
+// dst[bra component][ket component].
+// ----------------------------------------------------------------------------
+template <int LA, int LB, int LC, int LD>
+__device__ __forceinline__ void block_to_lds(const PrimPair* __restrict__ prims, const ShellXYZ* __restrict__ shells,
+                                             const Pair& bp, const Pair& kp, int S, int Sk, int s0, int kc,
+                                             double* __restrict__ dst) {
+  using K = Class<LA, LB, LC, LD>;
+  const ShellXYZ sA = shells[bp.sa], sB = shells[bp.sb], sC = shells[kp.sa], sD = shells[kp.sb];
+  QuartetGeom geo;
+  double AB[3], CD[3];
+  load_geom(sA, sB, sC, sD, geo, AB, CD);
+  const int Sb = S / Sk, sb = s0 & (Sb - 1), sk = s0 / Sb;
+  if constexpr (!K::kSplit) {
+    double acc[K::NA][K::NB][K::NC][K::ND];
+#pragma unroll
+    for (int e = 0; e < K::NBRA * K::NKET; ++e) (&acc[0][0][0][0])[e] = 0.0;
+    for (int ip = sb; ip < bp.np; ip += Sb) {
+      const PrimPair P = prims[bp.poff + ip];
+      for (int kq = sk; kq < kp.np; kq += Sk) {
+        PrimQ<K::NR> q;
+        prim_setup<K::NR>(P, prims[kp.poff + kq], geo, q);
+        accumulate_full<LA, LB, LC, LD>(q, AB, CD, acc);
+      }
+    }
+    group_sum<K::NBRA * K::NKET>(&acc[0][0][0][0], S);
+    if (s0 == 0)
+#pragma unroll
+      for (int e = 0; e < K::NBRA * K::NKET; ++e) dst[e] = (&acc[0][0][0][0])[e];
+  } else {
+    int ec[3], ed[3];
+    cart_xyz<LC>(kc / K::ND, ec);
+    cart_xyz<LD>(kc % K::ND, ed);
+    double wk[3][K::MM + 1];
+#pragma unroll
+    for (int x = 0; x < 3; ++x) ket_weights<K::MM>(ec[x], ed[x], CD[x], wk[x]);
+    double acc[K::NA][K::NB];
+#pragma unroll
+    for (int e = 0; e < K::NBRA; ++e) (&acc[0][0])[e] = 0.0;
+    for (int ip = sb; ip < bp.np; ip += Sb) {
+      const PrimPair P = prims[bp.poff + ip];
+      for (int kq = sk; kq < kp.np; kq += Sk) {
+        PrimQ<K::NR> q;
+        prim_setup<K::NR>(P, prims[kp.poff + kq], geo, q);
+        accumulate_split<LA, LB, LC, LD>(q, AB, wk, acc);
+      }
+    }
+    group_sum<K::NBRA>(&acc[0][0], S);
+    if (s0 == 0)
+#pragma unroll
+      for (int e = 0; e < K::NBRA; ++e) dst[e * K::NKET + kc] = (&acc[0][0])[e];
+  }
+}
+
+// Largest r with r (r + 1) / 2 <= idx.
+__device__ __forceinline__ int64_t tri_row(int64_t idx) {
+  int64_t r = (int64_t)((sqrt(8.0 * (double)idx + 1.0) - 1.0) * 0.5);
+  while (r * (r + 1) / 2 > idx) --r;
+  while ((r + 1) * (r + 2) / 2 <= idx) ++r;
+  return r;
+}
+
+// ----------------------------------------------------------------------------
+// Packed ERIs of one quartet class: every (bra pair, ket pair) combination,
+// enumerated from the block index, its Cartesian block evaluated into LDS and
+// its requested-basis elements stored from there (each unique AO quartet by
+// exactly one task, so the result needs no clearing).
+// Bound by the primitive chain of the contracted classes: a range of pairs
+// with many primitives spreads them over S lanes until a lane runs at most
+// kEriPrim (host side).  (H2O)2 6-31G*: the ssss blocks took 405 us with one
+// lane per quartet and 14 us split.
+// ----------------------------------------------------------------------------
+template <int LA, int LB, int LC, int LD>
+__global__ __launch_bounds__(256) void eri_kernel(EriArgs a) {
+  using K = Class<LA, LB, LC, LD>;
+  extern __shared__ double ebuf[];
+  int x = 0;
+  while (x + 1 < a.nrange && a.ranges[x + 1].block0 <= (int)blockIdx.x) ++x;
+  const EriRange r = a.ranges[x];
+  const int lanes = K::SPLIT * r.S;
+  const int local = threadIdx.x / lanes;
+  const int64_t t0 = (int64_t)(blockIdx.x - r.block0) * r.T;
+  const int64_t ntask = r.tri ? (int64_t)r.nbra * (r.nbra + 1) / 2 : (int64_t)r.nbra * r.nket;
+  auto task = [&](int64_t t, int& bra, int& ket) {
+    if (r.tri) {
+      const int64_t i = tri_row(t);
+      bra = r.bra0 + (int)i;
+      ket = r.ket0 + (int)(t - i * (i + 1) / 2);
+    } else {
+      bra = r.bra0 + (int)(t / r.nket);
+      ket = r.ket0 + (int)(t % r.nket);
+    }
+  };
+  if (local < r.T && t0 + local < ntask) {
+    int bra, ket;
+    task(t0 + local, bra, ket);
+    block_to_lds<LA, LB, LC, LD>(a.prims, a.shells, a.pairs[bra], a.pairs[ket], r.S, r.Sk, threadIdx.x & (r.S - 1),
+                                 (threadIdx.x / r.S) % K::SPLIT, ebuf + local * (K::NBRA * K::NKET));
+  }
+  __syncthreads();
+  const SphTerm* __restrict__ ta = a.terms + LA * kDfMaxFun;
+  const SphTerm* __restrict__ tb = a.terms + LB * kDfMaxFun;
+  const SphTerm* __restrict__ tc = a.terms + LC * kDfMaxFun;
+  const SphTerm* __restrict__ td = a.terms + LD * kDfMaxFun;
+  const int fa = a.nfun[LA], fb = a.nfun[LB], fc = a.nfun[LC], fd = a.nfun[LD];
+  const int nout = fa * fb * fc * fd;
+  for (int e = threadIdx.x; e < r.T * nout; e += blockDim.x) {
+    const int tl = e / nout;
+    if (t0 + tl >= ntask) break;
+    int rem = e - tl * nout;
+    const int w = rem % fd;
+    rem /= fd;
+    const int u = rem % fc;
+    rem /= fc;
+    const int q = rem % fb, p = rem / fb;
+    int bra, ket;
+    task(t0 + tl, bra, ket);
+    const Pair bp = a.pairs[bra], kp = a.pairs[ket];
+    if ((bp.sa == bp.sb && p < q) || (kp.sa == kp.sb && u < w)) continue;
+    const int64_t oa = a.shells[bp.sa].ao + p, ob = a.shells[bp.sb].ao + q;
+    const int64_t oc = a.shells[kp.sa].ao + u, od = a.shells[kp.sb].ao + w;
+    int64_t ab = oa > ob ? oa * (oa + 1) / 2 + ob : ob * (ob + 1) / 2 + oa;
+    int64_t cd = oc > od ? oc * (oc + 1) / 2 + od : od * (od + 1) / 2 + oc;
+    if (bra == ket && ab < cd) continue;
+    const double* __restrict__ blk = ebuf + tl * (K::NBRA * K::NKET);
+    double v = 0.0;
+    for (int i = 0; i < ta[p].n; ++i)
+      for (int j = 0; j < tb[q].n; ++j) {
+        const double* __restrict__ row = blk + (ta[p].idx[i] * K::NB + tb[q].idx[j]) * K::NKET;
+        const double fij = ta[p].c[i] * tb[q].c[j];
+        for (int k = 0; k < tc[u].n; ++k)
+          for (int l = 0; l < td[w].n; ++l)
+            v += fij * tc[u].c[k] * td[w].c[l] * row[tc[u].idx[k] * K::ND + td[w].idx[l]];
+      }
+    if (ab < cd) {
+      const int64_t s = ab;
+      ab = cd;
+      cd = s;
+    }
+    if (a.layout == 0) {
+      a.out[ab * a.np + cd] = v;
+      a.out[cd * a.np + ab] = v;
+    } else {
+      a.out[ab * (ab + 1) / 2 + cd] = v;
+    }
+  }
+}
+
+// ----------------------------------------------------------------------------
 // Launchers (instantiated per class in jk_class.hip)
 // ----------------------------------------------------------------------------
 template <int LA, int LB, int LC, int LD>
@@ -1384,6 +1535,12 @@ void request_lds(Kernel kernel, size_t bytes) {
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)bytes) != hipSuccess)
     (void)hipGetLastError();
+}
+
+template <int LA, int LB, int LC, int LD>
+void launch_eri_t(const EriArgs& a, int blocks, size_t lds, hipStream_t s) {
+  request_lds(eri_kernel<LA, LB, LC, LD>, lds);
+  hipLaunchKernelGGL((eri_kernel<LA, LB, LC, LD>), dim3((unsigned)blocks), dim3(256), lds, s, a);
 }
 
 template <int LA, int LB, int LC, int LD, int CA, int CB, int CC, int CD>
