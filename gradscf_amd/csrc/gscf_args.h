@@ -292,6 +292,18 @@ struct EriArgs {
   double* out;
 };
 
+// Schwarz blocks (pq|pq) of the pairs of one class: q[2 i] = max over the
+// requested-basis functions, q[2 i + 1] over the Cartesian components.
+struct SchwarzArgs {
+  const Pair* pairs;
+  const PrimPair* prims;
+  const ShellXYZ* shells;
+  int npairs;
+  const SphTerm* terms;     // [l][kDfMaxFun]
+  int nfun[kDfMaxL + 1];
+  double* q;
+};
+
 // Pair classes for l <= 2: index la*(la+1)/2 + lb with la >= lb.
 constexpr int kNumPairClasses = 6;
 __host__ __device__ constexpr int pair_class(int la, int lb) { return la * (la + 1) / 2 + lb; }

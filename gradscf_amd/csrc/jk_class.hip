@@ -28,4 +28,9 @@ void GSCF_NAME(launch_eri_c, GSCF_LA, GSCF_LB, GSCF_LC, GSCF_LD)(const EriArgs& 
                                                                hipStream_t s) {
   launch_eri_t<GSCF_LA, GSCF_LB, GSCF_LC, GSCF_LD>(a, blocks, lds, s);
 }
+#if GSCF_LA == GSCF_LC && GSCF_LB == GSCF_LD
+void GSCF_NAME(launch_schwarz_c, GSCF_LA, GSCF_LB, GSCF_LC, GSCF_LD)(const SchwarzArgs& a, int np, hipStream_t s) {
+  launch_schwarz_t<GSCF_LA, GSCF_LB>(a, np, s);
+}
+#endif
 }  // namespace gscf

@@ -148,6 +148,60 @@ static T* dev_upload(const std::vector<T>& v, hipStream_t s) {
   return p;
 }
 
+// Host tables uploaded as one buffer: parts are appended 16-byte aligned and
+// addressed by their offset once the buffer is on the device.
+struct Upload {
+  std::vector<char> host;
+  char* dev = nullptr;
+  template <class T>
+  size_t add(const std::vector<T>& v) {
+    const size_t at = (host.size() + 15) & ~(size_t)15;
+    host.resize(at + std::max<size_t>(1, v.size()) * sizeof(T));
+    if (!v.empty()) std::memcpy(host.data() + at, v.data(), v.size() * sizeof(T));
+    return at;
+  }
+  void send(hipStream_t s) {
+    HIP_OK(hipMalloc(&dev, host.size()));
+    HIP_OK(hipMemcpyAsync(dev, host.data(), host.size(), hipMemcpyHostToDevice, s));
+  }
+  template <class T>
+  T* at(size_t off) const { return reinterpret_cast<T*>(dev + off); }
+  char* release() {  // the caller frees the buffer
+    char* p = dev;
+    dev = nullptr;
+    return p;
+  }
+  ~Upload() {
+    if (dev) (void)hipFree(dev);
+  }
+};
+
+// Requested-basis functions of every l as terms of its Cartesian components;
+// nfun[l]: their number.
+static std::vector<SphTerm> function_terms(int cart, int (&nfun)[kDfMaxL + 1]) {
+  std::vector<SphTerm> terms((kDfMaxL + 1) * kDfMaxFun, SphTerm{});
+  for (int l = 0; l <= kDfMaxL; ++l) {
+    std::vector<std::vector<double>> rows;
+    if (cart) {
+      rows.assign(ncart_h(l), std::vector<double>(ncart_h(l), 0.0));
+      for (int k = 0; k < ncart_h(l); ++k) rows[k][k] = 1.0;
+    } else {
+      c2s_rows(l, rows);
+    }
+    nfun[l] = (int)rows.size();
+    for (size_t r = 0; r < rows.size(); ++r) {
+      SphTerm& t = terms[l * kDfMaxFun + r];
+      for (int k = 0; k < ncart_h(l); ++k) {
+        if (rows[r][k] == 0.0) continue;
+        if (t.n == kDfMaxTerms) throw Internal("solid harmonic with more Cartesian terms than the map holds");
+        t.idx[t.n] = k;
+        t.c[t.n++] = rows[r][k];
+      }
+    }
+  }
+  return terms;
+}
+
 struct Seg {
   int parent, ctr, l, np;
   double r[3];
@@ -283,6 +337,9 @@ struct PairSet {
   int* d_cinv = nullptr;
   int64_t nrows = 0;
   int nc_max = 0;
+  // device memory the pointers above (and the classes') point into
+  char* d_tables = nullptr;
+  int2* d_quartets = nullptr;
 };
 
 struct PlanData {
@@ -333,6 +390,7 @@ struct PlanData {
   // per launch stream: row lists of the exchange-row slabs of its classes, so
   // that each stream folds its own slabs as soon as its classes are done
   std::vector<int64_t*> d_lane_krp, d_lane_kent;
+  char* d_lane_tables = nullptr;   // their memory
   size_t part_nbd = 0;
   double* d_incore = nullptr;   // in-core integrals: stored Cartesian blocks of the J/K quartets
   size_t incore_doubles = 0;
@@ -360,6 +418,11 @@ struct PlanData {
   double* d_det_mol = nullptr;
   double* d_det_scale = nullptr;
   int* d_seg_atom = nullptr; // atm row of each segmented shell
+  SphTerm* d_terms = nullptr;  // [l][kDfMaxFun] requested-basis functions
+  int nfun[kDfMaxL + 1] = {0};
+  std::vector<int> p1e_order;  // all_pairs index of every d_pairs1e entry
+  char* d_tables = nullptr;     // memory of the plan's tables
+  char* d_mol_tables = nullptr; // memory of the molecule tables
   int* d_seg_ao = nullptr;   // first AO of each segmented shell in its molecule, requested basis
   // basis-parameter derivatives
   PrimAux* d_aux = nullptr;
@@ -458,6 +521,24 @@ void launch_jk_bra_class(int la, int lb, int lc, int ld, int pb, int pk, const B
   GSCF_CLASSES(X)
 #undef X
   throw Internal("no kernel for this angular-momentum class");
+}
+
+void launch_schwarz_c0000(const SchwarzArgs& a, int np, hipStream_t s);
+void launch_schwarz_c1010(const SchwarzArgs& a, int np, hipStream_t s);
+void launch_schwarz_c1111(const SchwarzArgs& a, int np, hipStream_t s);
+void launch_schwarz_c2020(const SchwarzArgs& a, int np, hipStream_t s);
+void launch_schwarz_c2121(const SchwarzArgs& a, int np, hipStream_t s);
+void launch_schwarz_c2222(const SchwarzArgs& a, int np, hipStream_t s);
+
+static void launch_schwarz_class(int la, int lb, const SchwarzArgs& a, int np, hipStream_t s) {
+  switch (pair_class(la, lb)) {
+    case 0: launch_schwarz_c0000(a, np, s); break;
+    case 1: launch_schwarz_c1010(a, np, s); break;
+    case 2: launch_schwarz_c1111(a, np, s); break;
+    case 3: launch_schwarz_c2020(a, np, s); break;
+    case 4: launch_schwarz_c2121(a, np, s); break;
+    default: launch_schwarz_c2222(a, np, s); break;
+  }
 }
 
 void launch_jk_class(int la, int lb, int lc, int ld, const JKArgs& a, hipStream_t s) {
@@ -692,32 +773,55 @@ __global__ void finalize_kernel(const double* __restrict__ jp, const double* __r
   out[i] = s;
 }
 
-// Quartet list of one sub-task: g -> (bra0 + b, ket0 + g - qoff[b]) with qoff[b] <= g < qoff[b+1].
-// Quartets of one (bra run, ket run) sub-task: bra b keeps the ket-run prefix
-// [0, qoff[b+1] - qoff[b]) (Schwarz-descending run).  The prefix is cut into
-// segments of seg kets (the ket windows of single-bra chunks) and each segment
-// is written in the run's primitive-count order: groups[k] = (begin, count) of
-// group k in order[], whose entries are run positions, ascending inside a
-// group, groups largest primitive count first.  Adjacent lanes then take kets
-// of near-equal primitive counts, so their loop trip counts agree, and every
-// segment keeps its set of kets.
-__global__ void expand_kernel(const int64_t* __restrict__ qoff, int nbra, int bra0, int ket0, int64_t nq,
-                              int seg, const int* __restrict__ order, const int2* __restrict__ groups,
-                              int ngroups, int2* __restrict__ out) {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= nq) return;
-  int lo = 0, hi = nbra;
+// Quartet lists of every (bra run, ket run) sub-task of a plan, one launch:
+// g -> (bra0 + b, ket0 + g - qoff[b]) with qoff[b] <= g - g0 < qoff[b+1].
+// Bra b keeps the ket-run prefix [0, qoff[b+1] - qoff[b]) (Schwarz-descending
+// run).  The prefix is cut into segments of seg kets (the ket windows of
+// single-bra chunks) and each segment is written in the run's primitive-count
+// order: groups[k] = (begin, count) of group k in order[], whose entries are
+// run positions, ascending inside a group, groups largest primitive count
+// first.  Adjacent lanes then take kets of near-equal primitive counts, so
+// their loop trip counts agree, and every segment keeps its set of kets.
+// (One launch, upload and synchronisation per sub-task took 5 of the 9 ms of
+// a plan for (H2O)3 6-31G*: 115 sub-tasks.)
+struct ExpandTask {
+  int64_t g0;      // first quartet of the sub-task in the plan's list
+  int64_t qoff;    // its nbra + 1 prefix sums in the plan's table
+  int nbra, bra0, ket0, seg;
+  int grp0, ngrp;  // groups of the ket run
+  int sorted;      // the chunk sort reads the list from the scratch copy
+  int pad;
+};
+
+__global__ __launch_bounds__(256) void expand_kernel(const ExpandTask* __restrict__ tasks, int ntask, int64_t total,
+                                                     const int64_t* __restrict__ qoff_all,
+                                                     const int* __restrict__ order_all,
+                                                     const int2* __restrict__ groups_all, int2* __restrict__ scratch,
+                                                     int2* __restrict__ out) {
+  const int64_t gg = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (gg >= total) return;
+  int t0 = 0, t1 = ntask;
+  while (t1 - t0 > 1) {
+    const int mid = (t0 + t1) >> 1;
+    if (tasks[mid].g0 <= gg) t0 = mid; else t1 = mid;
+  }
+  const ExpandTask t = tasks[t0];
+  const int64_t g = gg - t.g0;
+  const int64_t* __restrict__ qoff = qoff_all + t.qoff;
+  const int* __restrict__ order = order_all + t.ket0;
+  const int2* __restrict__ groups = groups_all + t.grp0;
+  int lo = 0, hi = t.nbra;
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
     if (qoff[mid] <= g) lo = mid; else hi = mid;
   }
   const int cnt = (int)(qoff[lo + 1] - qoff[lo]);
   const int r = (int)(g - qoff[lo]);
-  const int s0 = r - r % seg, s1 = (cnt - s0 > seg) ? s0 + seg : cnt;
+  const int s0 = r - r % t.seg, s1 = (cnt - s0 > t.seg) ? s0 + t.seg : cnt;
   int rr = r - s0, ket = r;
   // the groups partition the run, so their members in [s0, s1) number exactly
   // s1 - s0 and rr < s1 - s0 lands in one of them
-  for (int k = 0; k < ngroups; ++k) {
+  for (int k = 0; k < t.ngrp; ++k) {
     const int2 gr = groups[k];
     int a = 0, b = gr.y;
     while (a < b) {
@@ -736,7 +840,7 @@ __global__ void expand_kernel(const int64_t* __restrict__ qoff, int nbra, int br
     }
     rr -= c - a;
   }
-  out[g] = make_int2(bra0 + lo, ket0 + ket);
+  (t.sorted ? scratch : out)[gg] = make_int2(t.bra0 + lo, t.ket0 + ket);
 }
 
 // Order of the quartets inside every bra-major chunk: by ket primitive-pair
@@ -748,20 +852,38 @@ __global__ void expand_kernel(const int64_t* __restrict__ qoff, int nbra, int br
 // reads neighbouring grid rows.  One workgroup per chunk: 64-bit keys
 // (count, distance bits, position) bitonic-sorted in LDS, then the quartets
 // gathered through a scratch copy.  nq of a chunk is at most kSortMax.
+// Chunks of every class in one launch; src and dst are the plan's lists.
 constexpr int kSortMax = 8192;
-__global__ __launch_bounds__(256) void sort_chunk_kernel(const BraChunk* __restrict__ chunks,
+
+// Chunks [chunk0, next class's chunk0) of one class whose quartets start at q0
+// of the plan's list; sort 0: too long to sort, copied.
+struct SortClass {
+  int chunk0, sort;
+  int64_t q0;
+};
+
+__global__ __launch_bounds__(256) void sort_chunk_kernel(const SortClass* __restrict__ classes, int nclass,
+                                                         const BraChunk* __restrict__ chunks,
                                                          const Pair* __restrict__ pairs,
                                                          const ShellXYZ* __restrict__ shells,
-                                                         const int2* __restrict__ src, int2* __restrict__ dst) {
-  __shared__ uint64_t key[kSortMax];
+                                                         const int2* __restrict__ src_all, int2* __restrict__ dst_all) {
+  extern __shared__ uint64_t key[];
+  int k = 0;
+  while (k + 1 < nclass && classes[k + 1].chunk0 <= (int)blockIdx.x) ++k;
   const BraChunk c = chunks[blockIdx.x];
+  const int2* __restrict__ src = src_all + classes[k].q0 + c.q0;
+  int2* __restrict__ dst = dst_all + classes[k].q0 + c.q0;
   const int nq = c.nq;
+  if (!classes[k].sort) {
+    for (int i = threadIdx.x; i < nq; i += blockDim.x) dst[i] = src[i];
+    return;
+  }
   int np2 = 1;
   while (np2 < nq) np2 <<= 1;
   for (int i = threadIdx.x; i < np2; i += blockDim.x) {
-    uint64_t k = ~0ull;
+    uint64_t v = ~0ull;
     if (i < nq) {
-      const int2 q = src[c.q0 + i];
+      const int2 q = src[i];
       const Pair b = pairs[q.x], t = pairs[q.y];
       const ShellXYZ A = shells[b.sa], B = shells[b.sb], C = shells[t.sa], D = shells[t.sb];
       const double dx = 0.5 * (A.x + B.x - C.x - D.x), dy = 0.5 * (A.y + B.y - C.y - D.y),
@@ -769,9 +891,9 @@ __global__ __launch_bounds__(256) void sort_chunk_kernel(const BraChunk* __restr
       const float d2 = (float)(dx * dx + dy * dy + dz * dz);
       const uint32_t fb = __float_as_uint(d2) >> 1;  // non-negative: bits order as the values
       const uint32_t npk = 65535u - (uint32_t)min(t.np, 65535);
-      k = ((uint64_t)npk << 45) | ((uint64_t)fb << 14) | (uint64_t)i;
+      v = ((uint64_t)npk << 45) | ((uint64_t)fb << 14) | (uint64_t)i;
     }
-    key[i] = k;
+    key[i] = v;
   }
   __syncthreads();
   for (int size = 2; size <= np2; size <<= 1)
@@ -788,7 +910,7 @@ __global__ __launch_bounds__(256) void sort_chunk_kernel(const BraChunk* __restr
       }
       __syncthreads();
     }
-  for (int i = threadIdx.x; i < nq; i += blockDim.x) dst[c.q0 + i] = src[c.q0 + (int)(key[i] & 0x3fff)];
+  for (int i = threadIdx.x; i < nq; i += blockDim.x) dst[i] = src[(int)(key[i] & 0x3fff)];
 }
 
 // dmax[m][S][T] = max over batches and over the Cartesian block (S, T) of |D_m|
@@ -1089,88 +1211,58 @@ static void run_blocks(PlanData& P, const Pair* d_pairs, const std::vector<Block
   HIP_OK(hipFree(d_tasks));
 }
 
+// Schwarz blocks of every segment pair of d_pairs1e: max |(pq|pq)| over the
+// requested-basis functions into seg_q (all_pairs order), over the Cartesian
+// components into cart_q (schwarz_kernel).
 static void compute_schwarz(PlanData& P, std::vector<double>& seg_q, hipStream_t s,
                             std::vector<double>* cart_q = nullptr) {
   const int npair = (int)P.all_pairs.size();
-  // tasks sorted by pair class
-  std::vector<int> order(npair);
-  for (int i = 0; i < npair; ++i) order[i] = i;
-  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return P.all_class[x] < P.all_class[y]; });
-  std::vector<BlockTask> tasks;
-  std::vector<std::array<int, 4>> tcls;
-  std::vector<int64_t> base(npair);
-  int64_t total = 0;
-  for (int i : order) {
-    const Pair& pr = P.all_pairs[i];
-    const int la = P.seg[pr.sa].l, lb = P.seg[pr.sb].l;
-    const int na = ncart_h(la), nb = ncart_h(lb);
-    BlockTask t;
-    t.bra = t.ket = i;
-    t.base = total;
-    base[i] = total;
-    t.stride[0] = 1;
-    t.stride[1] = na;
-    t.stride[2] = na * nb;
-    t.stride[3] = na * nb * na;
-    for (int k = 0; k < 4; ++k) t.coff[k] = 0;
-    tasks.push_back(t);
-    tcls.push_back({la, lb, la, lb});
-    total += (int64_t)na * nb * na * nb;
-  }
-  double* d_out = nullptr;
-  HIP_OK(hipMalloc(&d_out, sizeof(double) * std::max<int64_t>(total, 1)));
-  run_blocks(P, P.d_all_pairs, tasks, tcls, d_out, s);
-  std::vector<double> h(total);
-  HIP_OK(hipMemcpy(h.data(), d_out, sizeof(double) * total, hipMemcpyDeviceToHost));
-  HIP_OK(hipFree(d_out));
   seg_q.assign(npair, 0.0);
   if (cart_q) cart_q->assign(npair, 0.0);
-  for (int i = 0; i < npair; ++i) {
-    const Pair& pr = P.all_pairs[i];
-    const int la = P.seg[pr.sa].l, lb = P.seg[pr.sb].l;
-    const int na = ncart_h(la), nb = ncart_h(lb);
-    const double* B = h.data() + base[i];
-    auto at = [&](int a, int b, int c, int d) { return B[((d * na + c) * nb + b) * na + a]; };
-    double largest = 0.0;
-    if (cart_q) {
-      double lc = 0.0;
-      for (int a = 0; a < na; ++a)
-        for (int b = 0; b < nb; ++b) lc = std::max(lc, std::fabs(at(a, b, a, b)));
-      (*cart_q)[i] = lc;
-    }
-    if (P.cart) {
-      for (int a = 0; a < na; ++a)
-        for (int b = 0; b < nb; ++b) largest = std::max(largest, std::fabs(at(a, b, a, b)));
-    } else {
-      std::vector<std::vector<double>> ta, tb;
-      c2s_rows(la, ta);
-      c2s_rows(lb, tb);
-      for (size_t sa = 0; sa < ta.size(); ++sa)
-        for (size_t sb = 0; sb < tb.size(); ++sb) {
-          double v = 0.0;
-          for (int a1 = 0; a1 < na; ++a1) {
-            if (ta[sa][a1] == 0) continue;
-            for (int a2 = 0; a2 < na; ++a2) {
-              if (ta[sa][a2] == 0) continue;
-              for (int b1 = 0; b1 < nb; ++b1) {
-                if (tb[sb][b1] == 0) continue;
-                for (int b2 = 0; b2 < nb; ++b2) {
-                  if (tb[sb][b2] == 0) continue;
-                  v += ta[sa][a1] * ta[sa][a2] * tb[sb][b1] * tb[sb][b2] * at(a1, b1, a2, b2);
-                }
-              }
-            }
-          }
-          largest = std::max(largest, std::fabs(v));
-        }
-    }
-    seg_q[i] = largest;
+  if (npair == 0) return;
+  double* d_q = nullptr;
+  HIP_OK(hipMalloc(&d_q, sizeof(double) * 2 * npair));
+  SchwarzArgs a;
+  a.prims = P.d_prims;
+  a.shells = P.d_shells;
+  a.terms = P.d_terms;
+  std::copy(P.nfun, P.nfun + kDfMaxL + 1, a.nfun);
+  static const int pl[kNumPairClasses][2] = {{0, 0}, {1, 0}, {1, 1}, {2, 0}, {2, 1}, {2, 2}};
+  for (int c = 0; c < kNumPairClasses; ++c) {
+    const int b = P.p1e_begin[c], e = P.p1e_begin[c + 1];
+    if (b == e) continue;
+    int np = 1;
+    for (int k = b; k < e; ++k) np = std::max(np, P.all_pairs[P.p1e_order[k]].np);
+    a.pairs = P.d_pairs1e + b;
+    a.npairs = e - b;
+    a.q = d_q + 2 * b;
+    launch_schwarz_class(pl[c][0], pl[c][1], a, np, s);
+  }
+  std::vector<double> h(2 * (size_t)npair);
+  const hipError_t launched = hipGetLastError();
+  const hipError_t copied = hipMemcpyAsync(h.data(), d_q, sizeof(double) * 2 * npair, hipMemcpyDeviceToHost, s);
+  const hipError_t done = hipStreamSynchronize(s);
+  (void)hipFree(d_q);
+  HIP_OK(launched);
+  HIP_OK(copied);
+  HIP_OK(done);
+  for (int k = 0; k < npair; ++k) {
+    seg_q[P.p1e_order[k]] = h[2 * k];
+    if (cart_q) (*cart_q)[P.p1e_order[k]] = h[2 * k + 1];
   }
 }
 
-static void build_c2s_maps(PlanData& P, hipStream_t s) {
-  std::vector<int> cidx((size_t)P.n_cart * 2, 0), sidx((size_t)P.n * 3, 0);
-  std::vector<double> ccoef((size_t)P.n_cart * 2, 0.0), scoef((size_t)P.n * 3, 0.0);
+struct C2sTables {
+  std::vector<int> cidx, sidx;
+  std::vector<double> ccoef, scoef;
+};
+
+static C2sTables c2s_maps(const PlanData& P) {
+  C2sTables t;
+  t.cidx.assign((size_t)P.n_cart * 2, 0);
+  t.sidx.assign((size_t)P.n * 3, 0);
+  t.ccoef.assign((size_t)P.n_cart * 2, 0.0);
+  t.scoef.assign((size_t)P.n * 3, 0.0);
   // positions are global AO indices, stored indices are local to the molecule
   for (int mo = 0; mo < P.nmol; ++mo)
   for (int sh = P.mol_bas[mo]; sh < P.mol_bas[mo + 1]; ++sh) {
@@ -1192,8 +1284,8 @@ static void build_c2s_maps(PlanData& P, hipStream_t s) {
         for (int f = 0; f < nf; ++f)
           if (T[m][f] != 0.0) {
             if (k >= 3) throw Internal("c2s map overflow");
-            sidx[(size_t)(sbase + m) * 3 + k] = cb + f - aoc0;
-            scoef[(size_t)(sbase + m) * 3 + k] = T[m][f];
+            t.sidx[(size_t)(sbase + m) * 3 + k] = cb + f - aoc0;
+            t.scoef[(size_t)(sbase + m) * 3 + k] = T[m][f];
             ++k;
           }
       }
@@ -1202,17 +1294,14 @@ static void build_c2s_maps(PlanData& P, hipStream_t s) {
         for (int m = 0; m < ns; ++m)
           if (T[m][f] != 0.0) {
             if (k >= 2) throw Internal("c2s map overflow");
-            cidx[(size_t)(cb + f) * 2 + k] = sbase + m - ao0;
-            ccoef[(size_t)(cb + f) * 2 + k] = T[m][f];
+            t.cidx[(size_t)(cb + f) * 2 + k] = sbase + m - ao0;
+            t.ccoef[(size_t)(cb + f) * 2 + k] = T[m][f];
             ++k;
           }
       }
     }
   }
-  P.d_c2s_idx = dev_upload(cidx, s);
-  P.d_c2s_coef = dev_upload(ccoef, s);
-  P.d_s2c_idx = dev_upload(sidx, s);
-  P.d_s2c_coef = dev_upload(scoef, s);
+  return t;
 }
 
 static int bucket_of(int np) {
@@ -1365,14 +1454,16 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
   // runs of each (class, molecule) in list order, for the intra-molecule pairing
   std::map<std::pair<int, int>, std::vector<int>> runs_of;
   for (int i = 0; i < (int)runs.size(); ++i) runs_of[{runs[i].cls, runs[i].mol}].push_back(i);
-  S.d_pairs = dev_upload(S.pairs, s);
-  int* d_run_order = dev_upload(run_order, s);
-  int2* d_run_groups = dev_upload(run_groups, s);
-  {
-    std::vector<double> pq = S.pair_q;
-    if (pq.empty()) pq.push_back(0.0);
-    S.d_pair_q = dev_upload(pq, s);
-  }
+  Upload up, work;  // tables the set keeps, tables of the expansion
+  const size_t o_pairs = up.add(S.pairs), o_pair_q = up.add(S.pair_q);
+  std::vector<ExpandTask> expand;
+  std::vector<int64_t> qoffs;
+  std::vector<SortClass> sort_classes;
+  std::vector<BraChunk> chunks;
+  std::vector<SubTask> subtasks;
+  struct Place { int64_t q0; size_t chunk0, task0; };
+  std::vector<Place> place;  // of every class in the three lists
+  int sort_len = 1;
   static const int pl[kNumPairClasses][2] = {{0, 0}, {1, 0}, {1, 1}, {2, 0}, {2, 1}, {2, 2}};
   S.nquartets = 0;
   S.part_total = 0;
@@ -1613,51 +1704,43 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
               }
               qc.part_end = S.part_total;
             }
-            if (qc.nbra_max >= 1) qc.d_chunks = dev_upload(qc.chunks, s);
-          }
-          HIP_OK(hipMalloc(&qc.d_quartets, sizeof(int2) * qc.nq));
-          for (const Pending& pd : pend) {
-            int64_t* d_qoff = dev_upload(pd.qoff, s);
-            hipLaunchKernelGGL(expand_kernel, dim3(nblocks((size_t)pd.nq)), dim3(256), 0, s, d_qoff, pd.nbra,
-                               pd.bra0, pd.ket0, pd.nq, pd.seg, d_run_order + pd.ket0, d_run_groups + run_g0[pd.rk],
-                               run_g0[pd.rk + 1] - run_g0[pd.rk], qc.d_quartets + pd.q0);
-            HIP_OK(hipGetLastError());
-            HIP_OK(hipStreamSynchronize(s));
-            HIP_OK(hipFree(d_qoff));
           }
           int64_t nq_chunk_max = 0;
           for (const BraChunk& c : qc.chunks) nq_chunk_max = std::max<int64_t>(nq_chunk_max, c.nq);
-          // (tuned chunk sizes above kSortMax keep the expansion order)
-          if (qc.d_chunks && !qc.chunks.empty() && nq_chunk_max <= kSortMax) {
-            int2* tmp = nullptr;
-            HIP_OK(hipMalloc(&tmp, sizeof(int2) * qc.nq));
-            HIP_OK(hipMemcpyAsync(tmp, qc.d_quartets, sizeof(int2) * qc.nq, hipMemcpyDeviceToDevice, s));
-            hipLaunchKernelGGL(sort_chunk_kernel, dim3((unsigned)qc.chunks.size()), dim3(256), 0, s, qc.d_chunks,
-                               S.d_pairs, S.d_shells, tmp, qc.d_quartets);
-            HIP_OK(hipGetLastError());
-            HIP_OK(hipStreamSynchronize(s));
-            HIP_OK(hipFree(tmp));
+          if (qc.nbra_max < 1) qc.chunks.clear();
+          place.push_back({S.nquartets, chunks.size(), subtasks.size()});
+          for (const Pending& pd : pend) {
+            expand.push_back({S.nquartets + pd.q0, (int64_t)qoffs.size(), pd.nbra, pd.bra0, pd.ket0, pd.seg,
+                              run_g0[pd.rk], run_g0[pd.rk + 1] - run_g0[pd.rk], !qc.chunks.empty(), 0});
+            qoffs.insert(qoffs.end(), pd.qoff.begin(), pd.qoff.end());
           }
-          qc.d_tasks = dev_upload(qc.tasks, s);
+          if (!qc.chunks.empty()) {
+            // (tuned chunk sizes above kSortMax keep the expansion order)
+            const bool sort = nq_chunk_max <= kSortMax;
+            sort_classes.push_back({(int)chunks.size(), sort, S.nquartets});
+            while (sort && sort_len < nq_chunk_max) sort_len <<= 1;
+            chunks.insert(chunks.end(), qc.chunks.begin(), qc.chunks.end());
+          }
+          subtasks.insert(subtasks.end(), qc.tasks.begin(), qc.tasks.end());
           S.nquartets += qc.nq;
           S.classes.push_back(std::move(qc));
         }
-  HIP_OK(hipFree(d_run_order));
-  HIP_OK(hipFree(d_run_groups));
+  const size_t o_chunks = up.add(chunks), o_tasks = up.add(subtasks);
   if (S.part_total * (int64_t)sizeof(double) > kPartCapBytes) {
     S.part_total = 0;
     for (QuartetClass& qc : S.classes) qc.part = false;
   }
+  size_t o_krp = 0, o_kent = 0, o_jrp = 0, o_jent = 0, o_row_dst = 0, o_row_n = 0, o_row_mol = 0;
   if (S.part_total > 0) {
     // CSR lists: K by global Cartesian row, J by ket pair
-    auto csr = [&](std::vector<std::pair<int64_t, int64_t>>& ent, int64_t nkeys, int64_t*& d_rp, int64_t*& d_ent) {
+    auto csr = [&](std::vector<std::pair<int64_t, int64_t>>& ent, int64_t nkeys, size_t& o_rp, size_t& o_ent) {
       std::vector<int64_t> rp(nkeys + 1, 0), off(std::max<size_t>(1, ent.size()));
       for (const auto& e : ent) ++rp[e.first + 1];
       for (int64_t k = 0; k < nkeys; ++k) rp[k + 1] += rp[k];
       std::vector<int64_t> fill(rp.begin(), rp.end() - 1);
       for (const auto& e : ent) off[fill[e.first]++] = e.second;
-      d_rp = dev_upload(rp, s);
-      d_ent = dev_upload(off, s);
+      o_rp = up.add(rp);
+      o_ent = up.add(off);
     };
     int64_t nrows = 0;
     for (int m = 0; m < P.nmol; ++m) nrows = std::max<int64_t>(nrows, (int64_t)P.mols[m].aoc0 + P.mols[m].nc);
@@ -1671,21 +1754,62 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
         S.nc_max = std::max(S.nc_max, P.mols[m].nc);
       }
     S.nrows = nrows;
-    S.d_row_dst = dev_upload(row_dst, s);
-    S.d_row_n = dev_upload(row_n, s);
-    S.d_row_mol = dev_upload(row_mol, s);
-    csr(kent, nrows * 8, S.d_krp, S.d_kent);
-    csr(jent, (int64_t)S.pairs.size(), S.d_jrp, S.d_jent);
+    o_row_dst = up.add(row_dst);
+    o_row_n = up.add(row_n);
+    o_row_mol = up.add(row_mol);
+    csr(kent, nrows * 8, o_krp, o_kent);
+    csr(jent, (int64_t)S.pairs.size(), o_jrp, o_jent);
     S.h_kent = std::move(kent);
     S.h_kent_cls = std::move(kent_cls);
   }
-  if (!colmap.empty()) {
-    S.d_colmap = dev_upload(colmap, s);
-    S.d_cinv = dev_upload(cinv, s);
-    S.d_shell_cofs = dev_upload(shell_cofs, s);
+  const size_t o_colmap = up.add(colmap), o_cinv = up.add(cinv), o_cofs = up.add(shell_cofs),
+               o_cspace = up.add(S.h_cspace), o_cinv_off = up.add(cinv_off);
+  up.send(s);
+  S.d_tables = up.release();
+  auto at = [&](size_t off) { return S.d_tables + off; };
+  S.d_pairs = (Pair*)at(o_pairs);
+  S.d_pair_q = (double*)at(o_pair_q);
+  if (S.part_total > 0) {
+    S.d_krp = (int64_t*)at(o_krp);
+    S.d_kent = (int64_t*)at(o_kent);
+    S.d_jrp = (int64_t*)at(o_jrp);
+    S.d_jent = (int64_t*)at(o_jent);
+    S.d_row_dst = (int64_t*)at(o_row_dst);
+    S.d_row_n = (int*)at(o_row_n);
+    S.d_row_mol = (int*)at(o_row_mol);
   }
-  S.d_cspace = dev_upload(S.h_cspace, s);
-  S.d_cinv_off = dev_upload(cinv_off, s);
+  if (!colmap.empty()) {
+    S.d_colmap = (int*)at(o_colmap);
+    S.d_cinv = (int*)at(o_cinv);
+    S.d_shell_cofs = (int*)at(o_cofs);
+  }
+  S.d_cspace = (int2*)at(o_cspace);
+  S.d_cinv_off = (int64_t*)at(o_cinv_off);
+  if (S.nquartets > 0) {
+    HIP_OK(hipMalloc(&S.d_quartets, sizeof(int2) * S.nquartets));
+    for (size_t c = 0; c < S.classes.size(); ++c) {
+      QuartetClass& qc = S.classes[c];
+      qc.d_quartets = S.d_quartets + place[c].q0;
+      if (!qc.chunks.empty()) qc.d_chunks = (BraChunk*)at(o_chunks) + place[c].chunk0;
+      qc.d_tasks = (SubTask*)at(o_tasks) + place[c].task0;
+    }
+    const size_t o_expand = work.add(expand), o_qoff = work.add(qoffs), o_order = work.add(run_order),
+                 o_groups = work.add(run_groups), o_sort = work.add(sort_classes);
+    work.send(s);
+    int2* scratch = nullptr;
+    if (!chunks.empty()) HIP_OK(hipMalloc(&scratch, sizeof(int2) * S.nquartets));
+    hipLaunchKernelGGL(expand_kernel, dim3(nblocks((size_t)S.nquartets)), dim3(256), 0, s,
+                       work.at<ExpandTask>(o_expand), (int)expand.size(), S.nquartets, work.at<int64_t>(o_qoff),
+                       work.at<int>(o_order), work.at<int2>(o_groups), scratch, S.d_quartets);
+    if (!chunks.empty())
+      hipLaunchKernelGGL(sort_chunk_kernel, dim3((unsigned)chunks.size()), dim3(256), sizeof(uint64_t) * sort_len, s,
+                         work.at<SortClass>(o_sort), (int)sort_classes.size(), (const BraChunk*)at(o_chunks),
+                         S.d_pairs, S.d_shells, scratch, S.d_quartets);
+    const hipError_t launched = hipGetLastError(), done = hipStreamSynchronize(s);
+    if (scratch) (void)hipFree(scratch);
+    HIP_OK(launched);
+    HIP_OK(done);
+  }
   S.built = true;
 }
 
@@ -1697,14 +1821,7 @@ static void free_pair_set(PairSet& S) {
     f(S.d_shells);
     f(S.d_prims);
   }
-  f(S.d_coef); f(S.d_blk); f(S.d_pairs); f(S.d_pair_q);
-  f(S.d_krp); f(S.d_kent); f(S.d_jrp); f(S.d_jent); f(S.d_row_dst); f(S.d_row_n); f(S.d_row_mol);
-  f(S.d_colmap); f(S.d_cspace); f(S.d_cinv_off); f(S.d_cinv); f(S.d_shell_cofs);
-  for (auto& c : S.classes) {
-    f(c.d_quartets);
-    f(c.d_tasks);
-    f(c.d_chunks);
-  }
+  f(S.d_coef); f(S.d_blk); f(S.d_tables); f(S.d_quartets);
   S = PairSet();
 }
 
@@ -1872,8 +1989,8 @@ static bool build_contracted_set(PlanData& P, hipStream_t s) {
 // balance_lanes), and build each stream's exchange-row reduction lists.
 static void assign_lanes(PlanData& P) {
   const int ns = (int)P.side.size() + 1;
-  for (int64_t* p : P.d_lane_krp) HIP_OK(hipFree(p));
-  for (int64_t* p : P.d_lane_kent) HIP_OK(hipFree(p));
+  if (P.d_lane_tables) HIP_OK(hipFree(P.d_lane_tables));
+  P.d_lane_tables = nullptr;
   P.d_lane_krp.clear();
   P.d_lane_kent.clear();
   P.lane_classes.assign(ns, {});
@@ -1893,8 +2010,10 @@ static void assign_lanes(PlanData& P) {
     std::vector<int> lane_of(S.classes.size(), 0);
     for (int l = 0; l < ns; ++l)
       for (int ci : P.lane_classes[l]) lane_of[ci] = l;
+    const int64_t nkeys = S.nrows * 8;  // (row, ket mask)
+    Upload up;
+    std::vector<size_t> o_rp, o_ent;
     for (int l = 0; l < ns; ++l) {
-      const int64_t nkeys = S.nrows * 8;  // (row, ket mask)
       std::vector<int64_t> rp(nkeys + 1, 0), off;
       for (size_t i = 0; i < S.h_kent.size(); ++i)
         if (lane_of[S.h_kent_cls[i]] == l) ++rp[S.h_kent[i].first + 1];
@@ -1903,16 +2022,22 @@ static void assign_lanes(PlanData& P) {
       std::vector<int64_t> fill(rp.begin(), rp.end() - 1);
       for (size_t i = 0; i < S.h_kent.size(); ++i)
         if (lane_of[S.h_kent_cls[i]] == l) off[fill[S.h_kent[i].first]++] = S.h_kent[i].second;
-      P.d_lane_krp.push_back(dev_upload(rp, nullptr));
-      P.d_lane_kent.push_back(dev_upload(off, nullptr));
+      o_rp.push_back(up.add(rp));
+      o_ent.push_back(up.add(off));
     }
+    up.send(nullptr);
+    for (int l = 0; l < ns; ++l) {
+      P.d_lane_krp.push_back(up.at<int64_t>(o_rp[l]));
+      P.d_lane_kent.push_back(up.at<int64_t>(o_ent[l]));
+    }
+    P.d_lane_tables = up.release();
     // the lists are read from the plan's non-blocking streams
     HIP_OK(hipDeviceSynchronize());
   }
 }
 
-// Side streams and fork/join events of the class launches, then the lanes.
-static void assign_streams(PlanData& P) {
+// Side streams and fork/join events of the class launches.
+static void make_streams(PlanData& P) {
   const int ns = std::max(1, std::min<int>(kMaxStreams, P.options.streams));
   for (int l = 1; l < ns; ++l) {
     hipStream_t st;
@@ -1923,7 +2048,6 @@ static void assign_streams(PlanData& P) {
     P.join_ev.push_back(ev);
   }
   if (ns > 1) HIP_OK(hipEventCreateWithFlags(&P.fork_ev, hipEventDisableTiming));
-  assign_lanes(P);
 }
 
 // Schwarz tables of the deterministic scale (det_scale_kernel): Cartesian
@@ -2004,7 +2128,8 @@ static void build_plan(PlanData& P, double cutoff, hipStream_t s) {
     sh[i].mol = P.seg[i].mol;
     sh[i].lseg = P.seg[i].lseg;
   }
-  P.d_shells = dev_upload(sh, s);
+  Upload up;
+  const size_t o_shells = up.add(sh);
   // all intra-molecule segmented pairs S >= T, molecule by molecule
   P.mol_pair0.assign(P.nmol + 1, 0);
   for (int m = 0; m < P.nmol; ++m) {
@@ -2024,9 +2149,8 @@ static void build_plan(PlanData& P, double cutoff, hipStream_t s) {
     P.prims.push_back(PrimPair{});
     P.aux.push_back(PrimAux{});
   }
-  P.d_prims = dev_upload(P.prims, s);
-  P.d_aux = dev_upload(P.aux, s);
-  P.d_all_pairs = dev_upload(P.all_pairs, s);
+  const size_t o_prims = up.add(P.prims), o_aux = up.add(P.aux), o_all_pairs = up.add(P.all_pairs);
+  size_t o_seg_prim0, o_slots, o_fsp, o_seg_atom, o_seg_ao, o_p1e, o_nuclei;
   {
     // primitive slots of every segmented shell and where they live in env
     const double pi = 3.14159265358979323846;
@@ -2043,12 +2167,68 @@ static void build_plan(PlanData& P, double cutoff, hipStream_t s) {
         fsp.push_back(f);
       }
     }
-    P.d_seg_prim0 = dev_upload(P.seg_prim0, s);
-    P.d_prim_slots = dev_upload(slots, s);
-    P.d_prim_fsp = dev_upload(fsp, s);
+    o_seg_prim0 = up.add(P.seg_prim0);
+    o_slots = up.add(slots);
+    o_fsp = up.add(fsp);
   }
-  // Schwarz bounds (parent-shell maxima, as the reference defines them per shell pair)
+  {
+    std::vector<int> at;
+    for (const Seg& g : P.seg) at.push_back(P.bas[g.parent * BAS_SLOTS + ATOM_OF]);
+    o_seg_atom = up.add(at);
+    std::vector<int> ao;
+    for (const Seg& g : P.seg)
+      ao.push_back(P.ao[g.parent] - P.mols[g.mol].ao0 + g.ctr * (P.cart ? ncart_h(g.l) : 2 * g.l + 1));
+    o_seg_ao = up.add(ao);
+  }
   const int npair = (int)P.all_pairs.size();
+  {
+    std::vector<int> order(npair);
+    for (int i = 0; i < npair; ++i) order[i] = i;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return P.all_class[x] < P.all_class[y]; });
+    std::vector<Pair> p1e;
+    int k = 0;
+    for (int c = 0; c < kNumPairClasses; ++c) {
+      P.p1e_begin[c] = k;
+      while (k < npair && P.all_class[order[k]] == c) p1e.push_back(P.all_pairs[order[k++]]);
+    }
+    P.p1e_begin[kNumPairClasses] = k;
+    P.p1e_order = std::move(order);
+    o_p1e = up.add(p1e);
+    std::vector<double> nuc;
+    for (int m = 0; m < P.nmol; ++m)
+      for (int a = P.mol_atm[m]; a < P.mol_atm[m + 1]; ++a) {
+        const int z = P.atm[a * ATM_SLOTS + CHARGE_OF];
+        if (z == 0) continue;
+        const double* r = P.env.data() + P.atm[a * ATM_SLOTS + PTR_COORD];
+        nuc.insert(nuc.end(), {r[0], r[1], r[2], (double)z, (double)m, (double)a});
+      }
+    P.nnuc = (int)(nuc.size() / 6);
+    if (nuc.empty()) nuc.assign(6, -1.0);
+    o_nuclei = up.add(nuc);
+  }
+  C2sTables maps = c2s_maps(P);
+  const size_t o_cidx = up.add(maps.cidx), o_ccoef = up.add(maps.ccoef), o_sidx = up.add(maps.sidx),
+               o_scoef = up.add(maps.scoef), o_terms = up.add(function_terms(P.cart, P.nfun));
+  up.send(s);
+  P.d_tables = up.release();
+  auto dev = [&](size_t off) { return P.d_tables + off; };
+  P.d_shells = (ShellXYZ*)dev(o_shells);
+  P.d_prims = (PrimPair*)dev(o_prims);
+  P.d_aux = (PrimAux*)dev(o_aux);
+  P.d_all_pairs = (Pair*)dev(o_all_pairs);
+  P.d_seg_prim0 = (int*)dev(o_seg_prim0);
+  P.d_prim_slots = (int2*)dev(o_slots);
+  P.d_prim_fsp = (double*)dev(o_fsp);
+  P.d_seg_atom = (int*)dev(o_seg_atom);
+  P.d_seg_ao = (int*)dev(o_seg_ao);
+  P.d_pairs1e = (Pair*)dev(o_p1e);
+  P.d_nuclei = (double*)dev(o_nuclei);
+  P.d_c2s_idx = (int*)dev(o_cidx);
+  P.d_c2s_coef = (double*)dev(o_ccoef);
+  P.d_s2c_idx = (int*)dev(o_sidx);
+  P.d_s2c_coef = (double*)dev(o_scoef);
+  P.d_terms = (SphTerm*)dev(o_terms);
+  // Schwarz bounds (parent-shell maxima, as the reference defines them per shell pair)
   std::vector<double>& q = P.seg_pair_q;
   q.assign(npair, 1.0);
   P.qmax_mol.assign(P.nmol, 0.0);
@@ -2083,21 +2263,12 @@ static void build_plan(PlanData& P, double cutoff, hipStream_t s) {
     const int m = P.seg[P.all_pairs[i].sa].mol;
     P.qmax_mol[m] = std::max(P.qmax_mol[m], q[i]);
   }
-  {
-    std::vector<int> at;
-    for (const Seg& g : P.seg) at.push_back(P.bas[g.parent * BAS_SLOTS + ATOM_OF]);
-    P.d_seg_atom = dev_upload(at, s);
-    std::vector<int> ao;
-    for (const Seg& g : P.seg)
-      ao.push_back(P.ao[g.parent] - P.mols[g.mol].ao0 + g.ctr * (P.cart ? ncart_h(g.l) : 2 * g.l + 1));
-    P.d_seg_ao = dev_upload(ao, s);
-  }
   // J/K pair set: parent shells with their general-contraction columns where
   // the basis has them (and the exchange slabs fit), segmented shells otherwise
   bool done = false;
   if (P.options.general_contraction && contracted_eligible(P)) done = build_contracted_set(P, s);
   if (!done) build_segmented_set(P, P.jk, true, s);
-  assign_streams(P);
+  make_streams(P);
   // molecule tables (the density-maximum blocks follow the J/K shell set)
   {
     std::vector<MolInfo> mi(P.nmol);
@@ -2117,36 +2288,16 @@ static void build_plan(PlanData& P, double cutoff, hipStream_t s) {
       mi[m].ns = P.mols[m].n;
       mi[m].pad = 0;
     }
-    P.d_molinfo = dev_upload(mi, s);
-    P.d_molao = dev_upload(P.mols, s);
-    HIP_OK(hipMalloc(&P.d_dmax, sizeof(double) * std::max<int64_t>(P.nd_tot, 1)));
+    Upload mol;
+    const size_t o_info = mol.add(mi), o_ao = mol.add(P.mols),
+                 o_dmax = mol.add(std::vector<double>((size_t)std::max<int64_t>(P.nd_tot, 1), 0.0));
+    mol.send(s);
+    P.d_mol_tables = mol.release();
+    P.d_molinfo = (MolInfo*)(P.d_mol_tables + o_info);
+    P.d_molao = (MolAO*)(P.d_mol_tables + o_ao);
+    P.d_dmax = (double*)(P.d_mol_tables + o_dmax);
   }
   if (P.options.deterministic) build_det_tables(P, s);
-  build_c2s_maps(P, s);
-  {
-    std::vector<int> order(npair);
-    for (int i = 0; i < npair; ++i) order[i] = i;
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return P.all_class[x] < P.all_class[y]; });
-    std::vector<Pair> p1e;
-    int k = 0;
-    for (int c = 0; c < kNumPairClasses; ++c) {
-      P.p1e_begin[c] = k;
-      while (k < npair && P.all_class[order[k]] == c) p1e.push_back(P.all_pairs[order[k++]]);
-    }
-    P.p1e_begin[kNumPairClasses] = k;
-    P.d_pairs1e = dev_upload(p1e, s);
-    std::vector<double> nuc;
-    for (int m = 0; m < P.nmol; ++m)
-      for (int a = P.mol_atm[m]; a < P.mol_atm[m + 1]; ++a) {
-        const int z = P.atm[a * ATM_SLOTS + CHARGE_OF];
-        if (z == 0) continue;
-        const double* r = P.env.data() + P.atm[a * ATM_SLOTS + PTR_COORD];
-        nuc.insert(nuc.end(), {r[0], r[1], r[2], (double)z, (double)m, (double)a});
-      }
-    P.nnuc = (int)(nuc.size() / 6);
-    if (nuc.empty()) nuc.assign(6, -1.0);
-    P.d_nuclei = dev_upload(nuc, s);
-  }
   HIP_OK(hipMalloc(&P.d_flag, sizeof(int)));
   HIP_OK(hipHostMalloc(&P.h_flag, sizeof(int)));
   HIP_OK(hipStreamSynchronize(s));
@@ -2238,21 +2389,16 @@ static void free_plan(PlanData& P) {
   };
   free_pair_set(P.jk);
   free_pair_set(P.seg_set);
-  f(P.d_shells); f(P.d_prims); f(P.d_all_pairs);
-  f(P.d_c2s_idx); f(P.d_c2s_coef); f(P.d_s2c_idx); f(P.d_s2c_coef);
+  f(P.d_tables); f(P.d_mol_tables);
   f(P.d_dc); f(P.d_jp); f(P.d_jpad); f(P.d_kp); f(P.d_flag); f(P.d_incore); f(P.d_part);
-  f(P.d_pairs1e); f(P.d_nuclei);
-  f(P.d_dmax); f(P.d_seg_atom); f(P.d_seg_ao);
   f(P.d_det_qblk); f(P.d_det_mol); f(P.d_det_scale);
-  f(P.d_molinfo); f(P.d_molao);
-  f(P.d_aux); f(P.d_seg_prim0); f(P.d_prim_slots); f(P.d_prim_fsp); f(P.d_gparam);
+  f(P.d_gparam);
   for (double* p : P.retired) f(p);
   for (hipEvent_t e : P.ev_pool) (void)hipEventDestroy(e);
   for (hipEvent_t e : P.join_ev) (void)hipEventDestroy(e);
   if (P.fork_ev) (void)hipEventDestroy(P.fork_ev);
   for (hipStream_t st : P.side) (void)hipStreamDestroy(st);
-  for (int64_t* p : P.d_lane_krp) f(p);
-  for (int64_t* p : P.d_lane_kent) f(p);
+  f(P.d_lane_tables);
   if (P.h_flag) (void)hipHostFree(P.h_flag);
 }
 
@@ -2585,7 +2731,10 @@ static void jk_build(PlanData& P, const double* density, int nb, double* out, in
 // is the identity per molecule (the kernels' work does not depend on the
 // density's values).
 static void balance_lanes(PlanData& P, hipStream_t s) {
-  if (P.side.empty() || !P.options.balance || P.jk.classes.empty()) return;
+  if (P.side.empty() || !P.options.balance || P.jk.classes.empty()) {
+    assign_lanes(P);
+    return;
+  }
   const size_t nn = (size_t)P.nn_tot;
   std::vector<double> eye(nn, 0.0);
   for (int m = 0; m < P.nmol; ++m)
@@ -3084,55 +3233,6 @@ __global__ void mirror_kernel(double* __restrict__ m, int nb, int n) {
   if (i >= nn * nb) return;
   const int r = (int)(i % nn / n), c = (int)(i % n);
   if (c > r) m[i] = m[i - (size_t)r * n - c + (size_t)c * n + r];
-}
-
-// Host tables uploaded as one buffer: parts are appended 16-byte aligned and
-// addressed by their offset once the buffer is on the device.
-struct Upload {
-  std::vector<char> host;
-  char* dev = nullptr;
-  template <class T>
-  size_t add(const std::vector<T>& v) {
-    const size_t at = (host.size() + 15) & ~(size_t)15;
-    host.resize(at + std::max<size_t>(1, v.size()) * sizeof(T));
-    if (!v.empty()) std::memcpy(host.data() + at, v.data(), v.size() * sizeof(T));
-    return at;
-  }
-  void send(hipStream_t s) {
-    HIP_OK(hipMalloc(&dev, host.size()));
-    HIP_OK(hipMemcpyAsync(dev, host.data(), host.size(), hipMemcpyHostToDevice, s));
-  }
-  template <class T>
-  const T* at(size_t off) const { return reinterpret_cast<const T*>(dev + off); }
-  ~Upload() {
-    if (dev) (void)hipFree(dev);
-  }
-};
-
-// Requested-basis functions of every l as terms of its Cartesian components;
-// nfun[l]: their number.
-static std::vector<SphTerm> function_terms(int cart, int (&nfun)[kDfMaxL + 1]) {
-  std::vector<SphTerm> terms((kDfMaxL + 1) * kDfMaxFun, SphTerm{});
-  for (int l = 0; l <= kDfMaxL; ++l) {
-    std::vector<std::vector<double>> rows;
-    if (cart) {
-      rows.assign(ncart_h(l), std::vector<double>(ncart_h(l), 0.0));
-      for (int k = 0; k < ncart_h(l); ++k) rows[k][k] = 1.0;
-    } else {
-      c2s_rows(l, rows);
-    }
-    nfun[l] = (int)rows.size();
-    for (size_t r = 0; r < rows.size(); ++r) {
-      SphTerm& t = terms[l * kDfMaxFun + r];
-      for (int k = 0; k < ncart_h(l); ++k) {
-        if (rows[r][k] == 0.0) continue;
-        if (t.n == kDfMaxTerms) throw Internal("solid harmonic with more Cartesian terms than the map holds");
-        t.idx[t.n] = k;
-        t.c[t.n++] = rows[r][k];
-      }
-    }
-  }
-  return terms;
 }
 
 // Segmented shells with their first AO in the requested basis, counted from
@@ -3670,6 +3770,7 @@ int gscf_direct_jk(const int32_t* atm, int32_t natm, const int32_t* bas, int32_t
       validate_tables(p.d, atm, natm, bas, nbas, env, nenv, cart);
       if (n != p.d.n || nb < 1) throw InvalidArgument("Direct J/K shape mismatch");
       build_plan(p.d, cutoff, (hipStream_t)stream);
+      assign_lanes(p.d);
       jk_build(p.d, density, nb, out, with_j, with_k, 0u, 0.0, (hipStream_t)stream);
       HIP_OK(hipStreamSynchronize((hipStream_t)stream));
     } catch (...) {

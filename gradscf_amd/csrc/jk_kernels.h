@@ -1401,6 +1401,71 @@ __device__ __forceinline__ void block_to_lds(const PrimPair* __restrict__ prims,
   }
 }
 
+// Schwarz bounds: T pairs per workgroup, their blocks (pq|pq) in LDS, the
+// largest magnitudes by LDS maxima.  A pair of contracted s shells has up to
+// 4096 primitive quartets, a chain of 1.5 ms on one lane ((H2O)16 cc-pVDZ);
+// S = Sb * Sk lanes share them.
+template <int LA, int LB>
+__global__ __launch_bounds__(256) void schwarz_kernel(SchwarzArgs a, int S, int Sk, int T) {
+  using K = Class<LA, LB, LA, LB>;
+  extern __shared__ double ebuf[];
+  constexpr int NB = K::NBRA;
+  unsigned long long* top = reinterpret_cast<unsigned long long*>(ebuf + T * NB * NB);  // [T][2]
+  const int lanes = K::SPLIT * S;
+  const int local = threadIdx.x / lanes;
+  const int64_t t0 = (int64_t)blockIdx.x * T;
+  for (int i = threadIdx.x; i < 2 * T; i += blockDim.x) top[i] = 0ull;
+  if (local < T && t0 + local < a.npairs) {
+    const Pair p = a.pairs[t0 + local];
+    block_to_lds<LA, LB, LA, LB>(a.prims, a.shells, p, p, S, Sk, threadIdx.x & (S - 1), (threadIdx.x / S) % K::SPLIT,
+                                 ebuf + local * NB * NB);
+  }
+  __syncthreads();
+  const SphTerm* __restrict__ ta = a.terms + LA * kDfMaxFun;
+  const SphTerm* __restrict__ tb = a.terms + LB * kDfMaxFun;
+  const int fa = a.nfun[LA], fb = a.nfun[LB];
+  // (magnitudes as bit patterns: non-negative doubles order as integers; a
+  // NaN is left out)
+  auto largest = [&](unsigned long long* m, double v) {
+    v = fabs(v);
+    if (v == v) atomicMax(m, (unsigned long long)__double_as_longlong(v));
+  };
+  for (int e = threadIdx.x; e < T * NB; e += blockDim.x)
+    if (t0 + e / NB < a.npairs) largest(top + 2 * (e / NB) + 1, ebuf[(e / NB) * NB * NB + (e % NB) * (NB + 1)]);
+  for (int e = threadIdx.x; e < T * fa * fb; e += blockDim.x) {
+    const int tl = e / (fa * fb), p = e % (fa * fb) / fb, q = e % fb;
+    if (t0 + tl >= a.npairs) break;
+    const double* __restrict__ blk = ebuf + tl * NB * NB;
+    double v = 0.0;
+    for (int i = 0; i < ta[p].n; ++i)
+      for (int j = 0; j < tb[q].n; ++j) {
+        const double* __restrict__ row = blk + (ta[p].idx[i] * K::NB + tb[q].idx[j]) * NB;
+        const double fij = ta[p].c[i] * tb[q].c[j];
+        for (int k = 0; k < ta[p].n; ++k)
+          for (int l = 0; l < tb[q].n; ++l)
+            v += fij * ta[p].c[k] * tb[q].c[l] * row[ta[p].idx[k] * K::NB + tb[q].idx[l]];
+      }
+    largest(top + 2 * tl, v);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < 2 * T; i += blockDim.x)
+    if (t0 + i / 2 < a.npairs) a.q[2 * t0 + i] = __longlong_as_double((long long)top[i]);
+}
+
+template <int LA, int LB>
+void launch_schwarz_t(const SchwarzArgs& a, int np, hipStream_t s) {
+  using K = Class<LA, LB, LA, LB>;
+  // bra and ket hold the same pair: the split is a square as far as the
+  // workgroup holds it
+  int Sb = 1, Sk = 1;
+  while (Sb * Sk < 64 && K::SPLIT * Sb * Sk < 128 && Sk < np) (Sb == Sk ? Sb : Sk) *= 2;
+  const size_t blk = sizeof(double) * K::NBRA * K::NBRA;
+  int T = 256 / (K::SPLIT * Sb * Sk);
+  while (T > 1 && T * blk > 48 * 1024) --T;
+  hipLaunchKernelGGL((schwarz_kernel<LA, LB>), dim3((unsigned)((a.npairs + T - 1) / T)), dim3(256),
+                     T * (blk + 2 * sizeof(double)), s, a, Sb * Sk, Sk, T);
+}
+
 // Largest r with r (r + 1) / 2 <= idx.
 __device__ __forceinline__ int64_t tri_row(int64_t idx) {
   int64_t r = (int64_t)((sqrt(8.0 * (double)idx + 1.0) - 1.0) * 0.5);
