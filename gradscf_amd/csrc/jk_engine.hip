@@ -264,7 +264,7 @@ struct QuartetClass {
   size_t per_slot = 0;      // LDS bytes of one bra slot for one density
   int row_len = 0;          // LDS exchange-row length (columns of the ket mask, widest molecule)
   int64_t nq = 0, nitems = 0;
-  double cost = 0.0;        // estimated work, for spreading launches over streams
+  double cost = 0.0;        // predicted or measured microseconds, for spreading launches over streams
   std::vector<SubTask> tasks;
   SubTask* d_tasks = nullptr;
   int2* d_quartets = nullptr;
@@ -623,12 +623,24 @@ __device__ __forceinline__ int find_mol(const MolAO* __restrict__ M, int nmol, i
 
 // Dc[b][P][Q] = sum T[p,P] T[q,Q] D[src b][p][q] (or D^T when transpose), per
 // molecule; the maps hold molecule-local indices at global AO positions.
+// With jp, the element's J and K accumulators are cleared in the same pass
+// (and its line of the padded ket-side J for the first npad densities).
 __global__ void dens_to_cart_kernel(const double* __restrict__ D, int64_t nn_tot, int nb, double* __restrict__ Dc,
                                     int64_t ncc_tot, const MolAO* __restrict__ M, int nmol,
-                                    const int* __restrict__ idx, const double* __restrict__ coef, int nbd) {
+                                    const int* __restrict__ idx, const double* __restrict__ coef, int nbd,
+                                    double* __restrict__ jp = nullptr, double* __restrict__ kp = nullptr,
+                                    double* __restrict__ jpad = nullptr, int npad = 0) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const size_t total = (size_t)nbd * ncc_tot;
   if (i >= total) return;
+  if (jp) {
+    jp[i] = 0.0;
+    kp[i] = 0.0;
+    if (i < (size_t)npad * ncc_tot) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) jpad[8 * i + k] = 0.0;
+    }
+  }
   const int bt = (int)(i / ncc_tot);
   const int64_t r = (int64_t)(i - (size_t)bt * ncc_tot);
   const MolAO m = M[find_mol(M, nmol, r, 1)];
@@ -663,38 +675,49 @@ __global__ void dens_to_cart_kernel(const double* __restrict__ D, int64_t nn_tot
 // reads eight slab rows per step so that many loads are in flight.
 // row_dst[R] / row_n[R] / row_mol[R]: first element, length and molecule of
 // row R of K.
-__global__ __launch_bounds__(64) void kpart_reduce_kernel(const double* __restrict__ part, int64_t stride,
-                                                          const int64_t* __restrict__ rp,
-                                                          const int64_t* __restrict__ ent,
-                                                          const int64_t* __restrict__ row_dst,
-                                                          const int* __restrict__ row_n,
-                                                          const int* __restrict__ row_mol,
-                                                          const int64_t* __restrict__ cinv_off,
-                                                          const int* __restrict__ cinv, int64_t ncc_tot,
-                                                          int atomic, double* __restrict__ kp) {
+// The wavefronts of a workgroup share the row's slab list (eight entries each
+// in turn) and add up in LDS: with one wavefront per row and column block the
+// list was a serial chain of dependent reads that outlasted the class kernels
+// of small molecules (in-core builds of (H2O)8: 650 us with one, 615 us with
+// four; 8 and 16 cost batches of small molecules 3-5 %, whose lists are short).
+constexpr int kPartReduceWaves = 4;
+__global__ __launch_bounds__(64 * kPartReduceWaves) void kpart_reduce_kernel(const double* __restrict__ part, int64_t stride,
+                                                            const int64_t* __restrict__ rp,
+                                                            const int64_t* __restrict__ ent,
+                                                            const int64_t* __restrict__ row_dst,
+                                                            const int* __restrict__ row_n,
+                                                            const int* __restrict__ row_mol,
+                                                            const int64_t* __restrict__ cinv_off,
+                                                            const int* __restrict__ cinv, int64_t ncc_tot,
+                                                            int atomic, double* __restrict__ kp) {
+  __shared__ double sums[kPartReduceWaves][64];
   const int64_t R = blockIdx.x;
   const int bt = blockIdx.z;
-  const int col = blockIdx.y * 64 + threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = kPartReduceWaves;
+  const int col = blockIdx.y * 64 + lane;
   const int n = row_n[R];
-  if (col >= n) return;
   const int m = row_mol[R];
   const double* __restrict__ pb = part + (size_t)bt * stride;
   double v[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   bool any = false;
-  for (int mask = 1; mask < 8; ++mask) {
+  for (int mask = 1; col < n && mask < 8; ++mask) {
     const int64_t e0 = rp[R * 8 + mask], e1 = rp[R * 8 + mask + 1];
     if (e0 == e1) continue;
     const int j = cinv[cinv_off[m * 8 + mask] + col];
     if (j < 0) continue;
     any = true;
-    int64_t e = e0;
-    for (; e + 8 <= e1; e += 8) {
+    int64_t e = e0 + 8 * wave;
+    for (; e + 8 <= e1; e += 8 * nw) {
 #pragma unroll
       for (int u = 0; u < 8; ++u) v[u] += pb[ent[e + u] + j];
     }
     for (int u = 0; e < e1; ++e, ++u) v[u] += pb[ent[e] + j];
   }
-  const double sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+  double sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+  sums[wave][lane] = sum;
+  __syncthreads();
+  if (wave != 0 || col >= n) return;
+  for (int w = 1; w < nw; ++w) sum += sums[w][lane];
   double* dst = kp + (size_t)bt * ncc_tot + row_dst[R] + col;
   if (!atomic) {
     *dst += sum;
@@ -1326,6 +1349,27 @@ constexpr int64_t kFillLanes = 32768;
 constexpr int64_t kFillGroups = 256;
 constexpr int64_t kMinPrim = 2;
 
+// Predicted microseconds that nq quartets of a class with npq primitive
+// quartets each add to its launch, and of a launch by itself: ps per quartet
+// and per primitive quartet of every class, fitted (non-negative, relative
+// error) to the class times of 14 plans between H2O and C20H42 / (H2O)24 in
+// 6-31G*, cc-pVDZ, 6-31G and STO-3G.  Spreading the classes over four streams
+// by these times leaves the longest stream within 1-10 % of the best spread
+// by measured times for 13 of them (C8H18: 33 %); a model of primitive quartets times
+// block size left it 30-80 % longer.  A contracted pattern's block is
+// (columns) times larger; its classes are taken at that multiple.
+constexpr double kLaunchUs = 20.0;
+static double class_cost_us(int la, int lb, int lc, int ld, int pb, int pk, int64_t nq, double npq) {
+  static const double ps[kNumQuartetClasses][2] = {
+      {52, 4.2},    {32, 5.8},    {204, 7.8},   {0, 20},      {244, 9.1},   {1513, 554},  {0, 18},
+      {278, 0},     {2134, 0},    {402, 32},    {0, 28},      {621, 35},    {1318, 326},  {1251, 0},
+      {2391, 842},  {2, 77},      {804, 15},    {1638, 458},  {1270, 68},   {2357, 2022}, {0, 7757}};
+  const int cb = pair_class(la, lb), ck = pair_class(lc, ld);
+  const double* p = ps[cb * (cb + 1) / 2 + ck];
+  const double cols = (double)(1 + (pb & 1)) * (1 + (pb >> 1)) * (1 + (pk & 1)) * (1 + (pk >> 1));
+  return 1e-6 * cols * (double)nq * (p[0] + p[1] * npq);
+}
+
 // Primitive split S = Sb * Sk (powers of two, S <= 64: the bra-major kernel
 // sums the S slices of a quartet across adjacent lanes) of a sub-task whose
 // bras and kets have np in [npb0, npb1] and [npk0, npk1]: the largest S that
@@ -1521,14 +1565,8 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
               t.nq = nq;
               t.S = t.Sk = 1;
               t.item0 = 0;
-              {
-                // rough work model: primitive quartets weighted by the class's
-                // Cartesian block size, plus a per-quartet digestion term
-                const double nblk = (double)ncart_h(qc.la) * ncart_h(qc.lb) * ncart_h(qc.lc) * ncart_h(qc.ld);
-                const double cols = (double)(1 + (pb & 1)) * (1 + (pb >> 1)) * (1 + (pk & 1)) * (1 + (pk >> 1));
-                const double npq = 0.25 * (double)(rb.npmin + rb.npmax) * (rk.npmin + rk.npmax);
-                qc.cost += (double)nq * (npq * (8.0 + 0.5 * nblk + 0.25 * nblk * (cols - 1.0)) + 4.0 * nblk * cols + 64.0);
-              }
+              qc.cost += class_cost_us(qc.la, qc.lb, qc.lc, qc.ld, pb, pk, nq,
+                                       0.25 * (double)(rb.npmin + rb.npmax) * (rk.npmin + rk.npmax));
               qc.nq += nq;
               qc.tasks.push_back(t);
               pend.push_back({std::move(qoff), rb.beg, rk.beg, nbra, t.q0, nq, rki, std::numeric_limits<int>::max(), rbi});
@@ -1722,6 +1760,7 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
             chunks.insert(chunks.end(), qc.chunks.begin(), qc.chunks.end());
           }
           subtasks.insert(subtasks.end(), qc.tasks.begin(), qc.tasks.end());
+          qc.cost += kLaunchUs;
           S.nquartets += qc.nq;
           S.classes.push_back(std::move(qc));
         }
@@ -2036,9 +2075,22 @@ static void assign_lanes(PlanData& P) {
   }
 }
 
+// Predicted time of one build's class launches one after another.
+static double predicted_us(const PlanData& P) {
+  double t = 0.0;
+  for (const QuartetClass& qc : P.jk.classes) t += qc.cost;
+  return t;
+}
+
 // Side streams and fork/join events of the class launches.
 static void make_streams(PlanData& P) {
-  const int ns = std::max(1, std::min<int>(kMaxStreams, P.options.streams));
+  // A further stream pays where it takes work off the others for longer than
+  // the host needs to fork and join it (about 10 us each): water / 6-31G (six
+  // classes, 120 us of launches one after another) takes 96 us a build on two
+  // streams, 123 us on four and 127 us on one; H2O / cc-pVDZ (21 classes)
+  // 197 us on four and 247 us on two.
+  constexpr double kStreamUs = 60.0;
+  const int ns = std::max(1, std::min({kMaxStreams, (int)P.options.streams, (int)(predicted_us(P) / kStreamUs)}));
   for (int l = 1; l < ns; ++l) {
     hipStream_t st;
     HIP_OK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
@@ -2478,17 +2530,14 @@ static void jk_build(PlanData& P, const double* density, int nb, double* out, in
     W = {P.d_dc, P.d_jp, P.d_jpad, P.d_kp, P.d_part};
   }
   hipLaunchKernelGGL(dens_to_cart_kernel, dim3(nblocks(ncc * nbd)), dim3(256), 0, s, density, P.nn_tot, nb, W.dc,
-                     P.ncc_tot, P.d_molao, P.nmol, P.d_c2s_idx, P.d_c2s_coef, nbd);
+                     P.ncc_tot, P.d_molao, P.nmol, P.d_c2s_idx, P.d_c2s_coef, nbd, W.jp, W.kp, W.jpad,
+                     with_j ? nb : 0);
   if (mixed || det)
     hipLaunchKernelGGL(dmax_kernel, dim3(nblocks((size_t)P.nd_tot)), dim3(256), 0, s, W.dc, P.ncc_tot, nbd,
                        P.d_molao, P.nmol, P.nd_tot, P.jk.d_blk, P.d_dmax);
   if (det)
     hipLaunchKernelGGL(det_scale_kernel, dim3((unsigned)P.nmol), dim3(256), 0, s, P.d_dmax, P.d_det_qblk,
                        P.d_molao, P.d_det_mol, P.d_det_scale);
-  hipLaunchKernelGGL(fill_kernel, dim3(nblocks(ncc * nbd)), dim3(256), 0, s, W.jp, ncc * nbd, 0.0);
-  if (with_j)
-    hipLaunchKernelGGL(fill_kernel, dim3(nblocks(8 * ncc * nb)), dim3(256), 0, s, W.jpad, 8 * ncc * nb, 0.0);
-  hipLaunchKernelGGL(fill_kernel, dim3(nblocks(ncc * nbd)), dim3(256), 0, s, W.kp, ncc * nbd, 0.0);
   const PairSet& S = P.jk;
   if (P.prof) ++P.prof_builds;
   // Class launches: in list order on the caller's stream while profiling (so
@@ -2685,7 +2734,7 @@ static void jk_build(PlanData& P, const double* density, int nb, double* out, in
   if (lane_reduce)
     for (size_t l = 0; l < P.lane_classes.size(); ++l)
       hipLaunchKernelGGL(kpart_reduce_kernel, dim3((unsigned)S.nrows, (unsigned)((S.nc_max + 63) / 64),
-                         (unsigned)nbd), dim3(64), 0, l == 0 ? s : P.side[l - 1], W.part, S.part_total,
+                         (unsigned)nbd), dim3(64 * kPartReduceWaves), 0, l == 0 ? s : P.side[l - 1], W.part, S.part_total,
                          P.d_lane_krp[l], P.d_lane_kent[l], S.d_row_dst, S.d_row_n, S.d_row_mol, S.d_cinv_off,
                          S.d_cinv, P.ncc_tot, 1, W.kp);
   if (fork) {
@@ -2698,7 +2747,7 @@ static void jk_build(PlanData& P, const double* density, int nb, double* out, in
     const int nbd_k = with_k ? nbd : nb;
     if (with_k && (psums & 1) && !lane_reduce)
       hipLaunchKernelGGL(kpart_reduce_kernel, dim3((unsigned)S.nrows, (unsigned)((S.nc_max + 63) / 64),
-                         (unsigned)nbd_k), dim3(64), 0, s, W.part, S.part_total, S.d_krp, S.d_kent,
+                         (unsigned)nbd_k), dim3(64 * kPartReduceWaves), 0, s, W.part, S.part_total, S.d_krp, S.d_kent,
                          S.d_row_dst, S.d_row_n, S.d_row_mol, S.d_cinv_off, S.d_cinv, P.ncc_tot, 0, W.kp);
     if (with_j && (psums & 2))
       hipLaunchKernelGGL(jpart_reduce_kernel, dim3((unsigned)S.pairs.size(), (unsigned)nb), dim3(64), 0, s,
@@ -2731,7 +2780,11 @@ static void jk_build(PlanData& P, const double* density, int nb, double* out, in
 // is the identity per molecule (the kernels' work does not depend on the
 // density's values).
 static void balance_lanes(PlanData& P, hipStream_t s) {
-  if (P.side.empty() || !P.options.balance || P.jk.classes.empty()) {
+  // Short builds keep the predicted times: two probe builds and their events
+  // take about 1.5 ms, which a spread 5-10 % better repays only over dozens of
+  // builds ((H2O)3 6-31G*, plan and one build: 3.0 ms with probes, 1.4 without).
+  constexpr double kProbeUs = 1000.0;
+  if (P.side.empty() || !P.options.balance || P.jk.classes.empty() || predicted_us(P) < kProbeUs) {
     assign_lanes(P);
     return;
   }

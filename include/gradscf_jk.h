@@ -100,8 +100,9 @@ int gscf_tuning_reset(void);
 typedef struct {
   int32_t general_contraction; /* 1: two-column s shells (cc-pVXZ 1s/2s) evaluated once per
                                   primitive quartet for both columns; 0 (default): as two segments */
-  int32_t streams;             /* 1..4 HIP streams the class launches of one J/K build are
-                                  spread over (fork/join on the caller's stream; default 4) */
+  int32_t streams;             /* 1..4: HIP streams the class launches of one J/K build are
+                                  spread over at most (fork/join on the caller's stream;
+                                  default 4; short builds use fewer) */
   int32_t partial_sums;        /* bit 0: a workgroup hands its exchange rows, bit 1 its ket-side
                                   J window, to a reduction pass as plain stores into per-build
                                   slabs instead of device-scope atomics (0..3; default 1) */
@@ -118,8 +119,10 @@ typedef struct {
                                   0 (default): FP64 atomics, equal to rounding */
   int32_t balance;             /* 1 (default): plan creation times every quartet class of one
                                   build alone (two builds of an identity density, HIP events)
-                                  and spreads the classes over the streams by those times;
-                                  0: by the plan-time work model (no probe builds) */
+                                  and spreads the classes over the streams by those times,
+                                  where the plan-time work model predicts class launches of
+                                  over 1 ms; shorter builds, and 0: by the model (no probe
+                                  builds) */
 } gscf_options;
 int gscf_options_set(const gscf_options* o);
 int gscf_options_get(gscf_options* o);
