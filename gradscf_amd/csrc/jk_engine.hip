@@ -2933,6 +2933,33 @@ static void int1e_gradient(PlanData& P, const double* dens, const double* wdens,
   HIP_OK(hipGetLastError());
 }
 
+// One launch per class of S, spread over the caller's stream and the plan's
+// side streams by the classes' predicted or measured times, longest first.
+// The derivative kernels are independent (device-scope adds into their
+// result), and one after another their tails left most of the chip idle.
+template <class F>
+static void for_classes_on_streams(PlanData& P, const PairSet& S, hipStream_t s, F&& launch) {
+  const int ns = (int)P.side.size() + 1;
+  std::vector<int> order(S.classes.size());
+  for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
+  std::stable_sort(order.begin(), order.end(),
+                   [&](int x, int y) { return S.classes[x].cost > S.classes[y].cost; });
+  if (ns > 1) {
+    HIP_OK(hipEventRecord(P.fork_ev, s));
+    for (hipStream_t st : P.side) HIP_OK(hipStreamWaitEvent(st, P.fork_ev, 0));
+  }
+  std::vector<double> load(ns, 0.0);
+  for (int ci : order) {
+    const int l = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+    load[l] += S.classes[ci].cost;
+    launch(S.classes[ci], l == 0 ? s : P.side[l - 1]);
+  }
+  for (size_t l = 0; l < P.side.size(); ++l) {
+    HIP_OK(hipEventRecord(P.join_ev[l], P.side[l]));
+    HIP_OK(hipStreamWaitEvent(s, P.join_ev[l], 0));
+  }
+}
+
 static void geometry_vjp(PlanData& P, const double* dens, const double* cj, const double* ck, double* grad,
                          hipStream_t s) {
   if (P.cutoff > 0) throw InvalidArgument("Screened direct J/K geometry AD requires cutoff=0");
@@ -2945,7 +2972,8 @@ static void geometry_vjp(PlanData& P, const double* dens, const double* cj, cons
       hipLaunchKernelGGL(dens_to_cart_kernel, dim3(nblocks(ncc)), dim3(256), 0, s, src[k], P.nn_tot, 1,
                          P.d_dc + k * ncc, P.ncc_tot, P.d_molao, P.nmol, P.d_c2s_idx, P.d_c2s_coef, 1);
   const PairSet& S = ensure_seg_set(P, s);
-  for (const QuartetClass& qc : S.classes) {
+  if ((size_t)3 * P.natm * sizeof(double) > kLdsBudget) throw InvalidArgument("too many atoms for the gradient kernel");
+  for_classes_on_streams(P, S, s, [&](const QuartetClass& qc, hipStream_t s) {
     GradArgs a;
     a.pairs = S.d_pairs;
     a.prims = P.d_prims;
@@ -2961,9 +2989,8 @@ static void geometry_vjp(PlanData& P, const double* dens, const double* cj, cons
     a.mols = P.d_molinfo;
     a.natm = P.natm;
     a.grad = grad;
-    if ((size_t)3 * P.natm * sizeof(double) > kLdsBudget) throw InvalidArgument("too many atoms for the gradient kernel");
     launch_grad_class(qc.la, qc.lb, qc.lc, qc.ld, a, s);
-  }
+  });
   HIP_OK(hipGetLastError());
 }
 
@@ -2988,7 +3015,7 @@ static void jk_param_vjp(PlanData& P, const double* dens, const double* cj, cons
       hipLaunchKernelGGL(dens_to_cart_kernel, dim3(nblocks(ncc)), dim3(256), 0, s, src[k], P.nn_tot, 1,
                          P.d_dc + k * ncc, P.ncc_tot, P.d_molao, P.nmol, P.d_c2s_idx, P.d_c2s_coef, 1);
   const PairSet& S = ensure_seg_set(P, s);
-  for (const QuartetClass& qc : S.classes) {
+  for_classes_on_streams(P, S, s, [&](const QuartetClass& qc, hipStream_t s) {
     ParamArgs a;
     a.pairs = S.d_pairs;
     a.prims = P.d_prims;
@@ -3007,7 +3034,7 @@ static void jk_param_vjp(PlanData& P, const double* dens, const double* cj, cons
     a.gcoef = P.d_gparam;
     a.gexp = P.d_gparam + nprim;
     launch_param_class(qc.la, qc.lb, qc.lc, qc.ld, a, s);
-  }
+  });
   hipLaunchKernelGGL(param_to_env_kernel, dim3(nblocks((size_t)nprim)), dim3(256), 0, s, nprim, P.d_prim_slots,
                      P.d_prim_fsp, P.d_gparam, P.d_gparam + nprim, env_grad);
   HIP_OK(hipGetLastError());
