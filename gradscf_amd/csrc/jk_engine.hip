@@ -287,6 +287,17 @@ struct QuartetClass {
 constexpr size_t kLdsBudget = 64 * 1024;
 constexpr size_t kLdsDeviceMax = 160 * 1024;
 constexpr size_t kKetLdsBytes = 16 * 1024;  // LDS ket-J window per density
+// Classes of up to this many Rys roots sum the ket-side J of a chunk's kets in
+// LDS whatever the schedule says.  Their quartets cost a few primitive
+// evaluations each, so the one global FP64 atomic per quartet and ket
+// component, executed at the memory side, bounds them: with those atomics
+// taken out, C20H42 / 6-31G* ran (ss|ss) in 223 us instead of 413 and (ps|ps)
+// in 201 instead of 334.  Summed over the bras of a chunk first: 291 and 276
+// us, and whole builds of (H2O)16 / cc-pVDZ 2.95 -> 2.74 ms, C20H42 6.04 ->
+// 5.80 ms, in-core (H2O)8 0.61 -> 0.46 ms.  With three roots and more the
+// quartets hide the atomics ((dp|ps) 312 us with and without) and the window
+// only takes LDS: (H2O)16 2.66 -> 2.78 ms with windows for three roots too.
+constexpr int kWindowRoots = 2;
 // Partial-sum slabs per density at most; a plan whose slabs would be larger
 // flushes with atomics instead.
 constexpr int64_t kPartCapBytes = int64_t(2) << 30;
@@ -1349,6 +1360,17 @@ constexpr int64_t kFillLanes = 32768;
 constexpr int64_t kFillGroups = 256;
 constexpr int64_t kMinPrim = 2;
 
+// Work of one chunk at most, in primitive quartets over all lane-items, with
+// kDigestPrims for the digestion of an item.  A chunk of 4096 items of 48
+// primitive quartets runs for 230 us or more, and a class of few such chunks
+// waits for the last of them on a nearly idle chip.  Together with the order
+// of falling work: 64 clusters of water 5.0 -> 4.65 ms, (H2O)16 2.74 -> 2.70,
+// C20H42 5.88 -> 5.75, two densities of (H2O)7 1.24 -> 1.16 ms a build (order
+// alone 4.71, 2.68, 5.80 and 1.23).  16000 costs more exchange-row flushes
+// than it saves (C20H42 6.74 ms), 64000 gains nothing further.
+constexpr double kChunkWork = 128000.0;
+constexpr double kDigestPrims = 6.0;
+
 // Predicted microseconds that nq quartets of a class with npq primitive
 // quartets each add to its launch, and of a launch by itself: ps per quartet
 // and per primitive quartet of every class, fitted (non-negative, relative
@@ -1597,7 +1619,7 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
             items += (int64_t)t.S * t.nq * split;
           }
           const int64_t fill_items = (items / kFillGroups + tu.threads - 1) / tu.threads * tu.threads;
-          const int64_t kChunkItems =
+          const int64_t class_items =
               std::min<int64_t>(tu.chunk_items, std::max<int64_t>(tu.threads, fill_items));
           if (with_chunks) {
             // bra-major chunks: consecutive bras of one sub-task, bounded LDS slots and lane-items
@@ -1629,6 +1651,7 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
               pack = pack > qc.tab_bytes + per_slot ? pack - qc.tab_bytes : per_slot;
             }
             qc.per_slot = per_slot;
+            std::vector<double> chunk_work;  // primitive quartets of a chunk's longest lane, digestion included
             // a slot wider than the packing budget still gets chunks of one
             // bra when one density's slot fits the device's LDS
             qc.nbra_max = per_slot > P.lds_max ? 0
@@ -1637,6 +1660,14 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
               Pending& pd = pend[ti];
               const SubTask& t = qc.tasks[ti];
               const int64_t per_q = (int64_t)t.S * split;
+              const Run &rb = runs[pd.rb], &rk = runs[pd.rk];
+              const double item_work = 0.25 * (rb.npmin + rb.npmax) * (rk.npmin + rk.npmax) / t.S + kDigestPrims;
+              const int64_t kChunkItems = std::min<int64_t>(
+                  class_items, std::max<int64_t>(tu.threads, (int64_t)(kChunkWork / item_work) / tu.threads * tu.threads));
+              auto add_chunk = [&](const BraChunk& c) {
+                qc.chunks.push_back(c);
+                chunk_work.push_back(item_work * (double)((c.nq * per_q + tu.threads - 1) / tu.threads));
+              };
               // a bra longer than one chunk is cut into windows of step kets;
               // shorter bras fit one window (cnt <= step)
               pd.seg = (int)std::min<int64_t>(std::numeric_limits<int>::max(),
@@ -1658,7 +1689,7 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
                     c.nbra = 1;
                     c.ket0 = pd.ket0 + (int32_t)k0;
                     c.nket = c.nq;
-                    qc.chunks.push_back(c);
+                    add_chunk(c);
                   }
                   ++b;
                   continue;
@@ -1682,7 +1713,7 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
                 c.nket = 0;
                 for (int bb = b; bb < e; ++bb)
                   c.nket = std::max<int32_t>(c.nket, (int32_t)(pd.qoff[bb + 1] - pd.qoff[bb]));
-                qc.chunks.push_back(c);
+                add_chunk(c);
                 b = e;
               }
             }
@@ -1700,16 +1731,24 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
                 for (int j = 0; j < c.nbra; ++j) cap += S.pairs[c.bra0 + j].np;
                 qc.stage_cap = std::max(qc.stage_cap, cap);
               }
-            // ket-side J in LDS for chunks whose ket window fits kKetLdsBytes per density
+            // chunks in order of falling work: the workgroups dispatched last,
+            // which a launch's end waits for, are then the shortest
+            {
+              std::vector<int> ord(qc.chunks.size());
+              for (size_t i = 0; i < ord.size(); ++i) ord[i] = (int)i;
+              std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return chunk_work[x] > chunk_work[y]; });
+              std::vector<BraChunk> sorted(qc.chunks.size());
+              for (size_t i = 0; i < ord.size(); ++i) sorted[i] = qc.chunks[ord[i]];
+              qc.chunks.swap(sorted);
+            }
+            // ket-side J in LDS for chunks of several bras whose ket window
+            // fits kKetLdsBytes per density
             qc.threads = tu.threads;
-            if (tu.ket_lds) {
-              const int cap = (int)(kKetLdsBytes / (sizeof(double) * wc * wd));
-              for (BraChunk& c : qc.chunks) {
-                if (c.nket > cap) c.nket = 0;
-                qc.nket_max = std::max(qc.nket_max, c.nket);
-              }
-            } else {
-              for (BraChunk& c : qc.chunks) c.nket = 0;
+            const bool windows = tu.ket_lds || nr <= kWindowRoots;
+            const int cap = windows ? (int)(kKetLdsBytes / (sizeof(double) * wc * wd)) : 0;
+            for (BraChunk& c : qc.chunks) {
+              if (c.nket > cap || (c.nbra == 1 && !tu.ket_lds)) c.nket = 0;
+              qc.nket_max = std::max(qc.nket_max, c.nket);
             }
             // partial slabs (segmented sets): each chunk's exchange rows
             // [nbra][rows][columns of the class's ket mask], then its ket
@@ -2619,13 +2658,16 @@ static void jk_build(PlanData& P, const double* density, int nb, double* out, in
     auto layout = [&](int nbd_l, int nbj_l, size_t cap, size_t& lds, int& nket_max, int& tab_lds) {
       lds = sizeof(double) * ((size_t)nbd_l * qc.nbra_max * (wa + wb) * b.n +
                               (size_t)nbj_l * qc.nbra_max * wa * wb * kJBraCopies);
-      nket_max = with_j ? qc.nket_max : 0;
-      const size_t jket_bytes = sizeof(double) * (size_t)nbj_l * nket_max * wc * wd;
-      if (nket_max && lds + jket_bytes <= cap) lds += jket_bytes; else nket_max = 0;
       // the slots' bra density blocks D_ab + D_ba of every Coulomb density
       if (with_j) lds += sizeof(double) * (size_t)nbj_l * qc.nbra_max * wa * wb;
       // (the kernel places the staging area 16-byte aligned after the slabs)
-      if (stage_cap) lds = ((lds + 15) & ~(size_t)15) + sizeof(double) * ((size_t)stage_rec * stage_cap + (qc.nbra_max + 2) / 2);
+      const size_t stage = stage_cap ? sizeof(double) * ((size_t)stage_rec * stage_cap + (qc.nbra_max + 2) / 2) : 0;
+      auto staged = [&](size_t slabs) { return stage ? ((slabs + 15) & ~(size_t)15) + stage : slabs; };
+      // the ket window only beside everything a launch needs, so that it
+      // never moves a class to another route
+      const size_t jket_bytes = sizeof(double) * (size_t)nbj_l * qc.nket_max * wc * wd;
+      nket_max = with_j && staged(lds + jket_bytes) <= cap ? qc.nket_max : 0;
+      lds = staged(nket_max ? lds + jket_bytes : lds);
       tab_lds = (b.mode == 2 || det) ? 0 : qc.tab_lds;  // stored blocks need no Rys table
       // (the kernel places the table 16-byte aligned after the staging area)
       const size_t tab_at = (lds + 15) & ~(size_t)15;
