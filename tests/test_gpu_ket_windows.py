@@ -1,7 +1,9 @@
 """Ket-side Coulomb sums in LDS windows: chunks of several bras whose kets fit
 the window, chunks of more kets than it holds, and chunks of one bra (no
 window) give the same bits under integer accumulation, where every quartet adds
-the same rounded terms whatever its chunk, and the oracle's values."""
+the same rounded terms whatever its chunk, and the oracle's values.  The four
+densities of one launch take more than half a CU's LDS (512-thread workgroups)
+except under lds_limit, where each has a launch of its own."""
 import numpy as np
 import pytest
 
