@@ -313,6 +313,7 @@ struct PairSet {
   ShellXYZ* d_shells = nullptr;   // owned only by contracted sets
   PrimPair* d_prims = nullptr;    // owned only by contracted sets
   PrimCoef* d_coef = nullptr;     // contracted sets: column coefficients per primitive pair
+  KetRec* d_kets = nullptr;       // per pair
   int* d_blk = nullptr;           // [nshell][2]: AO offset and width of each shell's density block
   std::vector<Pair> pairs;        // retained, class/pattern/molecule/bucket sorted
   std::vector<double> pair_q;
@@ -805,6 +806,21 @@ __global__ void finalize_kernel(const double* __restrict__ jp, const double* __r
     }
   }
   out[i] = s;
+}
+
+// Ket records of a pair list (cofs: first compact column of every shell per
+// mask of angular momenta, NULL for rows over all columns).
+__global__ __launch_bounds__(256) void ket_records_kernel(const Pair* __restrict__ pairs,
+                                                          const ShellXYZ* __restrict__ shells,
+                                                          const int* __restrict__ cofs, int npairs,
+                                                          KetRec* __restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= npairs) return;
+  const Pair p = pairs[i];
+  const ShellXYZ C = shells[p.sa], D = shells[p.sb];
+  const int mask = (1 << C.l) | (1 << D.l);
+  out[i] = {p.poff, p.np, C.ao, D.ao, cofs ? cofs[p.sa * 8 + mask] : C.ao, cofs ? cofs[p.sb * 8 + mask] : D.ao,
+            C.lseg, D.lseg, {C.x, C.y, C.z}, {C.x - D.x, C.y - D.y, C.z - D.z}};
 }
 
 // Quartet lists of every (bra run, ket run) sub-task of a plan, one launch:
@@ -1642,7 +1658,7 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
             }
             qc.row_len = row_len;
             const size_t per_slot = sizeof(double) * ((size_t)rows * row_len + (size_t)wa * wb * (kJBraCopies + 1) +
-                                                      (size_t)rec * bra_np_max + 1);
+                                                      (size_t)rec * bra_np_max + kBraRecDoubles);
             const int nr = (qc.la + qc.lb + qc.lc + qc.ld) / 2 + 1;
             size_t pack = std::min<size_t>((size_t)tu.lds_pack, P.lds_budget);
             if (tu.rys_lds && per_slot + rys_slice_bytes(nr) <= P.lds_budget) {
@@ -1680,7 +1696,8 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
                   // one long bra: several single-bra chunks
                   const int64_t step = std::max<int64_t>(1, kChunkItems / per_q);
                   for (int64_t k0 = 0; k0 < cnt; k0 += step) {
-                    BraChunk c;
+                    BraChunk c{};
+                    c.mol = rb.mol;
                     c.q0 = t.q0 + pd.qoff[b] + k0;
                     c.nq = (int32_t)std::min<int64_t>(step, cnt - k0);
                     c.S = t.S;
@@ -1694,7 +1711,8 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
                   ++b;
                   continue;
                 }
-                BraChunk c;
+                BraChunk c{};
+                c.mol = rb.mol;
                 c.q0 = t.q0 + pd.qoff[b];
                 c.S = t.S;
                 c.Sk = t.Sk;
@@ -1863,6 +1881,11 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
   }
   S.d_cspace = (int2*)at(o_cspace);
   S.d_cinv_off = (int64_t*)at(o_cinv_off);
+  if (!chunks.empty()) {
+    HIP_OK(hipMalloc(&S.d_kets, sizeof(KetRec) * S.pairs.size()));
+    hipLaunchKernelGGL(ket_records_kernel, dim3(nblocks(S.pairs.size())), dim3(256), 0, s, S.d_pairs, S.d_shells,
+                       S.d_shell_cofs, (int)S.pairs.size(), S.d_kets);
+  }
   if (S.nquartets > 0) {
     HIP_OK(hipMalloc(&S.d_quartets, sizeof(int2) * S.nquartets));
     for (size_t c = 0; c < S.classes.size(); ++c) {
@@ -1899,7 +1922,7 @@ static void free_pair_set(PairSet& S) {
     f(S.d_shells);
     f(S.d_prims);
   }
-  f(S.d_coef); f(S.d_blk); f(S.d_tables); f(S.d_quartets);
+  f(S.d_coef); f(S.d_blk); f(S.d_tables); f(S.d_quartets); f(S.d_kets);
   S = PairSet();
 }
 
@@ -2410,6 +2433,7 @@ static int64_t plan_bytes(const PlanData& P, int64_t npairs, int64_t nq, int64_t
   for (const Seg& g : P.seg) b += (int64_t)g.np * (sizeof(int2) + 3 * sizeof(double));  // slots, fsp, sums
   b += (int64_t)P.all_pairs.size() * 2 * sizeof(Pair);                        // all pairs, 1e pairs
   b += npairs * (sizeof(Pair) + sizeof(double));                              // screened pairs, pair_q
+  b += npairs * sizeof(KetRec);
   b += extra;                                                                 // contracted J/K shells and primitives
   b += (int64_t)P.n_cart * 2 * (sizeof(int) + sizeof(double)) + (int64_t)P.n * 3 * (sizeof(int) + sizeof(double));
   b += (int64_t)P.nmol * sizeof(MolInfo) + (int64_t)(P.nmol + 1) * sizeof(MolAO);
@@ -2640,6 +2664,7 @@ static void jk_build(PlanData& P, const double* density, int nb, double* out, in
       b.cache = P.d_incore + qc.cache_off;
     }
     b.pairs = S.d_pairs;
+    b.kets = S.d_kets;
     b.prims = S.d_prims;
     b.shells = S.d_shells;
     b.coef = S.d_coef;
@@ -2663,12 +2688,12 @@ static void jk_build(PlanData& P, const double* density, int nb, double* out, in
     const int stage_cap = b.mode == 2 ? 0 : qc.stage_cap;
     const int stage_rec = qc.pb ? kStagedPrimCoef : kStagedPrim;
     auto layout = [&](int nbd_l, int nbj_l, size_t cap, size_t& lds, int& nket_max, int& tab_lds) {
-      lds = sizeof(double) * ((size_t)nbd_l * qc.nbra_max * (wa + wb) * b.n +
+      lds = sizeof(double) * ((size_t)kBraRecDoubles * qc.nbra_max + (size_t)nbd_l * qc.nbra_max * (wa + wb) * b.n +
                               (size_t)nbj_l * qc.nbra_max * wa * wb * kJBraCopies);
       // the slots' bra density blocks D_ab + D_ba of every Coulomb density
       if (with_j) lds += sizeof(double) * (size_t)nbj_l * qc.nbra_max * wa * wb;
       // (the kernel places the staging area 16-byte aligned after the slabs)
-      const size_t stage = stage_cap ? sizeof(double) * ((size_t)stage_rec * stage_cap + (qc.nbra_max + 2) / 2) : 0;
+      const size_t stage = stage_cap ? sizeof(double) * (size_t)stage_rec * stage_cap : 0;
       auto staged = [&](size_t slabs) { return stage ? ((slabs + 15) & ~(size_t)15) + stage : slabs; };
       // the ket window only beside everything a launch needs, so that it
       // never moves a class to another route
@@ -2926,6 +2951,7 @@ static void incore_set(PlanData& P, int enable, hipStream_t s) {
     b.mode = 1;
     b.cache = buf + qc.cache_off;
     b.pairs = S.d_pairs;
+    b.kets = S.d_kets;
     b.prims = S.d_prims;
     b.shells = S.d_shells;
     b.coef = S.d_coef;
@@ -2943,8 +2969,8 @@ static void incore_set(PlanData& P, int enable, hipStream_t s) {
     // quartet's primitives in one order (the deterministic mode's in-core
     // builds equal its direct builds bit for bit)
     b.bra_stage = qc.stage_cap;
-    const size_t lds = qc.stage_cap ? sizeof(double) * ((size_t)(qc.pb ? kStagedPrimCoef : kStagedPrim) * qc.stage_cap +
-                                                        (qc.nbra_max + 2) / 2) : 0;
+    const size_t lds = sizeof(double) * ((size_t)kBraRecDoubles * qc.nbra_max +
+                                         (size_t)(qc.pb ? kStagedPrimCoef : kStagedPrim) * qc.stage_cap);
     launch_jk_bra_class(qc.la, qc.lb, qc.lc, qc.ld, qc.pb, qc.pk, b, lds, s);
   }
   HIP_OK(hipGetLastError());

@@ -625,7 +625,7 @@ struct Wide {
 // DET: deterministic digestion (integer adds of values scaled by dscale).
 template <int LA, int LB, int LC, int LD, int CA, int CB, int CC, int CD, bool MOMENTS, typename R, int MODE = 0,
           bool DET = false>
-__device__ __forceinline__ void bra_item(const BraArgs& a, const MolInfo& mi, const Pair& bp, const Pair& kp,
+__device__ __forceinline__ void bra_item(const BraArgs& a, const MolInfo& mi, const BraRec& bp, const KetRec& kp,
                                          const int2 qk, int slot, int s0, int S, int Sk, int kc, double* __restrict__ krow,
                                          double* __restrict__ jrow, double* __restrict__ jket, int kwin0,
                                          const double* __restrict__ tab, double* __restrict__ cq,
@@ -637,7 +637,6 @@ __device__ __forceinline__ void bra_item(const BraArgs& a, const MolInfo& mi, co
   constexpr int ROWS = WA + WB;
   const int ns = a.n;  // LDS row length
   const int Sb = S / Sk, sb = s0 & (Sb - 1), sk = s0 / Sb;
-  const ShellXYZ sA = a.shells[bp.sa], sB = a.shells[bp.sb], sC = a.shells[kp.sa], sD = a.shells[kp.sb];
   // digestion addresses: molecule bases are chunk-uniform (scalar), element
   // offsets 32-bit (n <= 16384 Cartesian AOs per molecule, checked at plan
   // creation)
@@ -646,15 +645,18 @@ __device__ __forceinline__ void bra_item(const BraArgs& a, const MolInfo& mi, co
   // (multiples of S), so consecutive groups take consecutive copies
   const int jcopy = (threadIdx.x >> (__ffs(S) - 1)) & (kJBraCopies - 1);
   QuartetGeom geo;
-  double ABd[3], CDd[3];
-  load_geom(sA, sB, sC, sD, geo, ABd, CDd);
-  const R AB[3] = {(R)ABd[0], (R)ABd[1], (R)ABd[2]};
-  const R CD_[3] = {(R)CDd[0], (R)CDd[1], (R)CDd[2]};
+#pragma unroll
+  for (int x = 0; x < 3; ++x) {
+    geo.A[x] = bp.A[x];
+    geo.C[x] = kp.C[x];
+  }
+  const R AB[3] = {(R)bp.AB[0], (R)bp.AB[1], (R)bp.AB[2]};
+  const R CD_[3] = {(R)kp.CD[0], (R)kp.CD[1], (R)kp.CD[2]};
   double f = DET ? dscale : 1.0;
-  if (bp.sa == bp.sb) f *= 0.5;
-  if (kp.sa == kp.sb) f *= 0.5;
+  if (bp.la == bp.lb) f *= 0.5;
+  if (kp.lc == kp.ld) f *= 0.5;
   if (qk.x == qk.y) f *= 0.5;
-  const int oa = sA.ao, ob = sB.ao;
+  const int oa = bp.oa, ob = bp.ob;
   if constexpr (!W::kSplit) {
     R acc[WA][WB][WC][WD];
     if constexpr (MODE == 2) {
@@ -785,10 +787,9 @@ __device__ __forceinline__ void bra_item(const BraArgs& a, const MolInfo& mi, co
       for (int e = 0; e < WA * WB * WC * WD; ++e) cq[e] = (double)(&acc[0][0][0][0])[e];
     }
     }
-    const unsigned oc = sC.ao, od = sD.ao;
+    const unsigned oc = kp.oc, od = kp.od;
     // LDS exchange-row columns of C and D (compact over the class's ket mask)
-    const unsigned kc0 = a.shell_cofs ? (unsigned)a.shell_cofs[kp.sa * 8 + a.cmask] : oc;
-    const unsigned kd0 = a.shell_cofs ? (unsigned)a.shell_cofs[kp.sb * 8 + a.cmask] : od;
+    const unsigned kc0 = kp.kc, kd0 = kp.kd;
     const unsigned ra = (unsigned)oa * n, rb = (unsigned)ob * n, rc = oc * n, rd = od * n;
     for (int bt = 0; bt < a.nbd; ++bt) {
       const double* __restrict__ Dm = a.dens + (size_t)bt * a.bstride + mi.base;
@@ -956,10 +957,9 @@ __device__ __forceinline__ void bra_item(const BraArgs& a, const MolInfo& mi, co
       for (int e = 0; e < WA * WB; ++e) cq[e] = (double)(&acc[0][0])[e];
     }
     }
-    const unsigned c = sC.ao + icw, d = sD.ao + idw;
+    const unsigned c = kp.oc + icw, d = kp.od + idw;
     // LDS exchange-row columns of this lane's C and D components
-    const unsigned xc = (a.shell_cofs ? (unsigned)a.shell_cofs[kp.sa * 8 + a.cmask] : sC.ao) + icw;
-    const unsigned xd = (a.shell_cofs ? (unsigned)a.shell_cofs[kp.sb * 8 + a.cmask] : sD.ao) + idw;
+    const unsigned xc = kp.kc + icw, xd = kp.kd + idw;
     const unsigned ra = (unsigned)oa * n, rb = (unsigned)ob * n;
     for (int bt = 0; bt < a.nbd; ++bt) {
       const double* __restrict__ Dm = a.dens + (size_t)bt * a.bstride + mi.base;
@@ -1059,79 +1059,89 @@ __global__ __launch_bounds__(512) void jk_bra_kernel(BraArgs a) {
   MolInfo mi;
   double dscale = 1.0;
   {
-    const int mol = a.shells[a.pairs[ch.bra0].sa].mol;
-    if constexpr (DET) dscale = a.det_scale[2 * mol];
-    const MolInfo m = a.mols[mol];
+    if constexpr (DET) dscale = a.det_scale[2 * ch.mol];
+    const MolInfo m = a.mols[ch.mol];
     mi.base = uniform_i64(m.base);
     mi.dbase = uniform_i64(m.dbase);
     mi.n = __builtin_amdgcn_readfirstlane(m.n);
     mi.nseg = __builtin_amdgcn_readfirstlane(m.nseg);
   }
   const int krow_size = a.nbd * a.nbra_max * ROWS * ns;
-  double* krow = lds;                      // [nbd][slot][ROWS][n]
-  double* jrow = lds + krow_size;          // [nbj][slot][copy][NA][NB]
+  BraRec* brec = reinterpret_cast<BraRec*>(lds);     // [slot]
+  double* krow = lds + kBraRecDoubles * a.nbra_max;  // [nbd][slot][ROWS][n]
+  double* jrow = krow + krow_size;                   // [nbj][slot][copy][NA][NB]
   const int jrow_size = a.nbj * a.nbra_max * kJBraCopies * W::NBRA;
   // ket-side J of the chunk's ket window: [nbj][nket_max][NC*ND]
   double* jket = (a.nket_max > 0 && ch.nket > 0) ? jrow + jrow_size : nullptr;
   const int jket_size = a.nbj * a.nket_max * W::NKET;
   const int zero_size = krow_size + jrow_size + (jket ? jket_size : 0);
-  for (int i = threadIdx.x; i < zero_size; i += blockDim.x) lds[i] = 0.0;
+  // the chunk's bra pairs and shells, read once by one lane each: no later
+  // step waits for a chain of table reads per slot
+  for (int j = threadIdx.x; j < ch.nbra; j += blockDim.x) {
+    const Pair p = a.pairs[ch.bra0 + j];
+    const ShellXYZ A = a.shells[p.sa], B = a.shells[p.sb];
+    brec[j] = {{A.x, A.y, A.z}, {A.x - B.x, A.y - B.y, A.z - B.z}, p.poff, p.np, A.ao, B.ao, A.lseg, B.lseg, 0, 0};
+  }
+  for (int i = threadIdx.x; i < zero_size; i += blockDim.x) krow[i] = 0.0;
+  __syncthreads();
   // D_ab + D_ba of every slot's bra block, per Coulomb density: read by the
   // bra-side and ket-side J digestion of every quartet of the slot
   const int dab_size = a.with_j ? a.nbj * a.nbra_max * W::NBRA : 0;
-  double* dabs = lds + krow_size + jrow_size + jket_size;
+  double* dabs = krow + krow_size + jrow_size + jket_size;
   for (int i = threadIdx.x; i < dab_size; i += blockDim.x) {
     const int e = i % W::NBRA;
     const int slot = (i / W::NBRA) % a.nbra_max;
     const int bt = i / (W::NBRA * a.nbra_max);
     double v = 0.0;
     if (slot < ch.nbra) {
-      const Pair bp = a.pairs[ch.bra0 + slot];
-      const unsigned oa = a.shells[bp.sa].ao + e / W::WB, ob = a.shells[bp.sb].ao + e % W::WB;
+      const unsigned oa = brec[slot].oa + e / W::WB, ob = brec[slot].ob + e % W::WB;
       const double* __restrict__ Dm = a.dens + (size_t)bt * a.bstride + mi.base;
       v = Dm[(size_t)oa * mi.n + ob] + Dm[(size_t)ob * mi.n + oa];
     }
     dabs[i] = v;
   }
-  // staged bra primitive pairs [records][kStagedPrim] and the first record
-  // of every slot (full-block segmented classes that evaluate)
+  // staged bra primitive pairs [records][kStagedPrim] (full-block classes
+  // that evaluate), a slot's from its record number `first`
   constexpr bool kStage = !W::kSplit && MODE != 2;
   // record doubles: p, P - A, e, 1/p (+ the bra's column coefficients)
   constexpr int kRec = kStagedPrim + (CA * CB > 1 ? 4 : 0);
-  const int stage_base = (krow_size + jrow_size + jket_size + dab_size + 1) & ~1;  // 16-byte aligned
-  const int stage_size = kStage && a.bra_stage ? kRec * a.bra_stage + (a.nbra_max + 2) / 2 : 0;
+  // (from lds; 16-byte aligned)
+  const int stage_base = (kBraRecDoubles * a.nbra_max + krow_size + jrow_size + jket_size + dab_size + 1) & ~1;
+  const int stage_size = kStage ? kRec * a.bra_stage : 0;
   double* bstage = lds + stage_base;
-  int* bslot = reinterpret_cast<int*>(bstage + kRec * a.bra_stage);
   if constexpr (kStage) {
     if (a.bra_stage) {
-      if (threadIdx.x == 0) {
+      for (int j = threadIdx.x; j < ch.nbra; j += blockDim.x) {
         int o = 0;
-        for (int j = 0; j < ch.nbra; ++j) {
-          bslot[j] = o;
-          o += a.pairs[ch.bra0 + j].np;
-        }
+        for (int k = 0; k < j; ++k) o += brec[k].np;
+        brec[j].first = o;
       }
       __syncthreads();
-      for (int j = 0; j < ch.nbra; ++j) {
-        const Pair bp = a.pairs[ch.bra0 + j];
-        double* dst = bstage + kRec * bslot[j];
-        for (int k = threadIdx.x; k < bp.np; k += blockDim.x) {
-          const PrimPair P = a.prims[bp.poff + k];
-          const ShellXYZ A = a.shells[bp.sa];
-          double* rec = dst + kRec * k;
-          rec[0] = P.p;
-          rec[1] = P.px - A.x;
-          rec[2] = P.py - A.y;
-          rec[3] = P.pz - A.z;
-          rec[4] = P.e;
-          rec[5] = P.ip;
-          if constexpr (CA * CB > 1) {
-            const PrimCoef c = a.coef[bp.poff + k];
-            rec[6] = c.ca[0];
-            rec[7] = c.ca[1];
-            rec[8] = c.cb[0];
-            rec[9] = c.cb[1];
-          }
+      // all slots' primitive pairs at once: a loop over the slots would wait
+      // for memory once per slot
+      const int nrec = brec[ch.nbra - 1].first + brec[ch.nbra - 1].np;
+      for (int i = threadIdx.x; i < nrec; i += blockDim.x) {
+        int lo = 0, hi = ch.nbra;
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if (brec[mid].first <= i) lo = mid; else hi = mid;
+        }
+        const BraRec& b = brec[lo];
+        const int k = b.poff + i - b.first;
+        const PrimPair P = a.prims[k];
+        double* rec = bstage + kRec * i;
+        rec[0] = P.p;
+        rec[1] = P.px - b.A[0];
+        rec[2] = P.py - b.A[1];
+        rec[3] = P.pz - b.A[2];
+        rec[4] = P.e;
+        rec[5] = P.ip;
+        if constexpr (CA * CB > 1) {
+          const PrimCoef c = a.coef[k];
+          rec[6] = c.ca[0];
+          rec[7] = c.ca[1];
+          rec[8] = c.cb[0];
+          rec[9] = c.cb[1];
         }
       }
     }
@@ -1172,14 +1182,13 @@ __global__ __launch_bounds__(512) void jk_bra_kernel(BraArgs a) {
     const int64_t g = ch.q0 + qr;
     const int2 qk = a.quartets[g];
     const int slot = qk.x - ch.bra0;
-    const Pair bp = a.pairs[qk.x];
-    const Pair kp = a.pairs[qk.y];
+    const BraRec& bp = brec[slot];
+    const KetRec kp = a.kets[qk.y];
     double* cq = nullptr;
     if constexpr (MODE != 0) cq = a.cache + ((size_t)g * W::SPLIT + kc) * kBlock;
     bool lowp = false;
     if constexpr (MIX) {
-      const int la = a.shells[bp.sa].lseg, lb = a.shells[bp.sb].lseg;
-      const int lc = a.shells[kp.sa].lseg, ld = a.shells[kp.sb].lseg;
+      const int la = bp.la, lb = bp.lb, lc = kp.lc, ld = kp.ld;
       const double* dm = a.dmax + mi.dbase;
       const int nsg = mi.nseg;
       const double d6 = fmax(fmax(fmax(dm[la * nsg + lb], dm[lc * nsg + ld]),
@@ -1195,11 +1204,11 @@ __global__ __launch_bounds__(512) void jk_bra_kernel(BraArgs a) {
       if (lowp) {
         bra_item<LA, LB, LC, LD, CA, CB, CC, CD, kMoments, float>(
             a, mi, bp, kp, qk, slot, s0, S, Sk, kc, krow, jrow, jket, ch.ket0, tab, cq, 1.0,
-            (kStage && a.bra_stage) ? bstage + kRec * bslot[slot] : nullptr, dabs);
+            (kStage && a.bra_stage) ? bstage + kRec * bp.first : nullptr, dabs);
         continue;
       }
     }
-    const double* bpl = (kStage && a.bra_stage) ? bstage + kRec * bslot[slot] : nullptr;
+    const double* bpl = (kStage && a.bra_stage) ? bstage + kRec * bp.first : nullptr;
     bra_item<LA, LB, LC, LD, CA, CB, CC, CD, kMoments, double, MODE, DET>(a, mi, bp, kp, qk, slot, s0, S, Sk, kc, krow,
                                                                            jrow, jket, ch.ket0, tab, cq, dscale, bpl,
                                                                            dabs);
@@ -1208,7 +1217,7 @@ __global__ __launch_bounds__(512) void jk_bra_kernel(BraArgs a) {
   // the chunk's molecule and the columns its exchange terms can reach (the
   // shells whose l is in the class's ket mask)
   const bool compact = a.shell_cofs != nullptr;
-  const int2 cspace = ((a.part_mode & 3) || compact) ? a.cspace[a.shells[a.pairs[ch.bra0].sa].mol * 8 + a.cmask]
+  const int2 cspace = ((a.part_mode & 3) || compact) ? a.cspace[ch.mol * 8 + a.cmask]
                                                      : make_int2(0, mi.n);
   if (a.part_mode & 1) {
     // exchange rows to the chunk's partial slab with plain stores, over the
@@ -1240,9 +1249,7 @@ __global__ __launch_bounds__(512) void jk_bra_kernel(BraArgs a) {
       if (col >= cspace.y) continue;
       col = a.colmap[cspace.x + col];
     }
-    const Pair bp = a.pairs[ch.bra0 + slot];
-    const MolInfo mi = a.mols[a.shells[bp.sa].mol];
-    const int row = r < W::WA ? a.shells[bp.sa].ao + r : a.shells[bp.sb].ao + (r - W::WA);
+    const int row = r < W::WA ? brec[slot].oa + r : brec[slot].ob + (r - W::WA);
     acc_flush<DET>(a.kp + (size_t)bt * a.bstride + mi.base + (size_t)row * mi.n + col, krow + i);
   }
   for (int i = threadIdx.x; i < jrow_size / kJBraCopies; i += blockDim.x) {
@@ -1264,9 +1271,7 @@ __global__ __launch_bounds__(512) void jk_bra_kernel(BraArgs a) {
       for (int c = 0; c < kJBraCopies; ++c) v += jrow[((bt * a.nbra_max + slot) * kJBraCopies + c) * W::NBRA + e];
     }
     if (acc_zero<DET>(&v)) continue;
-    const Pair bp = a.pairs[ch.bra0 + slot];
-    const MolInfo mi = a.mols[a.shells[bp.sa].mol];
-    const int row = a.shells[bp.sa].ao + e / W::WB, col = a.shells[bp.sb].ao + e % W::WB;
+    const int row = brec[slot].oa + e / W::WB, col = brec[slot].ob + e % W::WB;
     acc_flush<DET>(a.jp + (size_t)bt * a.bstride + mi.base + (size_t)row * mi.n + col, &v);
   }
   if (jket && (a.part_mode & 2)) {
@@ -1288,9 +1293,8 @@ __global__ __launch_bounds__(512) void jk_bra_kernel(BraArgs a) {
       const int bt = i / (W::NKET * ch.nket);
       const double* src = jket + ((size_t)bt * a.nket_max + w) * W::NKET + e;
       if (acc_zero<DET>(src)) continue;
-      const Pair kp = a.pairs[ch.ket0 + w];
-      const MolInfo mi = a.mols[a.shells[kp.sa].mol];
-      const int row = a.shells[kp.sa].ao + e / W::WD, col = a.shells[kp.sb].ao + e % W::WD;
+      const KetRec& kp = a.kets[ch.ket0 + w];
+      const int row = kp.oc + e / W::WD, col = kp.od + e % W::WD;
       acc_flush<DET>(a.jket_pad + 8 * ((size_t)bt * a.bstride + mi.base + (size_t)row * mi.n + col), src);
     }
   }

@@ -36,6 +36,7 @@ def test_windows_add_the_same_terms(oracle_mod, waters):
     outs = [_build(tables, sched, dict(deterministic=1, **opt), d)
             for sched, opt in ((dict(bras_max=1), {}), ({}, {}), (dict(bras_max=2), {}),
                                (dict(chunk_items=65536), {}), (dict(ket_lds=1), {}),
+                               (dict(bras_max=256, lds_pack=65536, chunk_items=65536), {}),
                                ({}, dict(lds_limit=16384)))]
     for o in outs[1:]:
         assert np.array_equal(o, outs[0])
