@@ -1028,8 +1028,9 @@ __device__ __forceinline__ void bra_item(const BraArgs& a, const MolInfo& mi, co
 // rows of the bra shells (Kp[a,c], Kp[a,d], Kp[b,c], Kp[b,d]), so they are
 // accumulated with LDS atomics in per-bra row slabs [rows of A, rows of B] x n
 // and flushed to global memory once per workgroup; the bra-side J block is
-// accumulated in LDS the same way.  Only the ket-side J terms go straight to
-// global atomics.  Global FP64 atomics are executed at the memory side on this
+// accumulated in LDS the same way.  Only the ket-side J terms go to global
+// atomics, one per quartet and component or (a.nket_max) one per window entry
+// after a sum over the chunk's bras in LDS.  Global FP64 atomics are executed at the memory side on this
 // platform, so their count, not FLOPs, is what this layout minimises.
 // With a.mixed set, a quartet whose Q_ij Q_kl max|D| (max over the six density
 // blocks it touches) is below a.thr may be evaluated in FP32 (roots, weights
