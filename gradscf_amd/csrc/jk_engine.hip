@@ -25,6 +25,7 @@
 #include "_generated/rys_table.inc"
 #include "gradscf_jk.h"
 #include "gscf_args.h"
+#include "launch_limits.h"
 
 namespace gscf {
 
@@ -823,8 +824,8 @@ __global__ __launch_bounds__(256) void ket_records_kernel(const Pair* __restrict
             C.lseg, D.lseg, {C.x, C.y, C.z}, {C.x - D.x, C.y - D.y, C.z - D.z}};
 }
 
-// Quartet lists of every (bra run, ket run) sub-task of a plan, one launch:
-// g -> (bra0 + b, ket0 + g - qoff[b]) with qoff[b] <= g - g0 < qoff[b+1].
+// Quartet lists of every (bra run, ket run) sub-task of a plan in one launch
+// (or as few as the grid allows): g -> (bra0 + b, ket0 + g - qoff[b]) with qoff[b] <= g - g0 < qoff[b+1].
 // Bra b keeps the ket-run prefix [0, qoff[b+1] - qoff[b]) (Schwarz-descending
 // run).  The prefix is cut into segments of seg kets (the ket windows of
 // single-bra chunks) and each segment is written in the run's primitive-count
@@ -839,17 +840,16 @@ struct ExpandTask {
   int64_t qoff;    // its nbra + 1 prefix sums in the plan's table
   int nbra, bra0, ket0, seg;
   int grp0, ngrp;  // groups of the ket run
-  int sorted;      // the chunk sort reads the list from the scratch copy
-  int pad;
 };
 
-__global__ __launch_bounds__(256) void expand_kernel(const ExpandTask* __restrict__ tasks, int ntask, int64_t total,
-                                                     const int64_t* __restrict__ qoff_all,
+// Quartets [first, first + count) of the list.
+__global__ __launch_bounds__(256) void expand_kernel(const ExpandTask* __restrict__ tasks, int ntask, int64_t first,
+                                                     int64_t count, const int64_t* __restrict__ qoff_all,
                                                      const int* __restrict__ order_all,
-                                                     const int2* __restrict__ groups_all, int2* __restrict__ scratch,
-                                                     int2* __restrict__ out) {
-  const int64_t gg = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gg >= total) return;
+                                                     const int2* __restrict__ groups_all, int2* __restrict__ out) {
+  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= count) return;
+  const int64_t gg = first + idx;
   int t0 = 0, t1 = ntask;
   while (t1 - t0 > 1) {
     const int mid = (t0 + t1) >> 1;
@@ -890,7 +890,7 @@ __global__ __launch_bounds__(256) void expand_kernel(const ExpandTask* __restric
     }
     rr -= c - a;
   }
-  (t.sorted ? scratch : out)[gg] = make_int2(t.bra0 + lo, t.ket0 + ket);
+  out[gg] = make_int2(t.bra0 + lo, t.ket0 + ket);
 }
 
 // Order of the quartets inside every bra-major chunk: by ket primitive-pair
@@ -901,40 +901,36 @@ __global__ __launch_bounds__(256) void expand_kernel(const ExpandTask* __restric
 // evaluation (grid expansion below the switch, asymptotic form above) and
 // reads neighbouring grid rows.  One workgroup per chunk: 64-bit keys
 // (count, distance bits, position) bitonic-sorted in LDS, then the quartets
-// gathered through a scratch copy.  nq of a chunk is at most kSortMax.
-// Chunks of every class in one launch; src and dst are the plan's lists.
+// gathered into the keys' places and written back: the list is sorted where it
+// is, whatever its size.  nq of a chunk is at most kSortMax.
+// Chunks of every class in one launch (or as few as the grid allows).
 constexpr int kSortMax = 8192;
 
 // Chunks [chunk0, next class's chunk0) of one class whose quartets start at q0
-// of the plan's list; sort 0: too long to sort, copied.
+// of the plan's list; sort 0: too long to sort.
 struct SortClass {
   int chunk0, sort;
   int64_t q0;
 };
 
 __global__ __launch_bounds__(256) void sort_chunk_kernel(const SortClass* __restrict__ classes, int nclass,
-                                                         const BraChunk* __restrict__ chunks,
+                                                         const BraChunk* __restrict__ chunks, int first,
                                                          const Pair* __restrict__ pairs,
-                                                         const ShellXYZ* __restrict__ shells,
-                                                         const int2* __restrict__ src_all, int2* __restrict__ dst_all) {
+                                                         const ShellXYZ* __restrict__ shells, int2* list) {
   extern __shared__ uint64_t key[];
+  const int ci = first + (int)blockIdx.x;
   int k = 0;
-  while (k + 1 < nclass && classes[k + 1].chunk0 <= (int)blockIdx.x) ++k;
-  const BraChunk c = chunks[blockIdx.x];
-  const int2* __restrict__ src = src_all + classes[k].q0 + c.q0;
-  int2* __restrict__ dst = dst_all + classes[k].q0 + c.q0;
+  while (k + 1 < nclass && classes[k + 1].chunk0 <= ci) ++k;
+  if (!classes[k].sort) return;
+  const BraChunk c = chunks[ci];
+  int2* q = list + classes[k].q0 + c.q0;
   const int nq = c.nq;
-  if (!classes[k].sort) {
-    for (int i = threadIdx.x; i < nq; i += blockDim.x) dst[i] = src[i];
-    return;
-  }
   int np2 = 1;
   while (np2 < nq) np2 <<= 1;
   for (int i = threadIdx.x; i < np2; i += blockDim.x) {
     uint64_t v = ~0ull;
     if (i < nq) {
-      const int2 q = src[i];
-      const Pair b = pairs[q.x], t = pairs[q.y];
+      const Pair b = pairs[q[i].x], t = pairs[q[i].y];
       const ShellXYZ A = shells[b.sa], B = shells[b.sb], C = shells[t.sa], D = shells[t.sb];
       const double dx = 0.5 * (A.x + B.x - C.x - D.x), dy = 0.5 * (A.y + B.y - C.y - D.y),
                    dz = 0.5 * (A.z + B.z - C.z - D.z);
@@ -960,7 +956,13 @@ __global__ __launch_bounds__(256) void sort_chunk_kernel(const SortClass* __rest
       }
       __syncthreads();
     }
-  for (int i = threadIdx.x; i < nq; i += blockDim.x) dst[i] = src[(int)(key[i] & 0x3fff)];
+  for (int i = threadIdx.x; i < nq; i += blockDim.x) {
+    const int2 v = q[key[i] & 0x3fff];
+    key[i] = (uint64_t)(uint32_t)v.x | (uint64_t)(uint32_t)v.y << 32;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < nq; i += blockDim.x)
+    q[i] = make_int2((int)(uint32_t)key[i], (int)(uint32_t)(key[i] >> 32));
 }
 
 // dmax[m][S][T] = max over batches and over the Cartesian block (S, T) of |D_m|
@@ -1806,7 +1808,7 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
           place.push_back({S.nquartets, chunks.size(), subtasks.size()});
           for (const Pending& pd : pend) {
             expand.push_back({S.nquartets + pd.q0, (int64_t)qoffs.size(), pd.nbra, pd.bra0, pd.ket0, pd.seg,
-                              run_g0[pd.rk], run_g0[pd.rk + 1] - run_g0[pd.rk], !qc.chunks.empty(), 0});
+                              run_g0[pd.rk], run_g0[pd.rk + 1] - run_g0[pd.rk]});
             qoffs.insert(qoffs.end(), pd.qoff.begin(), pd.qoff.end());
           }
           if (!qc.chunks.empty()) {
@@ -1897,19 +1899,20 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
     const size_t o_expand = work.add(expand), o_qoff = work.add(qoffs), o_order = work.add(run_order),
                  o_groups = work.add(run_groups), o_sort = work.add(sort_classes);
     work.send(s);
-    int2* scratch = nullptr;
-    if (!chunks.empty()) HIP_OK(hipMalloc(&scratch, sizeof(int2) * S.nquartets));
-    hipLaunchKernelGGL(expand_kernel, dim3(nblocks((size_t)S.nquartets)), dim3(256), 0, s,
-                       work.at<ExpandTask>(o_expand), (int)expand.size(), S.nquartets, work.at<int64_t>(o_qoff),
-                       work.at<int>(o_order), work.at<int2>(o_groups), scratch, S.d_quartets);
-    if (!chunks.empty())
-      hipLaunchKernelGGL(sort_chunk_kernel, dim3((unsigned)chunks.size()), dim3(256), sizeof(uint64_t) * sort_len, s,
+    // (a launch that fails ends the plan before the next one reads the list)
+    for_slices(S.nquartets, grid_blocks(256) * 256, [&](int64_t first, int64_t count) {
+      hipLaunchKernelGGL(expand_kernel, dim3(nblocks((size_t)count)), dim3(256), 0, s, work.at<ExpandTask>(o_expand),
+                         (int)expand.size(), first, count, work.at<int64_t>(o_qoff), work.at<int>(o_order),
+                         work.at<int2>(o_groups), S.d_quartets);
+      HIP_OK(hipGetLastError());
+    });
+    for_slices((int64_t)chunks.size(), grid_blocks(256), [&](int64_t first, int64_t count) {
+      hipLaunchKernelGGL(sort_chunk_kernel, dim3((unsigned)count), dim3(256), sizeof(uint64_t) * sort_len, s,
                          work.at<SortClass>(o_sort), (int)sort_classes.size(), (const BraChunk*)at(o_chunks),
-                         S.d_pairs, S.d_shells, scratch, S.d_quartets);
-    const hipError_t launched = hipGetLastError(), done = hipStreamSynchronize(s);
-    if (scratch) (void)hipFree(scratch);
-    HIP_OK(launched);
-    HIP_OK(done);
+                         (int)first, S.d_pairs, S.d_shells, S.d_quartets);
+      HIP_OK(hipGetLastError());
+    });
+    HIP_OK(hipStreamSynchronize(s));
   }
   S.built = true;
 }
@@ -2465,8 +2468,10 @@ static int64_t plan_bytes(const PlanData& P, int64_t nbd) {
 // densities (nonsymmetric K doubles the workspace): the exact size of every
 // table, with every intra-molecule canonical pair quartet retained (no
 // Schwarz screening is evaluated), at most one chunk per quartet and one
-// sub-task per pair of (class, bucket) runs.  Transient buffers (Schwarz blocks, one-electron staging) are freed
-// before a build and do not add to it.
+// sub-task per pair of (class, bucket) runs.  Transient buffers of plan
+// creation (Schwarz bounds, the expansion's prefix sums: 8 bytes per bra and
+// ket run) are freed before a build and do not add to it; the quartet list is
+// expanded and sorted where it stays.
 static int64_t forecast_bytes(PlanData& P, int nb) {
   build_segments(P);
   P.mol_pair0.assign(P.nmol + 1, 0);

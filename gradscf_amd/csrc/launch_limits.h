@@ -1,0 +1,25 @@
+// Sizes of one launch (host code, no HIP headers).
+//
+// A dispatch counts its work items per dimension in 32 bits: a launch with
+// gridDim.x * blockDim.x of 2^32 or more is refused.  Launches whose size
+// grows with the molecule are cut into slices below that.
+#pragma once
+#include <algorithm>
+#include <cstdint>
+
+namespace gscf {
+
+constexpr int64_t kGridThreads = (int64_t(1) << 32) - 1;
+constexpr int64_t kGridYZ = 65535;  // workgroups along y or z
+
+// Workgroups of `threads` lanes one launch may have along x.
+constexpr int64_t grid_blocks(int threads) { return kGridThreads / threads; }
+
+// launch(begin, count) over consecutive slices of [0, total), at most `limit`
+// entries each.
+template <class F>
+void for_slices(int64_t total, int64_t limit, F&& launch) {
+  for (int64_t begin = 0; begin < total; begin += limit) launch(begin, std::min(limit, total - begin));
+}
+
+}  // namespace gscf
