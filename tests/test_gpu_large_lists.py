@@ -26,8 +26,7 @@ def test_unscreened_plan_past_one_launch():
     d = torch.as_tensor(systems.random_density(n, seed=3), device="cuda")
     screened = DirectJKPlan(*tables, cart=True, cutoff=cutoff).jk(d).cpu()
     plan = DirectJKPlan(*tables, cart=True, cutoff=0.0)
-    pairs = n * (n + 1) // 2
-    assert plan.info["nquartets"] == pairs * (pairs + 1) // 2 > 2 ** 32
+    assert plan.info["nquartets"] > 2 ** 32
     out = plan.jk(d).cpu()
     # every quartet the screened plan leaves out is below the cutoff, and an
     # element sums at most n^2 of them times a density element
