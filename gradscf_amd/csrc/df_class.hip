@@ -25,7 +25,7 @@ __device__ __forceinline__ void df_blocks(const DfArgs& a, const DfRange& r, dou
   constexpr int NBRA = K::NBRA, NC = K::NC;
   const int lanes = K::SPLIT * r.S;
   const int local = threadIdx.x / lanes;
-  const int64_t t0 = (int64_t)(blockIdx.x - r.block0) * r.T;
+  const int64_t t0 = r.task0 + (int64_t)(blockIdx.x - r.block0) * r.T;
   const int64_t ntask = (int64_t)r.npair * a.nket;
   if (local < r.T && t0 + local < ntask) {
     const int64_t t = t0 + local;

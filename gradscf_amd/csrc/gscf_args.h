@@ -259,13 +259,15 @@ struct SphTerm {
 
 // Bra pairs [pair0, pair0 + npair) of one class (la, lb) with similar
 // primitive counts: T (bra pair, ket shell) tasks per block, each on
-// S (x ket components) lanes, blocks from block0 on.
+// S (x ket components) lanes, tasks from task0 and blocks from block0 on (a
+// range may be spread over several launches).
 struct DfRange {
   int la, lb;
   int pair0, npair;
   int S, T;
   int block0;
   int pad;
+  int64_t task0;
 };
 
 // Lanes over ket components: blocks of more than 36 Cartesian components do
@@ -294,12 +296,14 @@ struct DfArgs {
 // ----------------------------------------------------------------------------
 // Tasks (bra pair, ket pair) of two pair ranges with similar primitive counts
 // (tri: one range with itself, ket <= bra): T per block on S = Sb * Sk lanes
-// (x ket components) each, blocks from block0 on.
+// (x ket components) each, tasks from task0 and blocks from block0 on (a range
+// may be spread over several launches).
 struct EriRange {
   int bra0, nbra, ket0, nket;
   int S, Sk, T, tri;
   int block0;
   int pad;
+  int64_t task0;
 };
 
 struct EriArgs {

@@ -3490,7 +3490,7 @@ static void packed_eri(const int32_t* atm, int natm, const int32_t* bas, int nba
         for (size_t j = 0; j < runs[ck].size(); ++j) {
           if (cb == ck && j < i) continue;  // one order of two runs
           const Run &b = runs[cb][i], &k = runs[ck][j];
-          EriRange r{b.beg, b.end - b.beg, k.beg, k.end - k.beg, 1, 1, 1, cb == ck && i == j, (int)blocks, 0};
+          EriRange r{b.beg, b.end - b.beg, k.beg, k.end - k.beg, 1, 1, 1, cb == ck && i == j, 0, 0, 0};
           SubTask t;
           // runs are sorted: the first pair has the most primitives, the last the fewest
           choose_split(pairs[b.end - 1].np, pairs[b.beg].np, pairs[k.end - 1].np, pairs[k.beg].np, kEriPrim, t);
@@ -3502,15 +3502,21 @@ static void packed_eri(const int32_t* atm, int natm, const int32_t* bas, int nba
           r.Sk = t.Sk;
           const size_t blk = sizeof(double) * nbra * nket;
           r.T = (int)std::max<size_t>(1, std::min<size_t>({(size_t)256 / (r.S * split), kLdsBudget / blk, (size_t)share}));
-          L.lds = std::max(L.lds, blk * r.T);
           const int64_t tasks = r.tri ? (int64_t)r.nbra * (r.nbra + 1) / 2 : (int64_t)r.nbra * r.nket;
-          blocks += (tasks + r.T - 1) / r.T;
-          if (blocks > std::numeric_limits<int>::max()) throw Internal("too many packed ERI blocks");
-          ranges.push_back(r);
-          ++L.nrange;
+          cut_blocks((tasks + r.T - 1) / r.T, grid_blocks(256), blocks, [&](int64_t first, int64_t count, bool fresh) {
+            if (fresh) {
+              launches.push_back(L);
+              L = {cb, ck, (int)ranges.size(), 0, 0, 0};
+            }
+            r.task0 = first * r.T;
+            r.block0 = L.blocks;
+            ranges.push_back(r);
+            L.blocks += (int)count;
+            L.lds = std::max(L.lds, blk * r.T);
+            ++L.nrange;
+          });
         }
-      L.blocks = (int)blocks;
-      if (blocks) launches.push_back(L);
+      if (L.blocks) launches.push_back(L);
     }
   if (P.prims.empty()) P.prims.push_back(PrimPair{});
   EriArgs a;
@@ -3634,20 +3640,27 @@ static void density_fitting(const int32_t* atm, int natm, const int32_t* bas, in
       for (int i = b.beg; i < b.end;) {
         int e = i;
         while (e < b.end && pair_bucket(pairs[e]) == pair_bucket(pairs[i])) ++e;
-        DfRange r{b.la, b.lb, i, e - i, 1, 1, (int)blocks, 0};
+        DfRange r{b.la, b.lb, i, e - i, 1, 1, 0, 0, 0};
         const int64_t work = (int64_t)pairs[i].np * pairs[aux0[lc]].np;
         while (r.S < 16 && (int64_t)r.S * kDfPrim < work && 2 * r.S <= pairs[e - 1].np) r.S *= 2;
         r.T = (int)std::max<size_t>(1, std::min<size_t>({(size_t)256 / (r.S * df_split(b.la, b.lb, lc)), kLdsBudget / (8 * blk), share}));
-        L.lds = std::max(L.lds, 8 * blk * r.T);
-        blocks += ((int64_t)r.npair * nket + r.T - 1) / r.T;
-        if (blocks > std::numeric_limits<int>::max()) throw Internal("too many auxiliary integral blocks");
-        ranges.push_back(r);
-        ++L.nrange;
+        const int64_t range_tasks = (int64_t)r.npair * nket;
+        cut_blocks((range_tasks + r.T - 1) / r.T, grid_blocks(256), blocks, [&](int64_t first, int64_t count, bool fresh) {
+          if (fresh) {
+            launches.push_back(L);
+            L = {lc, (int)ranges.size(), 0, 0, 0};
+          }
+          r.task0 = first * r.T;
+          r.block0 = L.blocks;
+          ranges.push_back(r);
+          L.blocks += (int)count;
+          L.lds = std::max(L.lds, 8 * blk * r.T);
+          ++L.nrange;
+        });
         i = e;
       }
     }
-    L.blocks = (int)blocks;
-    launches.push_back(L);
+    if (L.blocks) launches.push_back(L);
   }
   if (P.prims.empty()) P.prims.push_back(PrimPair{});
   Upload up;
@@ -3663,7 +3676,6 @@ static void density_fitting(const int32_t* atm, int natm, const int32_t* bas, in
   a.m = m;
   a.out = out;
   for (const Launch& L : launches) {
-    if (L.blocks == 0) continue;
     a.ranges = up.at<DfRange>(o_ranges) + L.r0;
     a.nrange = L.nrange;
     a.ket0 = aux0[L.lc];

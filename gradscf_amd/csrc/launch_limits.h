@@ -22,4 +22,20 @@ void for_slices(int64_t total, int64_t limit, F&& launch) {
   for (int64_t begin = 0; begin < total; begin += limit) launch(begin, std::min(limit, total - begin));
 }
 
+// Cuts a range of `blocks` blocks into pieces of consecutive launches of at
+// most `limit` blocks.  used: blocks the open launch holds already, updated;
+// piece(first block, count, fresh) with fresh where the piece opens a new
+// launch (whose used is then zero).
+template <class F>
+void cut_blocks(int64_t blocks, int64_t limit, int64_t& used, F&& piece) {
+  for (int64_t first = 0; first < blocks;) {
+    const bool fresh = used == limit;
+    if (fresh) used = 0;
+    const int64_t count = std::min(blocks - first, limit - used);
+    piece(first, count, fresh);
+    used += count;
+    first += count;
+  }
+}
+
 }  // namespace gscf

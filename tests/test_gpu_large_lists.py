@@ -31,3 +31,44 @@ def test_unscreened_plan_past_one_launch():
     # every quartet the screened plan leaves out is below the cutoff, and an
     # element sums at most n^2 of them times a density element
     assert float((out - screened).abs().max()) < n * n * cutoff * float(d.abs().max())
+
+
+def test_packed_integrals_past_one_launch():
+    import torch
+    from gradscf_amd.jk import DirectJKPlan, packed_eri, packed_jk
+    n = 220
+    tables = hydrogens(n)
+    eri = packed_eri(*tables, cart=True)
+    d = torch.as_tensor(systems.random_density(n, seed=4), device="cuda")
+    ref = DirectJKPlan(*tables, cart=True, cutoff=0.0).jk(d)
+    # the bound of the other J/K comparisons (1e-10 per element)
+    assert float((torch.stack(packed_jk(eri, d)) - ref).abs().max()) < 1e-10
+
+
+def test_auxiliary_integrals_past_one_launch():
+    """500 orbital s shells of six primitives against 2200 auxiliary ones: the
+    rows of the first and the last auxiliary shells are those of a call with
+    these alone."""
+    import torch
+    from gradscf_amd.density_fitting import evaluate
+    rng = np.random.default_rng(2)
+    norb, naux, part = 500, 2200, 40
+    atm = np.zeros((8, 6), np.int32)
+    atm[:, 0] = 1
+    atm[:, 1] = 20 + 3 * np.arange(8)
+    atm[:, 2] = 1
+    orb_exp = 0.3 * 2.5 ** np.arange(6)
+    aux_exp = rng.uniform(0.2, 4.0, naux)
+    env = np.concatenate([np.zeros(20), rng.uniform(-0.5, 0.5, 24), orb_exp, rng.uniform(0.2, 1.0, 6), aux_exp,
+                          np.ones(naux)])
+
+    def bas(aux):
+        rows = [[i % 8, 0, 6, 1, 0, 44, 50, 0] for i in range(norb)]
+        return np.array(rows + [[i % 8, 0, 1, 1, 0, 56 + i, 56 + naux + i, 0] for i in aux], np.int32)
+
+    def three(aux):
+        return evaluate(atm, bas(aux), env, (len(aux), norb * (norb + 1) // 2), layout=3, cart=True, split=norb)
+
+    whole = three(range(naux))
+    assert torch.equal(whole[:part], three(range(part)))
+    assert torch.equal(whole[-part:], three(range(naux - part, naux)))

@@ -22,6 +22,21 @@ int slices(long long total, long long limit, long long* out, int cap) {
   });
   return n;
 }
+// pieces of `nr` ranges packed one after another: (range, first block, count, launch, blocks before it)
+int cuts(const long long* blocks, int nr, long long limit, long long* out, int cap) {
+  int n = 0;
+  int64_t used = 0, launch = 0;
+  for (int r = 0; r < nr; ++r)
+    gscf::cut_blocks(blocks[r], limit, used, [&](int64_t first, int64_t count, bool fresh) {
+      launch += fresh;
+      if (n < cap) {
+        const long long row[5] = {r, first, count, launch, used};
+        for (int k = 0; k < 5; ++k) out[5 * n + k] = row[k];
+      }
+      ++n;
+    });
+  return n;
+}
 }
 """
 
@@ -35,6 +50,7 @@ def limits(tmp_path_factory):
     lib = ctypes.CDLL(str(d / "shim.so"))
     lib.blocks.restype = ctypes.c_longlong
     lib.slices.argtypes = [ctypes.c_longlong, ctypes.c_longlong, ctypes.c_void_p, ctypes.c_int]
+    lib.cuts.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_longlong, ctypes.c_void_p, ctypes.c_int]
     return lib
 
 
@@ -61,3 +77,24 @@ def test_slices_cover_every_entry_once(limits, total, limit):
         assert begin == at and 0 < count <= limit
         at += count
     assert at == total and len(got) == -(-total // limit)
+
+
+@pytest.mark.parametrize("blocks,limit", [([5], 10), ([10], 10), ([11], 10), ([3, 4, 3], 10), ([3, 4, 4], 10),
+                                          ([0, 25, 0, 1], 10), ([7, 30, 2], 1), ([], 10),
+                                          # contracted s pairs of 181 hydrogens, 8 tasks a block
+                                          ([16471 * 16472 // 2 // 8 + 1, 40], (2 ** 32 - 1) // 256)])
+def test_cuts_fill_launches_in_order(limits, blocks, limit):
+    """Every block of every range lies in one launch, at the next free place
+    of it, and only the last launch is not full."""
+    arr = (ctypes.c_longlong * max(1, len(blocks)))(*blocks)
+    out = (ctypes.c_longlong * (5 * 256))()
+    n = limits.cuts(arr, len(blocks), limit, out, 256)
+    assert n <= 256
+    place, done = 0, [0] * len(blocks)
+    for i in range(n):
+        r, first, count, launch, used = out[5 * i:5 * i + 5]
+        assert first == done[r] and count > 0 and used + count <= limit
+        assert launch * limit + used == place
+        done[r] += count
+        place += count
+    assert done == list(blocks)
