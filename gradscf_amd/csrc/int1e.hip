@@ -10,6 +10,7 @@
 #include <algorithm>
 
 #include "gscf_device.h"
+#include "launch_limits.h"
 
 namespace gscf {
 
@@ -647,8 +648,10 @@ void launch_int1e_class(int la, int lb, bool sph, const Pair* pairs, int npairs,
                         const ShellXYZ* shells, const int* shell_ao, const double* nuclei, const MolInfo* mols,
                         double* s, double* t, double* v, hipStream_t st) {
   if (npairs <= 0) return;
-  Int1eArgs a{pairs, prims, shells, shell_ao, nuclei, npairs, mols, s, t, v};
-  const dim3 grid((npairs + 3) / 4), block(256);
+  // (four pairs a workgroup)
+  for_slices(npairs, 4 * grid_blocks(256), [&](int64_t first, int64_t count) {
+    Int1eArgs a{pairs + first, prims, shells, shell_ao, nuclei, (int)count, mols, s, t, v};
+    const dim3 grid((unsigned)((count + 3) / 4)), block(256);
 #define L1E(A, B)                                                                      \
   if (la == A && lb == B) {                                                            \
     if (sph && A == 2)                                                                 \
@@ -657,8 +660,9 @@ void launch_int1e_class(int la, int lb, bool sph, const Pair* pairs, int npairs,
       hipLaunchKernelGGL((int1e_kernel<A, B, false>), grid, block, 0, st, a);          \
     return;                                                                            \
   }
-  L1E(0, 0) L1E(1, 0) L1E(1, 1) L1E(2, 0) L1E(2, 1) L1E(2, 2)
+    L1E(0, 0) L1E(1, 0) L1E(1, 1) L1E(2, 0) L1E(2, 1) L1E(2, 2)
 #undef L1E
+  });
 }
 
 }  // namespace gscf

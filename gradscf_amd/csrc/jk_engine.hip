@@ -702,9 +702,9 @@ __global__ __launch_bounds__(64 * kPartReduceWaves) void kpart_reduce_kernel(con
                                                             const int* __restrict__ row_mol,
                                                             const int64_t* __restrict__ cinv_off,
                                                             const int* __restrict__ cinv, int64_t ncc_tot,
-                                                            int atomic, double* __restrict__ kp) {
+                                                            int atomic, int64_t row0, double* __restrict__ kp) {
   __shared__ double sums[kPartReduceWaves][64];
-  const int64_t R = blockIdx.x;
+  const int64_t R = row0 + blockIdx.x;
   const int bt = blockIdx.z;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = kPartReduceWaves;
   const int col = blockIdx.y * 64 + lane;
@@ -2812,12 +2812,16 @@ static void jk_build(PlanData& P, const double* density, int nb, double* out, in
       P.ev_used += 2;
     }
   }
+  auto reduce_rows = [&](const int64_t* rp, const int64_t* ent, int nd, int atomic, hipStream_t st) {
+    for_slices(S.nrows, grid_blocks(64 * kPartReduceWaves), [&](int64_t row0, int64_t rows) {
+      hipLaunchKernelGGL(kpart_reduce_kernel, dim3((unsigned)rows, (unsigned)((S.nc_max + 63) / 64), (unsigned)nd),
+                         dim3(64 * kPartReduceWaves), 0, st, W.part, S.part_total, rp, ent, S.d_row_dst, S.d_row_n,
+                         S.d_row_mol, S.d_cinv_off, S.d_cinv, P.ncc_tot, atomic, row0, W.kp);
+    });
+  };
   if (lane_reduce)
     for (size_t l = 0; l < P.lane_classes.size(); ++l)
-      hipLaunchKernelGGL(kpart_reduce_kernel, dim3((unsigned)S.nrows, (unsigned)((S.nc_max + 63) / 64),
-                         (unsigned)nbd), dim3(64 * kPartReduceWaves), 0, l == 0 ? s : P.side[l - 1], W.part, S.part_total,
-                         P.d_lane_krp[l], P.d_lane_kent[l], S.d_row_dst, S.d_row_n, S.d_row_mol, S.d_cinv_off,
-                         S.d_cinv, P.ncc_tot, 1, W.kp);
+      reduce_rows(P.d_lane_krp[l], P.d_lane_kent[l], nbd, 1, l == 0 ? s : P.side[l - 1]);
   if (fork) {
     for (size_t l = 0; l < P.side.size(); ++l) {
       HIP_OK(hipEventRecord(P.join_ev[l], P.side[l]));
@@ -2827,9 +2831,7 @@ static void jk_build(PlanData& P, const double* density, int nb, double* out, in
   if (S.part_total > 0) {
     const int nbd_k = with_k ? nbd : nb;
     if (with_k && (psums & 1) && !lane_reduce)
-      hipLaunchKernelGGL(kpart_reduce_kernel, dim3((unsigned)S.nrows, (unsigned)((S.nc_max + 63) / 64),
-                         (unsigned)nbd_k), dim3(64 * kPartReduceWaves), 0, s, W.part, S.part_total, S.d_krp, S.d_kent,
-                         S.d_row_dst, S.d_row_n, S.d_row_mol, S.d_cinv_off, S.d_cinv, P.ncc_tot, 0, W.kp);
+      reduce_rows(S.d_krp, S.d_kent, nbd_k, 0, s);
     if (with_j && (psums & 2))
       hipLaunchKernelGGL(jpart_reduce_kernel, dim3((unsigned)S.pairs.size(), (unsigned)nb), dim3(64), 0, s,
                          W.part, S.part_total, S.d_jrp, S.d_jent, S.d_pairs, S.d_shells, P.d_molinfo,

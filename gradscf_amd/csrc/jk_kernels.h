@@ -19,6 +19,7 @@
 
 #include "gscf_device.h"
 #include "gscf_args.h"
+#include "launch_limits.h"
 
 namespace gscf {
 
@@ -1467,8 +1468,14 @@ void launch_schwarz_t(const SchwarzArgs& a, int np, hipStream_t s) {
   const size_t blk = sizeof(double) * K::NBRA * K::NBRA;
   int T = 256 / (K::SPLIT * Sb * Sk);
   while (T > 1 && T * blk > 48 * 1024) --T;
-  hipLaunchKernelGGL((schwarz_kernel<LA, LB>), dim3((unsigned)((a.npairs + T - 1) / T)), dim3(256),
-                     T * (blk + 2 * sizeof(double)), s, a, Sb * Sk, Sk, T);
+  for_slices(a.npairs, T * grid_blocks(256), [&](int64_t first, int64_t count) {
+    SchwarzArgs p = a;
+    p.pairs += first;
+    p.q += 2 * first;
+    p.npairs = (int)count;
+    hipLaunchKernelGGL((schwarz_kernel<LA, LB>), dim3((unsigned)((count + T - 1) / T)), dim3(256),
+                       T * (blk + 2 * sizeof(double)), s, p, Sb * Sk, Sk, T);
+  });
 }
 
 // Largest r with r (r + 1) / 2 <= idx.

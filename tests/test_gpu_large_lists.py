@@ -72,3 +72,29 @@ def test_auxiliary_integrals_past_one_launch():
     whole = three(range(naux))
     assert torch.equal(whole[:part], three(range(part)))
     assert torch.equal(whole[-part:], three(range(naux - part, naux)))
+
+
+def test_one_electron_matrices_past_one_launch():
+    """11700 distant s functions: 6.8e7 pairs, one wavefront each."""
+    import torch
+    from gradscf_amd.jk import DirectJKPlan
+    n, a = 11700, 0.4
+    grid = np.stack(np.unravel_index(np.arange(n), (23, 23, 23)), -1) * 60.0
+    atm = np.zeros((n, 6), np.int32)
+    atm[0, 0] = 1
+    atm[:, 1] = 20 + 3 * np.arange(n)
+    atm[:, 2] = 1
+    env = np.concatenate([np.zeros(20), grid.ravel(), [a, (2 * a / np.pi) ** 0.75 * (4 * np.pi) ** 0.5]])
+    bas = np.zeros((n, 8), np.int32)
+    bas[:, 0] = np.arange(n)
+    bas[:, 2:4] = 1
+    bas[:, 5:7] = len(env) - 2, len(env) - 1
+    plan = DirectJKPlan(atm, bas, env, cart=True, cutoff=1e3)
+    s, t, v = plan.int1e()
+    dist = torch.as_tensor(np.sqrt((grid ** 2).sum(-1)), device="cuda")
+    nuc = -torch.erf((2 * a) ** 0.5 * dist) / dist
+    nuc[0] = -2 * (2 * a / np.pi) ** 0.5
+    # a few rounding errors of the (diagonal) value; all else is exactly zero
+    for m, ref in ((s, torch.ones_like(nuc)), (t, torch.full_like(nuc, 1.5 * a)), (v, nuc)):
+        assert float((m.diagonal() - ref).abs().max()) < 1e-13
+        assert int(torch.count_nonzero(m)) == n
