@@ -455,7 +455,57 @@ struct PlanData {
   std::vector<hipStream_t> side;
   hipEvent_t fork_ev = nullptr;
   std::vector<hipEvent_t> join_ev;
+  std::mutex side_mu;  // held by a call from its fork to its join (StreamFork)
   std::vector<std::vector<int>> lane_classes;  // class indices per stream (0 = caller's)
+};
+
+// One call's use of the plan's side streams, from the fork (construction) to
+// the join.  Calls that share no workspace (an allocation-free build beside a
+// derivative call) may run on two threads: the lock keeps one's records of the
+// shared events out of the other's fork and join.  Where the side streams
+// belong to a capture that the caller's stream has no part in, the call keeps
+// to its own stream (lanes() == 1) instead of ending up in that graph.
+// (Streams of their own for the derivative calls would share nothing, but a
+// process has four hardware queues: the basis gradient of (H2O)3 cc-pVDZ took
+// 966 us on them, 842 us on these.)
+class StreamFork {
+ public:
+  StreamFork(PlanData& plan, hipStream_t stream, bool wanted = true)
+      : P(plan), s(stream), lock(plan.side_mu, std::defer_lock) {
+    if (!wanted || P.side.empty()) return;
+    lock.lock();
+    // (the side streams are forked together: one stands for all)
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    unsigned long long id = 0, own = 0;
+    HIP_OK(hipStreamGetCaptureInfo(P.side[0], &st, &id));
+    if (st != hipStreamCaptureStatusNone) {
+      if (s) HIP_OK(hipStreamGetCaptureInfo(s, &st, &own));
+      if (!s || st != hipStreamCaptureStatusActive || own != id) {
+        lock.unlock();
+        return;
+      }
+    }
+    HIP_OK(hipEventRecord(P.fork_ev, s));
+    for (hipStream_t side : P.side) HIP_OK(hipStreamWaitEvent(side, P.fork_ev, 0));
+    on = true;
+  }
+  int lanes() const { return on ? (int)P.side.size() + 1 : 1; }
+  hipStream_t lane(int l) const { return l == 0 ? s : P.side[l - 1]; }  // lane 0: the caller's stream
+  void join() {
+    if (!on) return;
+    for (size_t l = 0; l < P.side.size(); ++l) {
+      HIP_OK(hipEventRecord(P.join_ev[l], P.side[l]));
+      HIP_OK(hipStreamWaitEvent(s, P.join_ev[l], 0));
+    }
+    on = false;
+    lock.unlock();
+  }
+
+ private:
+  PlanData& P;
+  hipStream_t s;
+  std::unique_lock<std::mutex> lock;
+  bool on = false;
 };
 
 // Per-class launchers, one translation unit each (jk_class.hip).
@@ -2618,21 +2668,18 @@ static void jk_build(PlanData& P, const double* density, int nb, double* out, in
   // Class launches: in list order on the caller's stream while profiling (so
   // that the per-class events time one kernel each), otherwise spread over
   // the plan's streams, forked from and joined back into the caller's stream.
-  const bool fork = !P.prof && !P.side.empty();
+  StreamFork streams(P, s, !P.prof);
+  const bool fork = streams.lanes() > 1;
   // with several streams each folds the exchange-row slabs of its own
   // classes right after them (device-scope adds into K), overlapping the
   // other streams' class kernels; otherwise one reduction after the join
   const int psums = (det || !W.part) ? 0 : P.options.partial_sums;
   const bool lane_reduce = fork && with_k && (psums & 1) && S.part_total > 0 &&
                            P.d_lane_krp.size() == P.lane_classes.size();
-  if (fork) {
-    HIP_OK(hipEventRecord(P.fork_ev, s));
-    for (hipStream_t st : P.side) HIP_OK(hipStreamWaitEvent(st, P.fork_ev, 0));
-  }
   std::vector<std::pair<int, hipStream_t>> launches;
   if (fork) {
     for (size_t l = 0; l < P.lane_classes.size(); ++l)
-      for (int ci : P.lane_classes[l]) launches.push_back({ci, l == 0 ? s : P.side[l - 1]});
+      for (int ci : P.lane_classes[l]) launches.push_back({ci, streams.lane((int)l)});
   } else {
     for (size_t ci = 0; ci < S.classes.size(); ++ci) launches.push_back({(int)ci, s});
   }
@@ -2821,13 +2868,8 @@ static void jk_build(PlanData& P, const double* density, int nb, double* out, in
   };
   if (lane_reduce)
     for (size_t l = 0; l < P.lane_classes.size(); ++l)
-      reduce_rows(P.d_lane_krp[l], P.d_lane_kent[l], nbd, 1, l == 0 ? s : P.side[l - 1]);
-  if (fork) {
-    for (size_t l = 0; l < P.side.size(); ++l) {
-      HIP_OK(hipEventRecord(P.join_ev[l], P.side[l]));
-      HIP_OK(hipStreamWaitEvent(s, P.join_ev[l], 0));
-    }
-  }
+      reduce_rows(P.d_lane_krp[l], P.d_lane_kent[l], nbd, 1, streams.lane((int)l));
+  streams.join();
   if (S.part_total > 0) {
     const int nbd_k = with_k ? nbd : nb;
     if (with_k && (psums & 1) && !lane_reduce)
@@ -3011,22 +3053,14 @@ static void int1e_gradient(PlanData& P, const double* dens, const double* wdens,
   static const int pl[kNumPairClasses][2] = {{0, 0}, {1, 0}, {1, 1}, {2, 0}, {2, 1}, {2, 2}};
   // the pair classes in turn over the caller's stream and the plan's side
   // streams: independent kernels of 17 to 57 us, 0.18 ms one after another;
-  // matrices and gradient of (H2O)16 cc-pVDZ 0.34 -> 0.30 ms.  (The matrices keep one stream: they use nothing of
-  // the plan that a second thread's call would share.)
-  if (!P.side.empty()) {
-    HIP_OK(hipEventRecord(P.fork_ev, s));
-    for (hipStream_t st : P.side) HIP_OK(hipStreamWaitEvent(st, P.fork_ev, 0));
-  }
+  // matrices and gradient of (H2O)16 cc-pVDZ 0.34 -> 0.30 ms.
+  StreamFork streams(P, s);
   for (int c = 0; c < kNumPairClasses; ++c) {
     const int b = P.p1e_begin[c], e = P.p1e_begin[c + 1];
-    const size_t l = (size_t)c % (P.side.size() + 1);
     launch_grad1e_class(pl[c][0], pl[c][1], P.d_pairs1e + b, e - b, P.d_prims, P.d_shells, P.d_seg_atom, P.d_nuclei,
-                        P.d_molinfo, P.d_dc, P.d_dc + ncc, P.natm, grad, l == 0 ? s : P.side[l - 1]);
+                        P.d_molinfo, P.d_dc, P.d_dc + ncc, P.natm, grad, streams.lane(c % streams.lanes()));
   }
-  for (size_t l = 0; l < P.side.size(); ++l) {
-    HIP_OK(hipEventRecord(P.join_ev[l], P.side[l]));
-    HIP_OK(hipStreamWaitEvent(s, P.join_ev[l], 0));
-  }
+  streams.join();
   HIP_OK(hipGetLastError());
 }
 
@@ -3036,25 +3070,18 @@ static void int1e_gradient(PlanData& P, const double* dens, const double* wdens,
 // result), and one after another their tails left most of the chip idle.
 template <class F>
 static void for_classes_on_streams(PlanData& P, const PairSet& S, hipStream_t s, F&& launch) {
-  const int ns = (int)P.side.size() + 1;
   std::vector<int> order(S.classes.size());
   for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
   std::stable_sort(order.begin(), order.end(),
                    [&](int x, int y) { return S.classes[x].cost > S.classes[y].cost; });
-  if (ns > 1) {
-    HIP_OK(hipEventRecord(P.fork_ev, s));
-    for (hipStream_t st : P.side) HIP_OK(hipStreamWaitEvent(st, P.fork_ev, 0));
-  }
-  std::vector<double> load(ns, 0.0);
+  StreamFork streams(P, s);
+  std::vector<double> load(streams.lanes(), 0.0);
   for (int ci : order) {
     const int l = (int)(std::min_element(load.begin(), load.end()) - load.begin());
     load[l] += S.classes[ci].cost;
-    launch(S.classes[ci], l == 0 ? s : P.side[l - 1]);
+    launch(S.classes[ci], streams.lane(l));
   }
-  for (size_t l = 0; l < P.side.size(); ++l) {
-    HIP_OK(hipEventRecord(P.join_ev[l], P.side[l]));
-    HIP_OK(hipStreamWaitEvent(s, P.join_ev[l], 0));
-  }
+  streams.join();
 }
 
 static void geometry_vjp(PlanData& P, const double* dens, const double* cj, const double* ck, double* grad,

@@ -243,7 +243,12 @@ int gscf_jk_build(gscf_plan* plan, const double* density, int32_t nb, double* ou
  * flushed by atomics (no partial slabs), so results equal gscf_jk_build's to
  * FP64 rounding.  Calls on one GPU share that array: calls that overlap on one
  * GPU (different streams or threads) race and must be serialised by the
- * caller.  The plan must not be profiling.  Without GSCF_FLAG_NO_VALIDATE the
+ * caller.  It uses nothing of the plan's workspace: gscf_int1e_gradient,
+ * gscf_jk_geometry_vjp, gscf_jk_param_vjp, gscf_int1e and gscf_eri_blocks of
+ * the same plan may run beside it, on another stream or thread, also while one
+ * of the two is under capture.  (Calls that do share the workspace, two
+ * gscf_jk_build or two derivative calls of one plan, must be serialised.)
+ * The plan must not be profiling.  Without GSCF_FLAG_NO_VALIDATE the
  * finite-density check synchronises the stream (pinned host flag, no
  * allocation). */
 int gscf_jk_build_noalloc(gscf_plan* plan, const double* density, int32_t nb, double* out,
