@@ -39,9 +39,9 @@ __global__ __launch_bounds__(256) void grad_kernel(GradArgs a) {
   for (int i = threadIdx.x; i < 3 * a.natm; i += blockDim.x) gl[i] = 0.0;
   __syncthreads();
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t item = t / NKET;
+  const int64_t item = a.item0 + t / NKET;
   if (item < a.nitems) {
-    const int kc = (int)(t - item * NKET);
+    const int kc = (int)(t % NKET);
     const int ic = kc / ND, id = kc - (kc / ND) * ND;
     int64_t g;
     const PrimSlice sl = map_item(a.tasks, a.ntasks, item, g);
@@ -184,11 +184,13 @@ __global__ __launch_bounds__(256) void grad_kernel(GradArgs a) {
 template <int LA, int LB, int LC, int LD>
 void launch_grad_t(const GradArgs& a, hipStream_t s) {
   constexpr int NKET = ncart(LC) * ncart(LD);
-  if (a.nitems <= 0) return;
-  const int64_t threads = a.nitems * NKET;
-  const int64_t blocks = (threads + 255) / 256;
-  hipLaunchKernelGGL((grad_kernel<LA, LB, LC, LD>), dim3((unsigned)blocks), dim3(256),
-                     sizeof(double) * 3 * a.natm, s, a);
+  for_slices(a.nitems, grid_items(NKET), [&](int64_t first, int64_t count) {
+    GradArgs p = a;
+    p.item0 = first;
+    p.nitems = first + count;
+    hipLaunchKernelGGL((grad_kernel<LA, LB, LC, LD>), dim3((unsigned)((count * NKET + 255) / 256)), dim3(256),
+                       sizeof(double) * 3 * a.natm, s, p);
+  });
 }
 
 }  // namespace gscf

@@ -91,6 +91,7 @@ struct JKArgs {
   const SubTask* tasks;
   int ntasks;
   int64_t nitems;
+  int64_t item0;        // first item of this launch (set by the launcher, with nitems its end)
   const double* dens;   // [nbd][sum_m n_m^2] Cartesian densities
   double* jp;           // [nbj][...] partial J (J = Jp + Jp^T)
   double* kp;           // [nbd][...] partial K
@@ -216,6 +217,7 @@ struct ParamArgs {
   const SubTask* tasks;
   int ntasks;
   int64_t nitems;
+  int64_t item0;         // first item of this launch (set by the launcher, with nitems its end)
   const double* dens;
   const double* cj;
   const double* ck;
@@ -346,6 +348,7 @@ struct GradArgs {
   const SubTask* tasks;
   int ntasks;
   int64_t nitems;
+  int64_t item0;         // first item of this launch (set by the launcher, with nitems its end)
   const double* dens;    // Cartesian D, cot_J, cot_K (per molecule n x n); cot may be null
   const double* cj;
   const double* ck;

@@ -1090,7 +1090,13 @@ __global__ void fixed_to_double_kernel(double* __restrict__ p, int64_t count, in
   p[i] = (double)v * scale[2 * m + 1];
 }
 
-static unsigned nblocks(size_t count) { return (unsigned)((count + 255) / 256); }
+// Workgroups of 256 lanes for one lane per entry.  (A larger grid would leave
+// entries out without an error.)
+static unsigned nblocks(size_t count) {
+  if ((int64_t)count > grid_items(1))
+    throw Internal("one launch cannot cover " + std::to_string(count) + " matrix elements");
+  return (unsigned)((count + 255) / 256);
+}
 
 // env_grad[exponent slot] += gexp; env_grad[coefficient slot] += fsp * gcoef
 // (the exponent slot is shared by the contraction columns of a shell).
@@ -1950,7 +1956,7 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
                  o_groups = work.add(run_groups), o_sort = work.add(sort_classes);
     work.send(s);
     // (a launch that fails ends the plan before the next one reads the list)
-    for_slices(S.nquartets, grid_blocks(256) * 256, [&](int64_t first, int64_t count) {
+    for_slices(S.nquartets, grid_items(1), [&](int64_t first, int64_t count) {
       hipLaunchKernelGGL(expand_kernel, dim3(nblocks((size_t)count)), dim3(256), 0, s, work.at<ExpandTask>(o_expand),
                          (int)expand.size(), first, count, work.at<int64_t>(o_qoff), work.at<int>(o_order),
                          work.at<int2>(o_groups), S.d_quartets);

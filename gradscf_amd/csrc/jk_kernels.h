@@ -336,7 +336,7 @@ __device__ __forceinline__ void acc_flush(double* dst, const double* src) {
 template <int LA, int LB, int LC, int LD, bool DET = false>
 __global__ __launch_bounds__(256) void jk_full_kernel(JKArgs a) {
   using K = Class<LA, LB, LC, LD>;
-  const int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t item = a.item0 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (item >= a.nitems) return;
   int64_t g;
   const PrimSlice sl = map_item(a.tasks, a.ntasks, item, g);
@@ -479,9 +479,9 @@ template <int LA, int LB, int LC, int LD, bool DET = false>
 __global__ __launch_bounds__(256) void jk_split_kernel(JKArgs a) {
   using K = Class<LA, LB, LC, LD>;
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t item = t / K::SPLIT;
+  const int64_t item = a.item0 + t / K::SPLIT;
   if (item >= a.nitems) return;
-  const int kc = (int)(t - item * K::SPLIT);
+  const int kc = (int)(t % K::SPLIT);
   const int ic = kc / K::ND, id = kc - (kc / K::ND) * K::ND;
   int64_t g;
   const PrimSlice sl = map_item(a.tasks, a.ntasks, item, g);
@@ -1578,29 +1578,35 @@ __global__ __launch_bounds__(256) void eri_kernel(EriArgs a) {
 template <int LA, int LB, int LC, int LD>
 void launch_jk_t(const JKArgs& a, hipStream_t s) {
   using K = Class<LA, LB, LC, LD>;
-  if (a.nitems <= 0) return;
-  const int64_t threads = a.nitems * K::SPLIT;
-  const int64_t blocks = (threads + 255) / 256;
-  if constexpr (K::kSplit) {
-    if (a.det_scale)
-      hipLaunchKernelGGL((jk_split_kernel<LA, LB, LC, LD, true>), dim3((unsigned)blocks), dim3(256), 0, s, a);
-    else
-      hipLaunchKernelGGL((jk_split_kernel<LA, LB, LC, LD>), dim3((unsigned)blocks), dim3(256), 0, s, a);
-  } else {
-    if (a.det_scale)
-      hipLaunchKernelGGL((jk_full_kernel<LA, LB, LC, LD, true>), dim3((unsigned)blocks), dim3(256), 0, s, a);
-    else
-      hipLaunchKernelGGL((jk_full_kernel<LA, LB, LC, LD>), dim3((unsigned)blocks), dim3(256), 0, s, a);
-  }
+  for_slices(a.nitems, grid_items(K::SPLIT), [&](int64_t first, int64_t count) {
+    JKArgs p = a;
+    p.item0 = first;
+    p.nitems = first + count;
+    const dim3 grid((unsigned)((count * K::SPLIT + 255) / 256)), block(256);
+    if constexpr (K::kSplit) {
+      if (a.det_scale)
+        hipLaunchKernelGGL((jk_split_kernel<LA, LB, LC, LD, true>), grid, block, 0, s, p);
+      else
+        hipLaunchKernelGGL((jk_split_kernel<LA, LB, LC, LD>), grid, block, 0, s, p);
+    } else {
+      if (a.det_scale)
+        hipLaunchKernelGGL((jk_full_kernel<LA, LB, LC, LD, true>), grid, block, 0, s, p);
+      else
+        hipLaunchKernelGGL((jk_full_kernel<LA, LB, LC, LD>), grid, block, 0, s, p);
+    }
+  });
 }
 
 template <int LA, int LB, int LC, int LD>
 void launch_blocks_t(const BlockArgs& a, hipStream_t s) {
   using K = Class<LA, LB, LC, LD>;
-  if (a.ntasks <= 0) return;
-  const int64_t threads = a.ntasks * K::NKET;
-  const int64_t blocks = (threads + 255) / 256;
-  hipLaunchKernelGGL((blocks_kernel<LA, LB, LC, LD>), dim3((unsigned)blocks), dim3(256), 0, s, a);
+  for_slices(a.ntasks, grid_items(K::NKET), [&](int64_t first, int64_t count) {
+    BlockArgs p = a;
+    p.tasks += first;
+    p.ntasks = count;
+    hipLaunchKernelGGL((blocks_kernel<LA, LB, LC, LD>), dim3((unsigned)((count * K::NKET + 255) / 256)), dim3(256), 0,
+                       s, p);
+  });
 }
 
 // Dynamic LDS above 64 KB (one-density launches of wide molecules) is
@@ -1622,12 +1628,15 @@ void launch_eri_t(const EriArgs& a, int blocks, size_t lds, hipStream_t s) {
 
 template <int LA, int LB, int LC, int LD, int CA, int CB, int CC, int CD>
 void launch_jk_bra_t(const BraArgs& a, size_t lds_bytes, hipStream_t s) {
-  if (a.nchunks <= 0) return;
-  const dim3 block(a.threads), grid((unsigned)a.nchunks);
-#define GSCF_BRA_LAUNCH(...)                                  \
-  do {                                                        \
-    request_lds(__VA_ARGS__, lds_bytes);                      \
-    hipLaunchKernelGGL((__VA_ARGS__), grid, block, lds_bytes, s, a); \
+#define GSCF_BRA_LAUNCH(...)                                                                               \
+  do {                                                                                                     \
+    request_lds(__VA_ARGS__, lds_bytes);                                                                   \
+    for_slices(a.nchunks, grid_blocks(a.threads), [&](int64_t first, int64_t count) {                      \
+      BraArgs p = a;                                                                                       \
+      p.chunks += first;                                                                                   \
+      p.nchunks = (int)count;                                                                              \
+      hipLaunchKernelGGL((__VA_ARGS__), dim3((unsigned)count), dim3(a.threads), lds_bytes, s, p);          \
+    });                                                                                                    \
   } while (0)
   // in-core integrals (FP64 blocks; segmented patterns only)
   if constexpr (CA * CB * CC * CD == 1) {

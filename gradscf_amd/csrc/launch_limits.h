@@ -1,8 +1,10 @@
 // Sizes of one launch (host code, no HIP headers).
 //
-// A dispatch counts its work items per dimension in 32 bits: a launch with
-// gridDim.x * blockDim.x of 2^32 or more is refused.  Launches whose size
-// grows with the molecule are cut into slices below that.
+// A dispatch counts its work items per dimension in 32 bits.  A launch with
+// gridDim.x * blockDim.x of 2^32 or more reports no error and runs only part of
+// its workgroups (seen with packed integrals of 220 hydrogens, 1.2e10 lanes:
+// most of the result was never written).  Launches whose size grows with the
+// molecule are cut into slices below that.
 #pragma once
 #include <algorithm>
 #include <cstdint>
@@ -10,10 +12,12 @@
 namespace gscf {
 
 constexpr int64_t kGridThreads = (int64_t(1) << 32) - 1;
-constexpr int64_t kGridYZ = 65535;  // workgroups along y or z
 
 // Workgroups of `threads` lanes one launch may have along x.
 constexpr int64_t grid_blocks(int threads) { return kGridThreads / threads; }
+
+// Items of `lanes` lanes each that one launch of 256-lane workgroups may have.
+constexpr int64_t grid_items(int lanes) { return grid_blocks(256) * 256 / lanes; }
 
 // launch(begin, count) over consecutive slices of [0, total), at most `limit`
 // entries each.

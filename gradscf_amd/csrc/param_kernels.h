@@ -36,9 +36,9 @@ __global__ __launch_bounds__(256) void param_kernel(ParamArgs a) {
   for (int i = threadIdx.x; i < 2 * a.nprim; i += blockDim.x) pl[i] = 0.0;
   __syncthreads();
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t item = t / NKET;
+  const int64_t item = a.item0 + t / NKET;
   if (item < a.nitems) {
-    const int kc = (int)(t - item * NKET);
+    const int kc = (int)(t % NKET);
     const int ic = kc / ND, id = kc - (kc / ND) * ND;
     int64_t g;
     const PrimSlice sl = map_item(a.tasks, a.ntasks, item, g);
@@ -195,11 +195,13 @@ __global__ __launch_bounds__(256) void param_kernel(ParamArgs a) {
 template <int LA, int LB, int LC, int LD>
 void launch_param_t(const ParamArgs& a, hipStream_t s) {
   constexpr int NKET = ncart(LC) * ncart(LD);
-  if (a.nitems <= 0) return;
-  const int64_t threads = a.nitems * NKET;
-  const int64_t blocks = (threads + 255) / 256;
-  hipLaunchKernelGGL((param_kernel<LA, LB, LC, LD>), dim3((unsigned)blocks), dim3(256),
-                     sizeof(double) * 2 * a.nprim, s, a);
+  for_slices(a.nitems, grid_items(NKET), [&](int64_t first, int64_t count) {
+    ParamArgs p = a;
+    p.item0 = first;
+    p.nitems = first + count;
+    hipLaunchKernelGGL((param_kernel<LA, LB, LC, LD>), dim3((unsigned)((count * NKET + 255) / 256)), dim3(256),
+                       sizeof(double) * 2 * a.nprim, s, p);
+  });
 }
 
 }  // namespace gscf

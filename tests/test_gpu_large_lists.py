@@ -98,3 +98,43 @@ def test_one_electron_matrices_past_one_launch():
     for m, ref in ((s, torch.ones_like(nuc)), (t, torch.full_like(nuc, 1.5 * a)), (v, nuc)):
         assert float((m.diagonal() - ref).abs().max()) < 1e-13
         assert int(torch.count_nonzero(m)) == n
+
+
+def _p_shells(n, exponent, coords):
+    """Tables of n single-primitive p shells with one exponent."""
+    atm = np.zeros((len(coords), 6), np.int32)
+    atm[:, 0] = 1
+    atm[:, 1] = 20 + 3 * np.arange(len(coords))
+    atm[:, 2] = 1
+    env = np.concatenate([np.zeros(20), coords.ravel(), [exponent, 1.0]])
+    bas = np.zeros((n, 8), np.int32)
+    bas[:, 0] = np.arange(n) % len(coords)
+    bas[:, 1:4] = 1
+    bas[:, 5:7] = len(env) - 2, len(env) - 1
+    return atm, bas, env
+
+
+def test_derivatives_past_one_launch():
+    """(pp|pp) derivatives of 260 p shells: 5.8e8 quartets of nine ket
+    components each, against central differences of J and K."""
+    import torch
+    from gradscf_amd.jk import DirectJKPlan
+    n, alpha, h = 260, 0.8, 1e-4
+    rng = np.random.default_rng(5)
+    grid = np.stack(np.unravel_index(np.arange(260), (7, 7, 7)), -1) * 1.2 + rng.uniform(-0.2, 0.2, (260, 3))
+    d, cj, ck = (torch.as_tensor(x, device="cuda") for x in systems.random_density(3 * n, nb=3, seed=12))
+    plan = DirectJKPlan(*_p_shells(n, alpha, grid), cart=True, cutoff=0.0)
+    assert plan.info["nquartets"] * 9 > 2 ** 32
+
+    def energy(exponent, coords):
+        j, k = DirectJKPlan(*_p_shells(n, exponent, coords), cart=True, cutoff=0.0).jk(d)
+        return float((cj * j).sum() + (ck * k).sum())
+
+    u = rng.normal(size=grid.shape)
+    grad = plan.jk_geometry_vjp(d, cj, ck).cpu().numpy()
+    slope = (energy(alpha, grid + h * u) - energy(alpha, grid - h * u)) / (2 * h)
+    # central differences: a third derivative times h^2 / 6
+    assert abs((grad * u).sum() - slope) < 1e-5 * np.abs(grad * u).sum()
+    env_grad = plan.jk_param_vjp(d, cj, ck)
+    slope = (energy(alpha + h, grid) - energy(alpha - h, grid)) / (2 * h)
+    assert abs(float(env_grad[-2]) - slope) < 1e-5 * abs(slope)

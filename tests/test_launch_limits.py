@@ -14,6 +14,7 @@ SHIM = r"""
 #include "launch_limits.h"
 extern "C" {
 long long blocks(int threads) { return gscf::grid_blocks(threads); }
+long long items(int lanes) { return gscf::grid_items(lanes); }
 int slices(long long total, long long limit, long long* out, int cap) {
   int n = 0;
   gscf::for_slices(total, limit, [&](int64_t b, int64_t c) {
@@ -48,7 +49,7 @@ def limits(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", f"-I{CSRC}", "-o", str(d / "shim.so"),
                     str(d / "shim.cc")], check=True)
     lib = ctypes.CDLL(str(d / "shim.so"))
-    lib.blocks.restype = ctypes.c_longlong
+    lib.blocks.restype = lib.items.restype = ctypes.c_longlong
     lib.slices.argtypes = [ctypes.c_longlong, ctypes.c_longlong, ctypes.c_void_p, ctypes.c_int]
     lib.cuts.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_longlong, ctypes.c_void_p, ctypes.c_int]
     return lib
@@ -65,6 +66,12 @@ def _slices(lib, total, limit):
 def test_grid_stays_below_the_work_item_limit(limits, threads):
     n = limits.blocks(threads)
     assert n * threads < 2 ** 32 <= (n + 1) * threads
+
+
+@pytest.mark.parametrize("lanes", [1, 3, 9, 18, 36])
+def test_items_of_several_lanes_stay_below_the_limit(limits, lanes):
+    n = limits.items(lanes)
+    assert -(-n * lanes // 256) * 256 < 2 ** 32 <= (n + 1) * lanes + 512
 
 
 @pytest.mark.parametrize("total,limit", [(0, 7), (1, 7), (6, 7), (7, 7), (8, 7), (100, 7), (100, 1),
