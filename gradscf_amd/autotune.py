@@ -80,7 +80,8 @@ def get_options() -> dict:
 
 
 def set_options(**kw) -> None:
-    """Change engine options; plans created afterwards use them."""
+    """Change engine options; plans created afterwards use them (and take
+    balance=1 at its word: every plan is measured, however short its builds)."""
     cur = get_options()
     unknown = set(kw) - set(cur)
     if unknown:

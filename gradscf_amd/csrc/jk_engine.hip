@@ -246,6 +246,7 @@ static void ensure_tuning() {
 // defaults: segmented general contractions (faster on the measured cc-pVDZ
 // workloads; a tuning table may switch it on), four launch streams
 static gscf_options g_options = {0, 4, 1, 0, 0, 1};
+static bool g_options_chosen = false;  // the caller has set them
 constexpr int kMaxMoleculeCartAO = 16384;  // per molecule (32-bit in-molecule offsets)
 constexpr int kMaxStreams = 4;
 
@@ -358,6 +359,7 @@ struct PairSet {
 struct PlanData {
   gscf_class_tuning tuning[kNumQuartetClasses];
   gscf_options options;
+  bool options_chosen = false;  // set by the caller: balance = 1 measures whatever the build's length
   size_t lds_budget = kLdsBudget;  // LDS of a launch over all densities (packing target)
   size_t lds_max = kLdsBudget;     // LDS of a one-density launch (device limit)
   int cart = 1, n = 0, n_cart = 0, nbas = 0, natm = 0;
@@ -1124,6 +1126,7 @@ static void validate_tables(PlanData& P, const int32_t* atm, int natm, const int
   ensure_tuning();
   std::copy(g_tuning, g_tuning + kNumQuartetClasses, P.tuning);
   P.options = g_options;
+  P.options_chosen = g_options_chosen;
   if (nmol < 1 || (nmol > 1 && (!mol_atm || !mol_bas)))
     throw InvalidArgument("A batched plan needs per-molecule atm and bas offsets");
   P.nmol = nmol;
@@ -2911,11 +2914,14 @@ static void jk_build(PlanData& P, const double* density, int nb, double* out, in
 // is the identity per molecule (the kernels' work does not depend on the
 // density's values).
 static void balance_lanes(PlanData& P, hipStream_t s) {
-  // Short builds keep the predicted times: two probe builds and their events
-  // take about 1.5 ms, which a spread 5-10 % better repays only over dozens of
-  // builds ((H2O)3 6-31G*, plan and one build: 3.0 ms with probes, 1.4 without).
+  // Short builds keep the predicted times unless the caller asked for measured
+  // ones: two probe builds and their events take 1.4 to 2.6 ms of plan time and
+  // change a build by -2 to +7 % (C4H10 343 us a build with predicted times,
+  // 348 with measured ones, (H2O)8 6-31G* 373 and 375, (H2O)2 cc-pVDZ 246 and
+  // 228), which repays them after a hundred builds if ever.
   constexpr double kProbeUs = 1000.0;
-  if (P.side.empty() || !P.options.balance || P.jk.classes.empty() || predicted_us(P) < kProbeUs) {
+  if (P.side.empty() || !P.options.balance || P.jk.classes.empty() ||
+      (!P.options_chosen && predicted_us(P) < kProbeUs)) {
     assign_lanes(P);
     return;
   }
@@ -3859,6 +3865,7 @@ int gscf_options_set(const gscf_options* o) {
     if (o->deterministic != 0 && o->deterministic != 1) throw InvalidArgument("deterministic must be 0 or 1");
     if (o->balance != 0 && o->balance != 1) throw InvalidArgument("balance must be 0 or 1");
     g_options = *o;
+    g_options_chosen = true;
   });
 }
 

@@ -121,10 +121,10 @@ typedef struct {
                                   0 (default): FP64 atomics, equal to rounding */
   int32_t balance;             /* 1 (default): plan creation times every quartet class of one
                                   build alone (two builds of an identity density, HIP events)
-                                  and spreads the classes over the streams by those times,
-                                  where the plan-time work model predicts class launches of
-                                  over 1 ms; shorter builds, and 0: by the model (no probe
-                                  builds) */
+                                  and spreads the classes over the streams by those times;
+                                  0: by the plan-time work model (no probe builds).  While
+                                  the options have never been set, builds of under 1 ms (by
+                                  the model) are spread by the model too */
 } gscf_options;
 int gscf_options_set(const gscf_options* o);
 int gscf_options_get(gscf_options* o);
