@@ -2961,7 +2961,7 @@ static void balance_lanes(PlanData& P, hipStream_t s) {
   P.ev_used = 0;
   HIP_OK(hipFree(d_dens));
   HIP_OK(hipFree(d_out));
-  for (size_t i = 0; i < t.size(); ++i) P.jk.classes[i].cost = t[i];
+  for (size_t i = 0; i < t.size(); ++i) P.jk.classes[i].cost = 1e3 * t[i];  // microseconds
   assign_lanes(P);
 }
 
