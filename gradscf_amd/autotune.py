@@ -23,6 +23,11 @@ LETTERS = "spdf"
 
 @dataclass(frozen=True)
 class Schedule:
+    """Upper bounds of one class's schedule: a plan takes fewer chunk_items and
+    target_prim where the class would leave the device idle, 512 threads where
+    a launch's LDS leaves one workgroup per compute unit, and ket windows in LDS
+    for one and two Rys roots whatever ket_lds says."""
+
     chunk_items: int = 4096
     bras_max: int = 16
     lds_pack: int = 32 * 1024

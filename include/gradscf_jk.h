@@ -44,18 +44,23 @@ extern "C" {
 typedef struct gscf_plan gscf_plan;
 
 /* Schedule parameters of one canonical quartet class (no counterpart in the
- * reference; set by the autotuner).  Class index c = cb*(cb+1)/2 + ck over
+ * reference; set by the autotuner).  Sizes are upper bounds that a plan lowers
+ * where its class would leave the device idle; no schedule changes results
+ * beyond the order of FP64 additions.  Class index c = cb*(cb+1)/2 + ck over
  * pair classes ss, ps, pp, ds, dp, dd = 0..5 with ck <= cb (0 = ssss ...
  * 20 = dddd).  Plans copy the process-wide table when they are created. */
 typedef struct {
   int32_t chunk_items;  /* lane-items per workgroup before a bra chunk is closed (64..2^20); fewer
-                           where their primitive quartets make a long chunk */
+                           where their primitive quartets make a long chunk or the class has
+                           fewer chunks than the device compute units */
   int32_t bras_max;     /* bra pairs (LDS exchange slots) per chunk (1..256) */
   int32_t lds_pack;     /* LDS bytes the slots of one workgroup may use (1024..65536) */
   int32_t rys_lds;      /* 1: stage the class's Rys table slice in LDS; 0: global table
                            (one or two roots: Boys-moment quadrature instead) */
-  int32_t target_prim;  /* primitive quartets per work item (primitive split), 1..4096 */
-  int32_t threads;      /* workgroup size, 256 or 512 */
+  int32_t target_prim;  /* primitive quartets per work item (primitive split), 1..4096; fewer,
+                           down to 2, where the class has too few items for the device */
+  int32_t threads;      /* workgroup size, 256 or 512; 256 becomes 512 for a launch whose LDS
+                           leaves one workgroup per compute unit */
   int32_t ket_lds;      /* 1: accumulate the ket-side J of each chunk's ket window in LDS;
                            0: only in classes of one or two Rys roots */
 } gscf_class_tuning;
