@@ -1474,12 +1474,13 @@ static double class_cost_us(int la, int lb, int lc, int ld, int pb, int pk, int6
 // bras and kets have np in [npb0, npb1] and [npk0, npk1]: the largest S that
 // leaves `target` primitive quartets per lane, shared between bra and ket so
 // that the longest lane runs the fewest iterations (the bra first on ties).
-static void choose_split(int npb0, int npb1, int npk0, int npk1, int64_t target, SubTask& t) {
+// With bra_only the ket's primitives stay together.
+static void choose_split(int npb0, int npb1, int npk0, int npk1, int64_t target, bool bra_only, SubTask& t) {
   const int64_t want = ((int64_t)npb1 * npk1 + target - 1) / target;
   int64_t rounds = (int64_t)npb1 * npk1;
   t.S = t.Sk = 1;
   for (int S = 2; S <= 64 && S <= want; S *= 2)
-    for (int Sk = 1; Sk <= S; Sk *= 2) {
+    for (int Sk = 1; Sk <= (bra_only ? 1 : S); Sk *= 2) {
       const int Sb = S / Sk;
       if (Sb > npb0 || Sk > npk0) continue;
       const int64_t r = (int64_t)((npb1 + Sb - 1) / Sb) * ((npk1 + Sk - 1) / Sk);
@@ -1676,35 +1677,13 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
           const int wa = ncart_h(qc.la) * (1 + (pb & 1)), wb = ncart_h(qc.lb) * (1 + (pb >> 1));
           const int wc = ncart_h(qc.lc) * (1 + (pk & 1)), wd = ncart_h(qc.ld) * (1 + (pk >> 1));
           const int split = (wa * wb * wc * wd > 36) ? wc * wd : 1;
-          // primitive split and chunk size: the schedule's values, or less
-          // work per lane and per workgroup where the class would otherwise
-          // leave the device idle (kFillLanes, kFillGroups)
-          double lane_work = 0.0;
-          for (const Pending& pd : pend) {
-            const Run &rb = runs[pd.rb], &rk = runs[pd.rk];
-            lane_work += 0.25 * (double)pd.nq * split * (rb.npmin + rb.npmax) * (rk.npmin + rk.npmax);
-          }
-          const int64_t kTargetPrim = std::max<int64_t>(
-              1, std::min<int64_t>(tu.target_prim, (int64_t)std::max(lane_work / kFillLanes, (double)kMinPrim)));
-          int64_t items = 0;
-          for (size_t ti = 0; ti < pend.size(); ++ti) {
-            SubTask& t = qc.tasks[ti];
-            const Run &rb = runs[pend[ti].rb], &rk = runs[pend[ti].rk];
-            choose_split(rb.npmin, rb.npmax, rk.npmin, rk.npmax, kTargetPrim, t);
-            t.item0 = qc.nitems;
-            qc.nitems += (int64_t)t.S * t.nq;
-            items += (int64_t)t.S * t.nq * split;
-          }
-          const int64_t fill_items = (items / kFillGroups + tu.threads - 1) / tu.threads * tu.threads;
-          const int64_t class_items =
-              std::min<int64_t>(tu.chunk_items, std::max<int64_t>(tu.threads, fill_items));
+          // LDS of one bra slot for one density
+          const int rows = wa + wb;
+          // full-block classes stage their chunk's bra primitive pairs in
+          // LDS (kStagedPrim doubles each, kStagedPrimCoef with bra columns)
+          const bool stage = split == 1;
+          const int rec = pb ? kStagedPrimCoef : kStagedPrim;
           if (with_chunks) {
-            // bra-major chunks: consecutive bras of one sub-task, bounded LDS slots and lane-items
-            const int rows = wa + wb;
-            // full-block classes stage their chunk's bra primitive pairs in
-            // LDS (kStagedPrim doubles each, kStagedPrimCoef with bra columns)
-            const bool stage = split == 1;
-            const int rec = pb ? kStagedPrimCoef : kStagedPrim;
             int bra_np_max = 0;
             if (stage)
               for (const Run& r : runs)
@@ -1718,8 +1697,41 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
               for (int m = 0; m < P.nmol; ++m) row_len = std::max(row_len, S.h_cspace[m * 8 + kmask].y);
             }
             qc.row_len = row_len;
-            const size_t per_slot = sizeof(double) * ((size_t)rows * row_len + (size_t)wa * wb * (kJBraCopies + 1) +
-                                                      (size_t)rec * bra_np_max + kBraRecDoubles);
+            qc.per_slot = sizeof(double) * ((size_t)rows * row_len + (size_t)wa * wb * (kJBraCopies + 1) +
+                                            (size_t)rec * bra_np_max + kBraRecDoubles);
+          }
+          // rows that do not fit: the global-atomic kernels, whose lanes add
+          // every slice's terms by themselves.  A slice more is then not a
+          // shorter chain but another set of device atomics: the schedule's
+          // target and the bra's primitives alone (C6H14 6-31G* at lds_limit
+          // 4096: 3.93 ms a build with the fill and ket slices, 2.78 without)
+          const bool wide = with_chunks && qc.per_slot > P.lds_max;
+          // primitive split and chunk size: the schedule's values, or less
+          // work per lane and per workgroup where the class would otherwise
+          // leave the device idle (kFillLanes, kFillGroups)
+          double lane_work = 0.0;
+          for (const Pending& pd : pend) {
+            const Run &rb = runs[pd.rb], &rk = runs[pd.rk];
+            lane_work += 0.25 * (double)pd.nq * split * (rb.npmin + rb.npmax) * (rk.npmin + rk.npmax);
+          }
+          const int64_t fill_prim = (int64_t)std::max(lane_work / kFillLanes, (double)kMinPrim);
+          const int64_t kTargetPrim = wide ? tu.target_prim : std::min<int64_t>(tu.target_prim, fill_prim);
+          int64_t items = 0;
+          for (size_t ti = 0; ti < pend.size(); ++ti) {
+            SubTask& t = qc.tasks[ti];
+            const Run &rb = runs[pend[ti].rb], &rk = runs[pend[ti].rk];
+            choose_split(rb.npmin, rb.npmax, rk.npmin, rk.npmax, kTargetPrim, wide, t);
+            t.item0 = qc.nitems;
+            qc.nitems += (int64_t)t.S * t.nq;
+            items += (int64_t)t.S * t.nq * split;
+          }
+          const int64_t fill_items = (items / kFillGroups + tu.threads - 1) / tu.threads * tu.threads;
+          const int64_t class_items =
+              std::min<int64_t>(tu.chunk_items, std::max<int64_t>(tu.threads, fill_items));
+          if (with_chunks) {
+            // bra-major chunks: consecutive bras of one sub-task, bounded LDS slots and lane-items
+            const int row_len = qc.row_len;
+            const size_t per_slot = qc.per_slot;
             const int nr = (qc.la + qc.lb + qc.lc + qc.ld) / 2 + 1;
             size_t pack = std::min<size_t>((size_t)tu.lds_pack, P.lds_budget);
             if (tu.rys_lds && per_slot + rys_slice_bytes(nr) <= P.lds_budget) {
@@ -1727,11 +1739,10 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
               qc.tab_bytes = rys_slice_bytes(nr);
               pack = pack > qc.tab_bytes + per_slot ? pack - qc.tab_bytes : per_slot;
             }
-            qc.per_slot = per_slot;
             std::vector<double> chunk_work;  // primitive quartets of a chunk's longest lane, digestion included
             // a slot wider than the packing budget still gets chunks of one
             // bra when one density's slot fits the device's LDS
-            qc.nbra_max = per_slot > P.lds_max ? 0
+            qc.nbra_max = wide ? 0
                           : (int)std::max<size_t>(1, std::min<size_t>((size_t)kChunkBrasMax, pack / per_slot));
             for (size_t ti = 0; qc.nbra_max >= 1 && ti < pend.size(); ++ti) {
               Pending& pd = pend[ti];
@@ -3534,7 +3545,7 @@ static void packed_eri(const int32_t* atm, int natm, const int32_t* bas, int nba
           EriRange r{b.beg, b.end - b.beg, k.beg, k.end - k.beg, 1, 1, 1, cb == ck && i == j, 0, 0, 0};
           SubTask t;
           // runs are sorted: the first pair has the most primitives, the last the fewest
-          choose_split(pairs[b.end - 1].np, pairs[b.beg].np, pairs[k.end - 1].np, pairs[k.beg].np, kEriPrim, t);
+          choose_split(pairs[b.end - 1].np, pairs[b.beg].np, pairs[k.end - 1].np, pairs[k.beg].np, kEriPrim, false, t);
           while (t.S * split > 256) {
             if (t.Sk > 1) t.Sk /= 2;
             t.S /= 2;
