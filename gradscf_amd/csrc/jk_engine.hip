@@ -3453,6 +3453,41 @@ __global__ __launch_bounds__(256) void packed_jk_kernel(const double* __restrict
   }
 }
 
+// J and K of few AOs: the integrals and one density in LDS, each thread sums
+// whole elements (J_ab over cd, K_ac over bd), so nothing is cleared, added
+// atomically or mirrored.  Bound by launches: with the three of the kernel
+// above (clear, rows, mirror) 7 functions took 21 us a call and 10 took 26, one
+// thread per integral with atomics 18.5 and 25, this kernel 17 and 20.
+constexpr int kPackedSmall = 12;  // 24 KB of integrals
+
+__global__ __launch_bounds__(256) void packed_jk_small_kernel(const double* __restrict__ eri, int s8, int np,
+                                                              const double* __restrict__ Dall, int n, int with_j,
+                                                              int with_k, int64_t kbase, double* __restrict__ out) {
+  constexpr int NP = kPackedSmall * (kPackedSmall + 1) / 2;
+  __shared__ double g[NP * (NP + 1) / 2], d[kPackedSmall * kPackedSmall];
+  const int nn = n * n;
+  const double* __restrict__ D = Dall + (size_t)blockIdx.x * nn;
+  double* __restrict__ o = out + (size_t)blockIdx.x * nn;
+  for (int i = threadIdx.x; i < np * np; i += blockDim.x) {
+    const int r = i / np, c = i - r * np;
+    if (c <= r) g[r * (r + 1) / 2 + c] = eri[s8 ? r * (r + 1) / 2 + c : i];
+  }
+  for (int i = threadIdx.x; i < nn; i += blockDim.x) d[i] = D[i];
+  __syncthreads();
+  auto pair = [](int i, int j) { return i > j ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i; };
+  for (int i = threadIdx.x; i < (with_j + with_k) * nn; i += blockDim.x) {
+    const bool is_j = with_j && i < nn;
+    const int e = i < nn ? i : i - nn, a = e / n, b = e - a * n;
+    double s = 0.0;
+    for (int x = 0; x < n; ++x)
+      for (int y = 0; y < (is_j ? x + 1 : n); ++y) {
+        const double v = is_j ? g[pair(pair(a, b), pair(x, y))] : g[pair(pair(a, x), pair(b, y))];
+        s += times(v, is_j && x != y ? d[x * n + y] + d[y * n + x] : d[x * n + y]);
+      }
+    o[(is_j ? 0 : kbase) + e] = s;
+  }
+}
+
 // upper triangle of every n x n matrix from its lower one
 __global__ void mirror_kernel(double* __restrict__ m, int nb, int n) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -3753,8 +3788,17 @@ static void packed_jk(const double* eri, int64_t eri_size, int ndim, const doubl
     throw Internal("Packed J/K dimensions do not match");
   if (!eri || !density || !out) throw Internal("Packed J/K requires device buffers");
   const size_t total = (size_t)(with_j + with_k) * nb * n * n;
-  hipLaunchKernelGGL(fill_kernel, dim3(nblocks(total)), dim3(256), 0, s, out, total, 0.0);
   const int64_t kbase = (int64_t)with_j * nb * n * n;
+  if (n <= kPackedSmall) {
+    for_slices(nb, grid_blocks(256), [&](int64_t first, int64_t count) {
+      const int64_t at = first * n * n;  // of the slice's first density
+      hipLaunchKernelGGL(packed_jk_small_kernel, dim3((unsigned)count), dim3(256), 0, s, eri, ndim == 1 ? 1 : 0,
+                         (int)np, density + at, n, with_j, with_k, kbase, out + at);
+    });
+    HIP_OK(hipGetLastError());
+    return;
+  }
+  hipLaunchKernelGGL(fill_kernel, dim3(nblocks(total)), dim3(256), 0, s, out, total, 0.0);
   auto launch = [&](auto kernel, int R) {
     const dim3 grid((unsigned)((n + R - 1) / R), (unsigned)n, (unsigned)nb);
     const size_t lds = with_k ? sizeof(double) * 2 * (R + 1) * (size_t)n : 0;
