@@ -127,8 +127,8 @@ constexpr int kJBraCopies = 8;
 
 // What the bra-major kernels read of a ket pair and of its shells, in one
 // record (five 16-byte loads a lane, two where both shells are s, in place of
-// ten or more loads from the pair, shell and column tables: the classes with
-// s shells spend 70 to 80% of their time with the address units busy).
+// ten or more loads from the pair, shell and column tables: the address units
+// are busy for 46 to 78 % of (ss|ss), (ps|ss) and (ps|ps) even so).
 // With the bra records and the staging of all slots at once: 64 water clusters
 // 4.70 -> 4.49 ms a build, in-core (H2O)8 cc-pVDZ 470 -> 440 us, (H2O)16 2.72 -> 2.66 ms.
 struct alignas(16) KetRec {

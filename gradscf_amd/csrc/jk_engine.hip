@@ -295,8 +295,8 @@ constexpr size_t kKetLdsBytes = 16 * 1024;  // LDS ket-J window per density
 // component, executed at the memory side, bounds them: with those atomics
 // taken out, C20H42 / 6-31G* ran (ss|ss) in 223 us instead of 413 and (ps|ps)
 // in 201 instead of 334.  Summed over the bras of a chunk first: 291 and 276
-// us, and whole builds of (H2O)16 / cc-pVDZ 2.95 -> 2.74 ms, C20H42 6.04 ->
-// 5.80 ms, in-core (H2O)8 0.61 -> 0.46 ms.  With three roots and more the
+// us, and whole builds of (H2O)16 / cc-pVDZ 2.83 -> 2.65 ms, C20H42 6.28 ->
+// 5.90 ms, in-core (H2O)8 0.46 -> 0.33 ms.  With three roots and more the
 // quartets hide the atomics ((dp|ps) 312 us with and without) and the window
 // only takes LDS: (H2O)16 2.66 -> 2.78 ms with windows for three roots too.
 constexpr int kWindowRoots = 2;
@@ -1440,11 +1440,13 @@ constexpr int64_t kMinPrim = 2;
 // Work of one chunk at most, in primitive quartets over all lane-items, with
 // kDigestPrims for the digestion of an item.  A chunk of 4096 items of 48
 // primitive quartets runs for 230 us or more, and a class of few such chunks
-// waits for the last of them on a nearly idle chip.  Together with the order
-// of falling work: 64 clusters of water 5.0 -> 4.65 ms, (H2O)16 2.74 -> 2.70,
-// C20H42 5.88 -> 5.75, two densities of (H2O)7 1.24 -> 1.16 ms a build (order
-// alone 4.71, 2.68, 5.80 and 1.23).  16000 costs more exchange-row flushes
-// than it saves (C20H42 6.74 ms), 64000 gains nothing further.
+// waits for the last of them on a nearly idle chip.  The order of falling work
+// gives most of what the two give (64 clusters of water 5.0 -> 4.7 ms, (H2O)16
+// 2.74 -> 2.68 when it came in); of the limit, with all that came after it:
+// two densities of (H2O)7 984 us without it and 963 with it, against more slab
+// flushes of long builds, (H2O)16 2.72 and 2.76 ms, C20H42 5.74-5.94 and 5.90-
+// 5.95, 64 clusters 4.35 and 4.40.  16000 flushes far too often (C20H42 6.74
+// ms), 64000 gains nothing further.
 constexpr double kChunkWork = 128000.0;
 constexpr double kDigestPrims = 6.0;
 
