@@ -1683,7 +1683,7 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
           const int rows = wa + wb;
           // full-block classes stage their chunk's bra primitive pairs in
           // LDS (kStagedPrim doubles each, kStagedPrimCoef with bra columns)
-          const bool stage = split == 1;
+          bool stage = split == 1;
           const int rec = pb ? kStagedPrimCoef : kStagedPrim;
           if (with_chunks) {
             int bra_np_max = 0;
@@ -1701,6 +1701,13 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
             qc.row_len = row_len;
             qc.per_slot = sizeof(double) * ((size_t)rows * row_len + (size_t)wa * wb * (kJBraCopies + 1) +
                                             (size_t)rec * bra_np_max + kBraRecDoubles);
+            // the bra's record must not cost a class its LDS route: where the
+            // rest of the slot fits, the primitives are read from memory
+            constexpr size_t kRecordBytes = sizeof(BraRec) - sizeof(double);
+            if (stage && qc.per_slot > P.lds_max && qc.per_slot - kRecordBytes <= P.lds_max) {
+              stage = false;
+              qc.per_slot -= sizeof(double) * (size_t)rec * bra_np_max;
+            }
           }
           // rows that do not fit: the global-atomic kernels, whose lanes add
           // every slice's terms by themselves.  A slice more is then not a
