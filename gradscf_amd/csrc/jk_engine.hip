@@ -350,6 +350,7 @@ struct PairSet {
   int64_t* d_cinv_off = nullptr;
   int* d_cinv = nullptr;
   int64_t nrows = 0;
+  double kent_mean = 0.0;  // entries per non-empty list of the whole list
   int nc_max = 0;
   // device memory the pointers above (and the classes') point into
   char* d_tables = nullptr;
@@ -405,6 +406,7 @@ struct PlanData {
   // per launch stream: row lists of the exchange-row slabs of its classes, so
   // that each stream folds its own slabs as soon as its classes are done
   std::vector<int64_t*> d_lane_krp, d_lane_kent;
+  std::vector<double> lane_mean;  // entries per non-empty list
   char* d_lane_tables = nullptr;   // their memory
   size_t part_nbd = 0;
   double* d_incore = nullptr;   // in-core integrals: stored Cartesian blocks of the J/K quartets
@@ -742,10 +744,22 @@ __global__ void dens_to_cart_kernel(const double* __restrict__ D, int64_t nn_tot
 // row R of K.
 // The wavefronts of a workgroup share the row's slab list (eight entries each
 // in turn) and add up in LDS: with one wavefront per row and column block the
-// list was a serial chain of dependent reads that outlasted the class kernels
-// of small molecules (in-core builds of (H2O)8: 650 us with one, 615 us with
-// four; 8 and 16 cost batches of small molecules 3-5 %, whose lists are short).
+// list is a serial chain of dependent reads, which lasts where there are few
+// rows to run beside it (in-core builds of C12H26 6-31G* 940 us with one, 910
+// with four, (H2O)8 cc-pVDZ 209 and 204).  Many rows fill the device by
+// themselves, and the wavefronts without a share of a short list only take its
+// places: 512 waters cc-pVDZ in core 985 us with one, 1090 with four, 2000
+// STO-3G 174 and 238, (H2O)16 330 and 338.
 constexpr int kPartReduceWaves = 4;
+
+// Wavefronts per row and column block: `groups` of these in the launch, `mean`
+// entries in a list.  (C20H42: 2800 groups, 90 to 260 entries, 2 % for four;
+// (H2O)16: 2800 and 14 to 24, 2 % for one; 64 clusters 6-31G*: 6000 and 30, 1
+// to 3 % for one.)
+static int part_reduce_waves(double mean, int64_t groups) {
+  return 64.0 * mean > (double)groups ? kPartReduceWaves : 1;
+}
+
 __global__ __launch_bounds__(64 * kPartReduceWaves) void kpart_reduce_kernel(const double* __restrict__ part, int64_t stride,
                                                             const int64_t* __restrict__ rp,
                                                             const int64_t* __restrict__ ent,
@@ -758,7 +772,7 @@ __global__ __launch_bounds__(64 * kPartReduceWaves) void kpart_reduce_kernel(con
   __shared__ double sums[kPartReduceWaves][64];
   const int64_t R = row0 + blockIdx.x;
   const int bt = blockIdx.z;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = kPartReduceWaves;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const int col = blockIdx.y * 64 + lane;
   const int n = row_n[R];
   const int m = row_mol[R];
@@ -1913,11 +1927,16 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
     auto csr = [&](std::vector<std::pair<int64_t, int64_t>>& ent, int64_t nkeys, size_t& o_rp, size_t& o_ent) {
       std::vector<int64_t> rp(nkeys + 1, 0), off(std::max<size_t>(1, ent.size()));
       for (const auto& e : ent) ++rp[e.first + 1];
-      for (int64_t k = 0; k < nkeys; ++k) rp[k + 1] += rp[k];
+      int64_t keys = 0;
+      for (int64_t k = 0; k < nkeys; ++k) {
+        keys += rp[k + 1] > 0;
+        rp[k + 1] += rp[k];
+      }
       std::vector<int64_t> fill(rp.begin(), rp.end() - 1);
       for (const auto& e : ent) off[fill[e.first]++] = e.second;
       o_rp = up.add(rp);
       o_ent = up.add(off);
+      return keys;
     };
     int64_t nrows = 0;
     for (int m = 0; m < P.nmol; ++m) nrows = std::max<int64_t>(nrows, (int64_t)P.mols[m].aoc0 + P.mols[m].nc);
@@ -1934,7 +1953,8 @@ static void build_pair_set(PlanData& P, PairSet& S, std::vector<PairCand>& cand,
     o_row_dst = up.add(row_dst);
     o_row_n = up.add(row_n);
     o_row_mol = up.add(row_mol);
-    csr(kent, nrows * 8, o_krp, o_kent);
+    const int64_t kent_keys = csr(kent, nrows * 8, o_krp, o_kent);
+    S.kent_mean = (double)kent.size() / std::max<int64_t>(1, kent_keys);
     csr(jent, (int64_t)S.pairs.size(), o_jrp, o_jent);
     S.h_kent = std::move(kent);
     S.h_kent_cls = std::move(kent_cls);
@@ -2176,6 +2196,7 @@ static void assign_lanes(PlanData& P) {
   P.d_lane_tables = nullptr;
   P.d_lane_krp.clear();
   P.d_lane_kent.clear();
+  P.lane_mean.clear();
   P.lane_classes.assign(ns, {});
   std::vector<int> order(P.jk.classes.size());
   for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
@@ -2200,7 +2221,12 @@ static void assign_lanes(PlanData& P) {
       std::vector<int64_t> rp(nkeys + 1, 0), off;
       for (size_t i = 0; i < S.h_kent.size(); ++i)
         if (lane_of[S.h_kent_cls[i]] == l) ++rp[S.h_kent[i].first + 1];
-      for (int64_t k = 0; k < nkeys; ++k) rp[k + 1] += rp[k];
+      int64_t keys = 0;
+      for (int64_t k = 0; k < nkeys; ++k) {
+        keys += rp[k + 1] > 0;
+        rp[k + 1] += rp[k];
+      }
+      P.lane_mean.push_back((double)rp[nkeys] / std::max<int64_t>(1, keys));
       off.assign(std::max<int64_t>(1, rp[nkeys]), 0);
       std::vector<int64_t> fill(rp.begin(), rp.end() - 1);
       for (size_t i = 0; i < S.h_kent.size(); ++i)
@@ -2888,21 +2914,23 @@ static void jk_build(PlanData& P, const double* density, int nb, double* out, in
       P.ev_used += 2;
     }
   }
-  auto reduce_rows = [&](const int64_t* rp, const int64_t* ent, int nd, int atomic, hipStream_t st) {
-    for_slices(S.nrows, grid_blocks(64 * kPartReduceWaves), [&](int64_t row0, int64_t rows) {
-      hipLaunchKernelGGL(kpart_reduce_kernel, dim3((unsigned)rows, (unsigned)((S.nc_max + 63) / 64), (unsigned)nd),
-                         dim3(64 * kPartReduceWaves), 0, st, W.part, S.part_total, rp, ent, S.d_row_dst, S.d_row_n,
+  auto reduce_rows = [&](const int64_t* rp, const int64_t* ent, double mean, int nd, int atomic, hipStream_t st) {
+    const int cols = (S.nc_max + 63) / 64;
+    const int waves = part_reduce_waves(mean, S.nrows * cols * nd);
+    for_slices(S.nrows, grid_blocks(64 * waves), [&](int64_t row0, int64_t rows) {
+      hipLaunchKernelGGL(kpart_reduce_kernel, dim3((unsigned)rows, (unsigned)cols, (unsigned)nd),
+                         dim3(64 * waves), 0, st, W.part, S.part_total, rp, ent, S.d_row_dst, S.d_row_n,
                          S.d_row_mol, S.d_cinv_off, S.d_cinv, P.ncc_tot, atomic, row0, W.kp);
     });
   };
   if (lane_reduce)
     for (size_t l = 0; l < P.lane_classes.size(); ++l)
-      reduce_rows(P.d_lane_krp[l], P.d_lane_kent[l], nbd, 1, streams.lane((int)l));
+      reduce_rows(P.d_lane_krp[l], P.d_lane_kent[l], P.lane_mean[l], nbd, 1, streams.lane((int)l));
   streams.join();
   if (S.part_total > 0) {
     const int nbd_k = with_k ? nbd : nb;
     if (with_k && (psums & 1) && !lane_reduce)
-      reduce_rows(S.d_krp, S.d_kent, nbd_k, 0, s);
+      reduce_rows(S.d_krp, S.d_kent, S.kent_mean, nbd_k, 0, s);
     if (with_j && (psums & 2))
       hipLaunchKernelGGL(jpart_reduce_kernel, dim3((unsigned)S.pairs.size(), (unsigned)nb), dim3(64), 0, s,
                          W.part, S.part_total, S.d_jrp, S.d_jent, S.d_pairs, S.d_shells, P.d_molinfo,
