@@ -753,14 +753,16 @@ __global__ void dens_to_cart_kernel(const double* __restrict__ D, int64_t nn_tot
 constexpr int kPartReduceWaves = 4;
 
 // Wavefronts per row and column block: `groups` of these in the launch, `mean`
-// entries in a list.  (C20H42: 2800 groups, 90 to 260 entries, 2 % for four;
-// (H2O)16: 2800 and 14 to 24, 2 % for one; 64 clusters 6-31G*: 6000 and 30, 1
-// to 3 % for one.)
+// entries in a list.  (In-core builds: C20H42, 2800 groups, 40 to 260 entries,
+// and (H2O)12, 3000 and 30, 1 to 2 % for four; (H2O)16 at cutoff 1e-10, 2800
+// and 14 to 24, 2 % for one; 64 clusters 6-31G*, 15600 and 26 to 58, 1 to 3 %
+// for one.)
 static int part_reduce_waves(double mean, int64_t groups) {
-  return 64.0 * mean > (double)groups ? kPartReduceWaves : 1;
+  return 128.0 * mean > (double)groups ? kPartReduceWaves : 1;
 }
 
-__global__ __launch_bounds__(64 * kPartReduceWaves) void kpart_reduce_kernel(const double* __restrict__ part, int64_t stride,
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void kpart_reduce_kernel(const double* __restrict__ part, int64_t stride,
                                                             const int64_t* __restrict__ rp,
                                                             const int64_t* __restrict__ ent,
                                                             const int64_t* __restrict__ row_dst,
@@ -769,10 +771,10 @@ __global__ __launch_bounds__(64 * kPartReduceWaves) void kpart_reduce_kernel(con
                                                             const int64_t* __restrict__ cinv_off,
                                                             const int* __restrict__ cinv, int64_t ncc_tot,
                                                             int atomic, int64_t row0, double* __restrict__ kp) {
-  __shared__ double sums[kPartReduceWaves][64];
+  __shared__ double sums[NW][64];
   const int64_t R = row0 + blockIdx.x;
   const int bt = blockIdx.z;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = blockIdx.y * 64 + lane;
   const int n = row_n[R];
   const int m = row_mol[R];
@@ -786,7 +788,7 @@ __global__ __launch_bounds__(64 * kPartReduceWaves) void kpart_reduce_kernel(con
     if (j < 0) continue;
     any = true;
     int64_t e = e0 + 8 * wave;
-    for (; e + 8 <= e1; e += 8 * nw) {
+    for (; e + 8 <= e1; e += 8 * NW) {
 #pragma unroll
       for (int u = 0; u < 8; ++u) v[u] += pb[ent[e + u] + j];
     }
@@ -796,7 +798,7 @@ __global__ __launch_bounds__(64 * kPartReduceWaves) void kpart_reduce_kernel(con
   sums[wave][lane] = sum;
   __syncthreads();
   if (wave != 0 || col >= n) return;
-  for (int w = 1; w < nw; ++w) sum += sums[w][lane];
+  for (int w = 1; w < NW; ++w) sum += sums[w][lane];
   double* dst = kp + (size_t)bt * ncc_tot + row_dst[R] + col;
   if (!atomic) {
     *dst += sum;
@@ -2917,8 +2919,9 @@ static void jk_build(PlanData& P, const double* density, int nb, double* out, in
   auto reduce_rows = [&](const int64_t* rp, const int64_t* ent, double mean, int nd, int atomic, hipStream_t st) {
     const int cols = (S.nc_max + 63) / 64;
     const int waves = part_reduce_waves(mean, S.nrows * cols * nd);
+    auto kernel = waves == 1 ? kpart_reduce_kernel<1> : kpart_reduce_kernel<kPartReduceWaves>;
     for_slices(S.nrows, grid_blocks(64 * waves), [&](int64_t row0, int64_t rows) {
-      hipLaunchKernelGGL(kpart_reduce_kernel, dim3((unsigned)rows, (unsigned)cols, (unsigned)nd),
+      hipLaunchKernelGGL(kernel, dim3((unsigned)rows, (unsigned)cols, (unsigned)nd),
                          dim3(64 * waves), 0, st, W.part, S.part_total, rp, ent, S.d_row_dst, S.d_row_n,
                          S.d_row_mol, S.d_cinv_off, S.d_cinv, P.ncc_tot, atomic, row0, W.kp);
     });
