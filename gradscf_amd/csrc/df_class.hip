@@ -25,7 +25,7 @@ __device__ __forceinline__ void df_blocks(const DfArgs& a, const DfRange& r, dou
   constexpr int NBRA = K::NBRA, NC = K::NC;
   const int lanes = K::SPLIT * r.S;
   const int local = threadIdx.x / lanes;
-  const int64_t t0 = r.task0 + (int64_t)(blockIdx.x - r.block0) * r.T;
+  const int64_t t0 = ((int64_t)blockIdx.x - r.block0) * r.T;
   const int64_t ntask = (int64_t)r.npair * a.nket;
   if (local < r.T && t0 + local < ntask) {
     const int64_t t = t0 + local;
@@ -79,7 +79,7 @@ template <int LC>
 __global__ __launch_bounds__(256) void df_kernel(DfArgs a) {
   extern __shared__ double buf[];
   int k = 0;
-  while (k + 1 < a.nrange && a.ranges[k + 1].block0 <= (int)blockIdx.x) ++k;
+  while (k + 1 < a.nrange && a.ranges[k + 1].block0 <= (int64_t)blockIdx.x) ++k;
   const DfRange r = a.ranges[k];
   switch (r.la * 8 + r.lb) {
     case 0: df_blocks<0, 0, LC>(a, r, buf); break;

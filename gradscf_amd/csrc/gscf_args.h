@@ -261,15 +261,13 @@ struct SphTerm {
 
 // Bra pairs [pair0, pair0 + npair) of one class (la, lb) with similar
 // primitive counts: T (bra pair, ket shell) tasks per block, each on
-// S (x ket components) lanes, tasks from task0 and blocks from block0 on (a
-// range may be spread over several launches).
+// S (x ket components) lanes, blocks from block0 on (negative where the range
+// began in an earlier launch: its first task here is -block0 T).
 struct DfRange {
   int la, lb;
   int pair0, npair;
   int S, T;
-  int block0;
-  int pad;
-  int64_t task0;
+  int64_t block0;
 };
 
 // Lanes over ket components: blocks of more than 36 Cartesian components do
@@ -298,14 +296,12 @@ struct DfArgs {
 // ----------------------------------------------------------------------------
 // Tasks (bra pair, ket pair) of two pair ranges with similar primitive counts
 // (tri: one range with itself, ket <= bra): T per block on S = Sb * Sk lanes
-// (x ket components) each, tasks from task0 and blocks from block0 on (a range
-// may be spread over several launches).
+// (x ket components) each, blocks from block0 on (negative where the range
+// began in an earlier launch: its first task here is -block0 T).
 struct EriRange {
   int bra0, nbra, ket0, nket;
   int S, Sk, T, tri;
-  int block0;
-  int pad;
-  int64_t task0;
+  int64_t block0;
 };
 
 struct EriArgs {

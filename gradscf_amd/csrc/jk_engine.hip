@@ -3617,7 +3617,7 @@ static void packed_eri(const int32_t* atm, int natm, const int32_t* bas, int nba
         for (size_t j = 0; j < runs[ck].size(); ++j) {
           if (cb == ck && j < i) continue;  // one order of two runs
           const Run &b = runs[cb][i], &k = runs[ck][j];
-          EriRange r{b.beg, b.end - b.beg, k.beg, k.end - k.beg, 1, 1, 1, cb == ck && i == j, 0, 0, 0};
+          EriRange r{b.beg, b.end - b.beg, k.beg, k.end - k.beg, 1, 1, 1, cb == ck && i == j, 0};
           SubTask t;
           // runs are sorted: the first pair has the most primitives, the last the fewest
           choose_split(pairs[b.end - 1].np, pairs[b.beg].np, pairs[k.end - 1].np, pairs[k.beg].np, kEriPrim, false, t);
@@ -3635,8 +3635,7 @@ static void packed_eri(const int32_t* atm, int natm, const int32_t* bas, int nba
               launches.push_back(L);
               L = {cb, ck, (int)ranges.size(), 0, 0, 0};
             }
-            r.task0 = first * r.T;
-            r.block0 = L.blocks;
+            r.block0 = L.blocks - first;
             ranges.push_back(r);
             L.blocks += (int)count;
             L.lds = std::max(L.lds, blk * r.T);
@@ -3767,7 +3766,7 @@ static void density_fitting(const int32_t* atm, int natm, const int32_t* bas, in
       for (int i = b.beg; i < b.end;) {
         int e = i;
         while (e < b.end && pair_bucket(pairs[e]) == pair_bucket(pairs[i])) ++e;
-        DfRange r{b.la, b.lb, i, e - i, 1, 1, 0, 0, 0};
+        DfRange r{b.la, b.lb, i, e - i, 1, 1, 0};
         const int64_t work = (int64_t)pairs[i].np * pairs[aux0[lc]].np;
         while (r.S < 16 && (int64_t)r.S * kDfPrim < work && 2 * r.S <= pairs[e - 1].np) r.S *= 2;
         r.T = (int)std::max<size_t>(1, std::min<size_t>({(size_t)256 / (r.S * df_split(b.la, b.lb, lc)), kLdsBudget / (8 * blk), share}));
@@ -3777,8 +3776,7 @@ static void density_fitting(const int32_t* atm, int natm, const int32_t* bas, in
             launches.push_back(L);
             L = {lc, (int)ranges.size(), 0, 0, 0};
           }
-          r.task0 = first * r.T;
-          r.block0 = L.blocks;
+          r.block0 = L.blocks - first;
           ranges.push_back(r);
           L.blocks += (int)count;
           L.lds = std::max(L.lds, 8 * blk * r.T);

@@ -1501,11 +1501,11 @@ __global__ __launch_bounds__(256) void eri_kernel(EriArgs a) {
   using K = Class<LA, LB, LC, LD>;
   extern __shared__ double ebuf[];
   int x = 0;
-  while (x + 1 < a.nrange && a.ranges[x + 1].block0 <= (int)blockIdx.x) ++x;
+  while (x + 1 < a.nrange && a.ranges[x + 1].block0 <= (int64_t)blockIdx.x) ++x;
   const EriRange r = a.ranges[x];
   const int lanes = K::SPLIT * r.S;
   const int local = threadIdx.x / lanes;
-  const int64_t t0 = r.task0 + (int64_t)(blockIdx.x - r.block0) * r.T;
+  const int64_t t0 = ((int64_t)blockIdx.x - r.block0) * r.T;
   const int64_t ntask = r.tri ? (int64_t)r.nbra * (r.nbra + 1) / 2 : (int64_t)r.nbra * r.nket;
   auto task = [&](int64_t t, int& bra, int& ket) {
     if (r.tri) {
